@@ -1,0 +1,303 @@
+"""What the framework is timed on: the work a program built on it does, through its public entry points.
+
+Seven kinds of work, each over the sizes it has in real use:
+
+* ``linear``   one quantised linear layer (``HQQLinearTritonSavable``), one row to a few thousand;
+* ``ffn``      one expert's feed-forward block (``MixtralBLockSparseTop2MLP_HQQ``) on a decode batch;
+* ``moe``      a sparse-MoE block (``SparseMoeWrapper``): router, grouping and eight resident experts on the tokens of
+               a decode batch or of a prompt;
+* ``request``  a whole request, greedy: the prompt, then decode steps replayed from a HIP graph, all experts resident;
+* ``offload``  decode steps driven from the host with part of the experts in pinned host memory;
+* ``prompt``   the prompt pass of the model, alone, at the start of a cache or behind cached tokens;
+* ``convert``  a fp16 layer quantised with hqq's solver and repacked: what loading an unquantised model does.
+
+Layer sizes are those of the repository's model configuration (hidden 4096, FFN 14336, attention 4-bit in groups of 64,
+experts 2-bit in groups of 16 or 3-bit in groups of 64, 8-bit scales and zeros); models have fewer layers, each of the
+full size, so that one is made quickly.  Weights are random.  A trained router is decisive and a trained
+head confident, random ones are neither: the embeddings (or the hidden states given to a block) lean towards two experts
+per layer, some experts more popular than others, and the head answers a token's embedding with one next token, so
+that neither the experts nor the tokens of a run hang on the last bit of a sum."""
+from __future__ import annotations
+
+import math
+import os
+import sys
+
+import torch
+from torch import nn
+
+_PACKAGE = os.path.abspath("mixtral-offloading_amd")
+if _PACKAGE not in sys.path:
+    sys.path.insert(1, _PACKAGE)
+
+from mixtral_offloading_amd import build_model as bm  # noqa: E402
+from mixtral_offloading_amd.custom_layers import HQQLinearTritonSavable  # noqa: E402
+from mixtral_offloading_amd.hqq_core import BaseQuantizeConfig  # noqa: E402
+from mixtral_offloading_amd.mixtral_model import DecodeGraph  # noqa: E402
+
+HIDDEN, FFN, HEADS, KV_HEADS, HEAD_DIM, EXPERTS, VOCAB = 4096, 14336, 32, 8, 128, 8, 32000
+GROUP = {2: 16, 3: 64, 4: 64}
+# (n, k) of the model's layers: q and o, k and v, the experts' up and down projections
+LAYERS = ((HIDDEN, HIDDEN), (KV_HEADS * HEAD_DIM, HIDDEN), (FFN, HIDDEN), (HIDDEN, FFN))
+LEAN = (6.0, 5.4)  # how far a token leans to its two experts, in standard deviations of the other experts' logits
+
+
+# ------------------------------------------------------------------ the cases
+def _linear(bits, n, k, rows, meta8=True):
+    return {"kind": "linear", "bits": bits, "group": GROUP[bits], "n": n, "k": k, "rows": rows, "meta8": meta8}
+
+
+def listed():
+    return [
+        # the smallest call there is: a query projection of one decoded token, nearly all latency
+        {"name": "linear_w4_1_row", **_linear(4, HIDDEN, HIDDEN, 1)},
+        # an expert's down projection on a ragged part of a prompt
+        {"name": "linear_w2_333_rows", **_linear(2, HIDDEN, FFN, 333)},
+        # one expert on one token: the unit of work of batch-1 decoding
+        {"name": "ffn_w2_1_row", "kind": "ffn", "bits": 2, "rows": 1},
+        # a decode batch of sixteen sequences: every expert is read for two to six rows
+        {"name": "moe_w2_16_tokens", "kind": "moe", "bits": 2, "tokens": 16},
+        # the 3-bit variant on a larger decode batch: about a dozen rows an expert
+        {"name": "moe_w3_45_tokens", "kind": "moe", "bits": 3, "tokens": 45},
+        # a prompt's MoE block: some hundreds of rows for the popular experts, tens for the others
+        {"name": "moe_w2_700_tokens", "kind": "moe", "bits": 2, "tokens": 700},
+        # short chat turn: the repository's 64-token prompt and 32 tokens decoded from a graph
+        {"name": "request_w2_64_32", "kind": "request", "bits": 2, "layers": 4, "prompt": 64, "new": 32},
+        # the 3-bit variant with a longer prompt and a short answer
+        {"name": "request_w3_300_16", "kind": "request", "bits": 3, "layers": 2, "prompt": 300, "new": 16},
+        # experts in host memory, four of eight per layer on the card: bound by the host link
+        {"name": "offload_w2_8_tokens", "kind": "offload", "bits": 2, "layers": 2, "resident": 4, "cached": 64, "tokens": 8},
+        # the repository's 128-token prompt
+        {"name": "prompt_w2_128_tokens", "kind": "prompt", "bits": 2, "layers": 2, "cached": 0, "tokens": 128},
+        # a long document as prompt
+        {"name": "prompt_w2_1999_tokens", "kind": "prompt", "bits": 2, "layers": 2, "cached": 0, "tokens": 1999},
+        # quantising one expert projection of an unquantised model
+        {"name": "convert_w2", "kind": "convert", "bits": 2, "n": FFN, "k": HIDDEN},
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(("linear", "linear", "linear", "ffn", "ffn", "moe", "moe", "request", "offload", "prompt", "prompt", "convert"))
+    if kind == "linear":
+        bits = rng.choice((2, 3, 4))
+        if rng.random() < 0.7:
+            n, k = rng.choice(LAYERS)
+        else:  # layers of any other model: whole groups, widths that need not fill a tile
+            n, k = 128 * _log_int(rng, 4, 96), 64 * _log_int(rng, 8, 192)
+        return _linear(bits, n, k, _log_int(rng, 1, 4096), rng.random() < 0.75)
+    if kind == "ffn":
+        return {"kind": "ffn", "bits": rng.choice((2, 2, 3, 4)), "rows": _log_int(rng, 1, 64)}
+    if kind == "moe":
+        return {"kind": "moe", "bits": rng.choice((2, 2, 3)), "tokens": _log_int(rng, 1, 2000)}
+    if kind == "request":
+        return {"kind": "request", "bits": rng.choice((2, 2, 3)), "layers": rng.choice((1, 2, 3)),
+                "prompt": _log_int(rng, 2, 900), "new": rng.randint(4, 24)}
+    if kind == "offload":
+        return {"kind": "offload", "bits": rng.choice((2, 2, 3)), "layers": 1, "resident": rng.choice((2, 3, 4, 6)),
+                "cached": _log_int(rng, 2, 600), "tokens": rng.randint(4, 12)}
+    if kind == "prompt":
+        return {"kind": "prompt", "bits": rng.choice((2, 2, 3)), "layers": rng.choice((1, 2)),
+                "cached": rng.choice((0, 0, 0, _log_int(rng, 16, 500))), "tokens": _log_int(rng, 2, 1400)}
+    n, k = rng.choice(LAYERS)
+    return {"kind": "convert", "bits": rng.choice((2, 3, 4)), "n": n, "k": k}
+
+
+# ------------------------------------------------------------------ what a program has in hand before the call
+def _quant_config(bits, meta8=True, optimize=False):
+    cfg = BaseQuantizeConfig(nbits=bits, group_size=GROUP[bits], quant_zero=meta8, quant_scale=meta8)
+    cfg["weight_quant_params"]["optimize"] = optimize
+    return cfg
+
+
+def _generator(seed):
+    return torch.Generator(device="cuda").manual_seed(seed)
+
+
+def _fp16_linear(n, k, gen):
+    lin = nn.Linear(k, n, bias=False, device="meta", dtype=torch.float16)
+    lin.weight = nn.Parameter((torch.randn((n, k), device="cuda", generator=gen) * 0.02).half(), requires_grad=False)
+    return lin
+
+
+def _leaning(count, gates, gen):
+    """(count, hidden): noise of unit size plus, for every router of ``gates``, a lean towards two of its experts."""
+    x = torch.randn((count, HIDDEN), device="cuda", generator=gen)
+    for gate in gates:
+        rows = gate.weight.float()
+        rows = rows / rows.norm(dim=1, keepdim=True)
+        popular = 0.5 * torch.randn(EXPERTS, device="cuda", generator=gen)
+        u = torch.rand((count, EXPERTS), device="cuda", generator=gen).clamp_(1e-6, 1 - 1e-6)
+        two = (popular - torch.log(-torch.log(u))).topk(2, dim=1).indices
+        x += LEAN[0] * rows[two[:, 0]] + LEAN[1] * rows[two[:, 1]]
+    return x
+
+
+def _model(bits, layers, seed, positions, resident=EXPERTS):
+    """The repository's model with ``layers`` layers, ``resident`` of eight experts per layer on the card."""
+    quant = bm.QuantConfig(ffn_config=_quant_config(bits), attn_config=_quant_config(4))
+    offload = bm.OffloadConfig(main_size=layers * resident, offload_size=layers * (EXPERTS - resident), buffer_size=4,
+                               offload_per_layer=EXPERTS - resident)
+    config = bm.mixtral_config(num_hidden_layers=layers)
+    model = bm.build_model(torch.device("cuda:0"), quant, offload, model_config=config, seed=seed, max_positions=positions)
+    gen = _generator(seed + 1)
+    rows = _leaning(VOCAB, [l.block_sparse_moe.gate for l in model.model.layers], gen)
+    after = torch.randperm(VOCAB, device="cuda", generator=gen)  # the token that follows
+    model.model.embed_tokens.weight.data.copy_(4.0 * rows)
+    model.lm_head.weight.data[after] = (0.02 * rows).half()
+    return model, gen
+
+
+def _tokens(count, gen):
+    return torch.randint(0, VOCAB, (count,), device="cuda", generator=gen)
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind == "linear":
+        gen = _generator(seed)
+        layer = HQQLinearTritonSavable(_fp16_linear(case["n"], case["k"], gen), _quant_config(case["bits"], case["meta8"]))
+        return {"kind": kind, "layer": layer, "x": torch.randn((case["rows"], case["k"]), device="cuda", generator=gen).half()}
+    if kind == "ffn":
+        gen = _generator(seed)
+        quant = bm.QuantConfig(ffn_config=_quant_config(case["bits"]), attn_config=_quant_config(4))
+        expert = bm.make_random_expert(bm.mixtral_config(), quant, gen, torch.device("cuda:0"))
+        return {"kind": kind, "expert": expert, "x": torch.randn((case["rows"], HIDDEN), device="cuda", generator=gen).half()}
+    if kind == "moe":
+        model, gen = _model(case["bits"], 1, seed, 64)
+        block = model.model.layers[0].block_sparse_moe
+        return {"kind": kind, "block": block, "x": _leaning(case["tokens"], [block.gate], gen).half()[None]}
+    if kind == "request":
+        room = case["prompt"] + case["new"] + 2
+        model, gen = _model(case["bits"], case["layers"], seed, room)
+        prompt = _tokens(case["prompt"], gen)
+        decode = DecodeGraph(model, room)
+        decode.prefill(prompt)
+        decode.capture()
+        return {"kind": kind, "model": model, "decode": decode, "prompt": prompt, "new": case["new"]}
+    if kind == "offload":
+        room = case["cached"] + case["tokens"]
+        model, gen = _model(case["bits"], case["layers"], seed, room, case["resident"])
+        cache = model.new_cache(room)
+        prompt = _tokens(case["cached"], gen)
+        first = model.forward(prompt, cache, 0)[-1].argmax()
+        return {"kind": kind, "model": model, "cache": cache, "token": first, "start": case["cached"], "steps": case["tokens"]}
+    if kind == "prompt":
+        room = case["cached"] + case["tokens"]
+        model, gen = _model(case["bits"], case["layers"], seed, room)
+        cache = model.new_cache(room)
+        if case["cached"]:
+            model.forward(_tokens(case["cached"], gen), cache, 0)
+        return {"kind": kind, "model": model, "cache": cache, "ids": _tokens(case["tokens"], gen), "start": case["cached"]}
+    gen = _generator(seed)
+    return {"kind": kind, "linear": _fp16_linear(case["n"], case["k"], gen), "config": _quant_config(case["bits"], optimize=True)}
+
+
+# ------------------------------------------------------------------ one pass
+def _flat(cache):
+    return [t for pair in cache for t in pair]
+
+
+def run(state):
+    kind = state["kind"]
+    if kind == "linear":
+        return state["layer"](state["x"])
+    if kind == "ffn":
+        return state["expert"](state["x"])
+    if kind == "moe":
+        return state["block"](state["x"])
+    if kind == "request":
+        decode = state["decode"]
+        ids, _ = state["model"].generate_graph(state["prompt"], state["new"], decode)
+        return {"ids": ids, "logits": decode.logits, "cache": _flat(decode.cache)}
+    if kind == "offload":
+        token, logits = state["token"], []
+        for i in range(state["steps"]):
+            logits.append(state["model"].forward(token.view(1), state["cache"], state["start"] + i))
+            token = logits[-1][-1].argmax()
+        return {"logits": torch.cat(logits), "cache": _flat(state["cache"])}
+    if kind == "prompt":
+        return {"logits": state["model"].forward(state["ids"], state["cache"], state["start"]), "cache": _flat(state["cache"])}
+    layer = HQQLinearTritonSavable(state["linear"], state["config"])
+    meta = layer.meta
+    return {"codes": layer.W_q.as_subclass(torch.Tensor), "scale_q": meta["scale_q"], "zero_q": meta["zero_q"],
+            "meta": [meta[m][v] for m in ("meta_scale", "meta_zero") for v in ("scale", "zero")]}
+
+
+# ------------------------------------------------------------------ what a pass cannot do without
+def _layer_bytes(bits, n, k, meta8=True):
+    codes = 4 * ((n + 9) // 10) * k if bits == 3 else n * k * bits // 8
+    entries = n * k // GROUP[bits]
+    return codes + (2 * entries + 4 * (entries // 128) + 4 if meta8 else 4 * entries)
+
+
+def _expert_bytes(bits):
+    return 2 * _layer_bytes(bits, FFN, HIDDEN) + _layer_bytes(bits, HIDDEN, FFN)
+
+
+def _attention_weight_bytes():
+    return sum(_layer_bytes(4, n, HIDDEN) for n in (HIDDEN, HIDDEN, KV_HEADS * HEAD_DIM, KV_HEADS * HEAD_DIM))
+
+
+def _experts_used(tokens):
+    return EXPERTS * (1 - (1 - 2 / EXPERTS) ** tokens)
+
+
+def _block_work(bits, layers, tokens, cached, head=True):
+    """``tokens`` new tokens through the model at once."""
+    kv_row = 2 * 2 * KV_HEADS * HEAD_DIM
+    proj = HIDDEN * (2 * HIDDEN + 2 * KV_HEADS * HEAD_DIM)
+    nbytes = layers * (_attention_weight_bytes() + _experts_used(tokens) * _expert_bytes(bits) + kv_row * (cached + tokens))
+    flops = layers * (2.0 * tokens * (proj + 2 * 3 * HIDDEN * FFN) + 4.0 * HEADS * HEAD_DIM * tokens * (cached + (tokens + 1) / 2))
+    nbytes += 2 * tokens * HIDDEN
+    if head:
+        nbytes += 2 * VOCAB * HIDDEN + 2 * tokens * VOCAB
+        flops += 2.0 * tokens * VOCAB * HIDDEN
+    return nbytes, flops
+
+
+def work(case):
+    kind = case["kind"]
+    if kind == "linear":
+        n, k, m = case["n"], case["k"], case["rows"]
+        nbytes, flops = _layer_bytes(case["bits"], n, k, case["meta8"]) + 2 * m * (n + k), 2.0 * m * n * k
+    elif kind == "ffn":
+        m = case["rows"]
+        nbytes, flops = _expert_bytes(case["bits"]) + 4 * m * HIDDEN, 2.0 * m * 3 * HIDDEN * FFN
+    elif kind == "moe":
+        t = case["tokens"]
+        nbytes = _experts_used(t) * _expert_bytes(case["bits"]) + 4 * t * HIDDEN + 2 * EXPERTS * (HIDDEN + t)
+        flops = 2.0 * t * (2 * 3 * HIDDEN * FFN + EXPERTS * HIDDEN)
+    elif kind == "request":
+        nbytes, flops = _block_work(case["bits"], case["layers"], case["prompt"], 0)
+        for i in range(case["new"] - 1):
+            b, f = _block_work(case["bits"], case["layers"], 1, case["prompt"] + i)
+            nbytes, flops = nbytes + b, flops + f
+    elif kind == "offload":
+        nbytes, flops = 0, 0
+        for i in range(case["tokens"]):
+            b, f = _block_work(case["bits"], case["layers"], 1, case["cached"] + i)
+            nbytes, flops = nbytes + b, flops + f
+    elif kind == "prompt":
+        nbytes, flops = _block_work(case["bits"], case["layers"], case["tokens"], case["cached"])
+    else:  # at most twenty iterations of the solver, about ten operations a weight
+        n, k = case["n"], case["k"]
+        nbytes, flops = 2 * n * k + _layer_bytes(case["bits"], n, k), 200.0 * n * k
+    return {"bytes": int(nbytes), "flops": int(flops)}
+
+
+def tolerance(case):
+    """Relative error by kind of work, about four times what a comparison of each path with fp32 arithmetic on the same
+    de-quantised weights, or with another of the framework's own kernels, shows."""
+    kind = case["kind"]
+    if kind == "linear":
+        return {"rel": 2e-3}
+    if kind in ("ffn", "moe"):
+        return {"rel": 4e-3}
+    if kind in ("request", "offload", "prompt"):
+        return {"rel": 6e-3}
+    # the solver's last bits decide codes on a rounding boundary
+    return {"rel": 1e-3, "differ": 1e-3}
