@@ -301,3 +301,118 @@ def tolerance(case):
         return {"rel": 6e-3}
     # the solver's last bits decide codes on a rounding boundary
     return {"rel": 1e-3, "differ": 1e-3}
+
+
+# ------------------------------------------------------------------ the same in 64 bits
+def _codes64(packed, bits, n):
+    """(n, k) codes: field i of a packed row's F fields is output row F * row + i, the first field in the top bits."""
+    words = packed.as_subclass(torch.Tensor).to(torch.int64) & 0xFFFFFFFF
+    fields = 10 if bits == 3 else 8 // bits
+    rows = torch.stack([(words >> (bits * (fields - 1 - i))) & ((1 << bits) - 1) for i in range(fields)], dim=1)
+    return rows.reshape(-1, words.shape[1])[:n].double()
+
+
+def _table64(meta, which):
+    """A scale or zero table, one row per group: fp16, or 8-bit codes with fp16 scales and zeros of their own."""
+    if not meta.get("quant_" + which):
+        return meta[which].double().reshape(-1)
+    codes, inner = meta[which + "_q"].double().reshape(-1), meta["meta_" + which]
+    scale, zero = inner["scale"].double().reshape(-1), inner["zero"].double().reshape(-1)
+    return ((codes.reshape(-1, scale.numel()) - zero) * scale).reshape(-1)
+
+
+def _weight64(layer):
+    n, k = (int(v) for v in layer.meta["shape"])
+    scale, zero = _table64(layer.meta, "scale").reshape(-1, k), _table64(layer.meta, "zero").reshape(-1, k)
+    codes = _codes64(layer.W_q, layer.meta["nbits"], n).reshape(-1, scale.shape[0], k)  # row n belongs to group n mod G
+    return ((codes - zero) * scale).reshape(n, k)
+
+
+def _ffn64(weights, x):
+    a = x @ weights[0].T
+    return (a * torch.sigmoid(a) * (x @ weights[2].T)) @ weights[1].T
+
+
+def _moe64(gate, experts, x):
+    logits = x @ gate.T
+    probs, chosen = torch.softmax(logits, dim=1).topk(2, dim=1)
+    probs = probs / probs.sum(dim=1, keepdim=True)
+    out = torch.zeros_like(x)
+    for e in range(EXPERTS):
+        token, slot = torch.where(chosen == e)
+        if token.numel():
+            out[token] += probs[token, slot, None] * _ffn64(experts[e], x[token])
+    return out, logits
+
+
+def _block_weights64(block):
+    modules = [m._expert[0] for m in block.experts.resident_group(block.layer_id)]
+    return block.gate.weight.double(), [tuple(_weight64(w) for w in (m.w1, m.w2, m.w3)) for m in modules]
+
+
+def _model_weights64(model):
+    layers = []
+    for layer in model.model.layers:
+        attn = layer.self_attn
+        layers.append((layer.input_layernorm, [_weight64(p) for p in (attn.q_proj, attn.k_proj, attn.v_proj, attn.o_proj)],
+                       layer.post_attention_layernorm, *_block_weights64(layer.block_sparse_moe)))
+    return layers
+
+
+def _norm64(norm, x):
+    return norm.weight.double() * x * torch.rsqrt(x.pow(2).mean(dim=-1, keepdim=True) + norm.variance_epsilon)
+
+
+def _forward64(model, layers, ids):
+    """A whole sequence from the start: its logits, and every layer's rotated keys and its values (heads, tokens, size)."""
+    count, x, cache = ids.numel(), model.model.embed_tokens.weight[ids].double(), []
+    freq = 1.0 / model.config.rope_theta ** (torch.arange(0, HEAD_DIM, 2, device="cuda", dtype=torch.float64) / HEAD_DIM)
+    angle = torch.outer(torch.arange(count, device="cuda", dtype=torch.float64), freq)
+    cos, sin = torch.cat((angle, angle), dim=1).cos(), torch.cat((angle, angle), dim=1).sin()
+
+    def rotated(t):
+        return t * cos + torch.cat((-t[..., HEAD_DIM // 2:], t[..., :HEAD_DIM // 2]), dim=-1) * sin
+
+    later = torch.ones((count, count), dtype=torch.bool, device="cuda").triu(1)
+    for norm, (wq, wk, wv, wo), post, gate, experts in layers:
+        h = _norm64(norm, x)
+        q, k, v = ((h @ w.T).view(count, -1, HEAD_DIM).transpose(0, 1) for w in (wq, wk, wv))
+        q, k = rotated(q), rotated(k)
+        cache += [k, v.contiguous()]
+        heads = []
+        for i in range(HEADS):
+            j = i * KV_HEADS // HEADS
+            scores = (q[i] @ k[j].T / math.sqrt(HEAD_DIM)).masked_fill(later, float("-inf"))
+            heads.append(torch.softmax(scores, dim=-1) @ v[j])
+        x = x + torch.cat(heads, dim=1) @ wo.T
+        x = x + _moe64(gate, experts, _norm64(post, x))[0]
+    return _norm64(model.model.norm, x) @ model.lm_head.weight.double().T, cache
+
+
+@torch.no_grad()
+def exact(case, seed):
+    """What ``run`` gives, in 64 bits from the stored codes, tables and weights, nothing rounded on the way.  Not for
+    decoding behind a cache that ``prepare`` filled, and not for the quantiser, whose solver is defined in 32 bits."""
+    kind = case["kind"]
+    if kind in ("offload", "convert") or case.get("cached"):
+        return None
+    state = prepare(case, seed)
+    if kind == "linear":
+        return state["x"].double() @ _weight64(state["layer"]).T
+    if kind == "ffn":
+        return _ffn64([_weight64(getattr(state["expert"], w)) for w in ("w1", "w2", "w3")], state["x"].double())
+    if kind == "moe":
+        x = state["x"][0].double()
+        out, logits = _moe64(*_block_weights64(state["block"]), x)
+        return out[None], logits
+    model = state["model"]
+    layers = _model_weights64(model)
+    if kind == "prompt":
+        logits, cache = _forward64(model, layers, state["ids"])
+        return {"logits": logits, "cache": cache}
+    ids, made = state["prompt"], []
+    for _ in range(case["new"]):
+        logits = _forward64(model, layers, ids)[0][-1:]
+        made.append(logits.argmax(dim=-1))
+        ids = torch.cat((ids, made[-1]))
+    return {"ids": torch.cat(made), "logits": logits, "cache": [None] * (2 * case["layers"])}
