@@ -11,9 +11,17 @@
 // One thread owns CP neighbouring groups (4, 2 or 1, by what the registers hold) and keeps their values in registers,
 // so every iteration of the solver is register arithmetic; consecutive threads read consecutive pieces of a row, so
 // every row is a coalesced streaming read of 4 to 16 bytes per thread.  The solver
-// stops for the WHOLE tensor at once: a first pass adds up the error of every iteration (fp64 atomics), a one-thread
-// kernel finds the iteration the host loop would have stopped at, and a second pass repeats that many iterations and
-// writes the result.  All arithmetic is fp32 with separate multiplies and adds, as the tensor ops it replaces.
+// stops for the WHOLE tensor at once: passes of kQChunk iterations add up the error of every iteration (fp64 atomics)
+// and leave the zero points they reached in one of the two output vectors (the next pass reads it and writes the
+// other, so both ends of a pass are at hand); every block of a later pass finds from the errors so far whether the
+// host loop would have stopped, and returns if so; the last pass repeats the iterations of the one pass the stop fell
+// into and writes the result.  All arithmetic is fp32 with separate multiplies and adds, as the tensor ops it replaces.
+//
+// Bound by the vector units: an iteration is sixteen or so operations a value.  It was over a hundred: the shrinkage's
+// power took most of them and a full division the next, and all iterations ran before the stop was looked for.  The
+// power is evaluated only where its term can be other than zero (shrink_skip), the division is a reciprocal corrected
+// to the same rounding (divide_by).  14336 x 4096, 2-bit in groups of 16, stopped within the third of five passes: all
+// passes together 2185 -> 520 us, with the same bits; about 30 us an iteration.
 #include "hqq_common.hpp"
 
 #include <cmath>
@@ -23,6 +31,7 @@ namespace {
 
 constexpr int kQThreads = 256;
 constexpr int kQMaxIters = 64;
+constexpr int kQChunk = 4; // iterations between two looks at the stop: a pass more costs one read of the tensor
 
 struct QuantParams {
     const void *w;
@@ -37,7 +46,8 @@ struct QuantParams {
     float *inv_scale; // (cols)
     float *zero;      // (cols)
     double *err;      // [kQMaxIters] sums of |w - w_r| per iteration
-    int *stop;        // [1] iterations the second pass runs
+    int first;        // solver pass: its first iteration
+    float skip;       // shrink_skip(): residuals up to this one shrink to zero
 };
 
 // CP consecutive values starting at element `at` (a multiple of CP)
@@ -67,13 +77,100 @@ __device__ __forceinline__ float shrink_lp(float x, float inv_beta, float pm1)
     return x > 0.f ? r : (x < 0.f ? -r : 0.f);
 }
 
-// PASS 0: no refinement, write the result.  PASS 1: add up the error of every iteration.  PASS 2: run *p.stop
-// iterations, write the result.
+// x / s correctly rounded, from inv = 1 / s correctly rounded: the first two steps bring the quotient to within an ulp,
+// and one more correction by the exact residual rounds it as a division does (Markstein 1990), five operations for about
+// twice as many slots.  For |s| and |x| where neither residual nor quotient leaves the normal range: see divide_safe.
+__device__ __forceinline__ float divide_by(float x, float s, float inv)
+{
+    float q = x * inv;
+    q = __builtin_fmaf(__builtin_fmaf(-s, q, x), inv, q);
+    return __builtin_fmaf(__builtin_fmaf(-s, q, x), inv, q);
+}
+// x = q - zero with q whole: zero itself, or not below the distance of neighbouring floats around a whole number
+__device__ __forceinline__ bool divide_safe(float scale, float zero)
+{
+    const float a = __builtin_fabsf(zero);
+    return scale > 0x1p-60f && scale < 0x1p60f && (a == 0.f || (a > 0x1p-60f && a < 0x1p60f));
+}
+
+// One iteration of the solver on a column: its zero point moves, its error is returned.  The plain sums are made again
+// with divisions and the shrinkage in them where a lane of the wave may need either.
+template <int GS, int CP>
+__device__ __forceinline__ float solver_step(const QuantParams &p, const float (&w)[GS][CP], int j, float scale, float inv,
+                                             float inv_beta, float &zero)
+{
+    float e = 0.f, acc = 0.f, top = 0.f;
+#pragma unroll
+    for (int r = 0; r < GS; ++r) {
+        const float ws = w[r][j] * scale;
+        float q = __builtin_rintf(ws + zero);
+        q = __builtin_fminf(__builtin_fmaxf(q, 0.f), p.max_v);
+        const float a = __builtin_fabsf(w[r][j] - divide_by(q - zero, scale, inv));
+        e += a;
+        top = __builtin_fmaxf(top, a);
+        acc += q - ws;
+    }
+    if (__any(top > p.skip || !divide_safe(scale, zero))) {
+        const float pm1 = p.lp - 1.0f;
+        e = 0.f, acc = 0.f;
+#pragma unroll
+        for (int r = 0; r < GS; ++r) {
+            float q = __builtin_rintf(w[r][j] * scale + zero);
+            q = __builtin_fminf(__builtin_fmaxf(q, 0.f), p.max_v);
+            const float d = w[r][j] - (q - zero) / scale;
+            e += __builtin_fabsf(d);
+            const float we = shrink_lp(d, inv_beta, pm1);
+            acc += q - (w[r][j] - we) * scale;
+            __builtin_amdgcn_sched_barrier(0); // one power at a time: interleaved, their registers spill
+        }
+    }
+    zero = acc / (float)GS;
+    return e;
+}
+
+// The iteration count of the host loop, from the errors of its first `known` iterations: it updates zero, then stops at
+// the first iteration whose error (taken before the update) is not below the best so far.  0: not stopped yet.  All
+// threads of the block call it.
+__device__ __forceinline__ int solver_stop(const QuantParams &p, int known)
+{
+    __shared__ float mean[kQMaxIters];
+    __shared__ int stop;
+    if ((int)threadIdx.x < known)
+        mean[threadIdx.x] = (float)(p.err[threadIdx.x] / ((double)p.rows * (double)p.cols));
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float best = 1e4f;
+        int n = 0;
+        for (int it = 0; it < known && n == 0; ++it) {
+            if (mean[it] < best)
+                best = mean[it];
+            else
+                n = it + 1;
+        }
+        stop = n;
+    }
+    __syncthreads();
+    return stop;
+}
+
+// PASS 0: no refinement, write the result.  PASS 1: kQChunk iterations of the solver from p.first on, their errors added
+// up, unless an earlier one was the last.  PASS 2: the iterations that count of the pass the stop fell into, the result.
 template <int GS, int CP, int PASS> __global__ __launch_bounds__(kQThreads) void quantize_groups_kernel(QuantParams p)
 {
     const int64_t c = ((int64_t)blockIdx.x * kQThreads + threadIdx.x) * CP; // first group of the thread
     const bool on = c < p.cols;
     const int64_t cc = on ? c : p.cols - CP;
+    int first = 0, last = 0;
+    if constexpr (PASS == 1) {
+        if (p.first > 0 && solver_stop(p, p.first) != 0)
+            return;
+        first = p.first;
+        last = first + kQChunk < p.iters ? first + kQChunk : p.iters;
+    } else if constexpr (PASS == 2) {
+        last = solver_stop(p, p.iters);
+        last = last ? last : p.iters;
+        first = (last - 1) / kQChunk * kQChunk;
+    }
     float w[GS][CP];
 #pragma unroll
     for (int r = 0; r < GS; ++r)
@@ -94,28 +191,32 @@ template <int GS, int CP, int PASS> __global__ __launch_bounds__(kQThreads) void
             zero[j] = __builtin_rintf(zero[j]);
     }
     if constexpr (PASS != 0) {
-        const int iters = PASS == 1 ? p.iters : *p.stop;
-        __shared__ double red[kQThreads / 64];
+        // the pass at iteration f finds its zero points in p.zero if f / kQChunk is odd, in p.inv_scale if it is even
+        // (and not 0), and leaves them in the other one
+        const bool odd = (first / kQChunk) & 1;
+        if (first > 0) {
+            const float *from = odd ? p.zero : p.inv_scale;
+#pragma unroll
+            for (int j = 0; j < CP; ++j)
+                zero[j] = from[cc + j];
+        }
+        __shared__ double red[kQChunk][kQThreads / 64];
         double beta = p.beta; // the host loop keeps beta as a double and hands 1 / beta to fp32 tensor ops
-        const float pm1 = p.lp - 1.0f;
-        for (int it = 0; it < iters; ++it) {
+        for (int it = 0; it < first; ++it)
+            beta *= p.kappa;
+        float inv[CP];
+#pragma unroll
+        for (int j = 0; j < CP; ++j)
+            inv[j] = 1.0f / scale[j];
+#pragma unroll 1
+        for (int it = first; it < last; ++it) {
             const float inv_beta = (float)(1.0 / beta);
             float e = 0.f;
 #pragma unroll
             for (int j = 0; j < CP; ++j) {
-                float ej = 0.f, acc = 0.f;
-#pragma unroll
-                for (int r = 0; r < GS; ++r) {
-                    float q = __builtin_rintf(w[r][j] * scale[j] + zero[j]);
-                    q = __builtin_fminf(__builtin_fmaxf(q, 0.f), p.max_v);
-                    const float wr = (q - zero[j]) / scale[j];
-                    const float d = w[r][j] - wr;
-                    ej += __builtin_fabsf(d);
-                    const float we = shrink_lp(d, inv_beta, pm1);
-                    acc += q - (w[r][j] - we) * scale[j];
-                }
-                zero[j] = acc / (float)GS;
-                e += ej;
+                float sc = scale[j];
+                asm volatile("" : "+v"(sc)); // keeps w * scale out of registers of its own across iterations
+                e += solver_step<GS, CP>(p, w, j, sc, inv[j], inv_beta, zero[j]);
             }
             beta *= p.kappa;
             if constexpr (PASS == 1) {
@@ -124,15 +225,22 @@ template <int GS, int CP, int PASS> __global__ __launch_bounds__(kQThreads) void
                 for (int off = 32; off > 0; off >>= 1)
                     s += __shfl_xor(s, off, 64);
                 if ((threadIdx.x & 63) == 0)
-                    red[threadIdx.x >> 6] = s;
-                __syncthreads();
-                if (threadIdx.x == 0) {
-                    double t = 0.0;
-                    for (int i = 0; i < kQThreads / 64; ++i)
-                        t += red[i];
-                    atomicAdd(&p.err[it], t);
-                }
-                __syncthreads();
+                    red[it - first][threadIdx.x >> 6] = s;
+            }
+        }
+        if constexpr (PASS == 1) {
+            __syncthreads();
+            if ((int)threadIdx.x < last - first) {
+                double t = 0.0;
+                for (int i = 0; i < kQThreads / 64; ++i)
+                    t += red[threadIdx.x][i];
+                atomicAdd(&p.err[first + threadIdx.x], t);
+            }
+            if (on) {
+                float *to = odd ? p.inv_scale : p.zero;
+#pragma unroll
+                for (int j = 0; j < CP; ++j)
+                    to[c + j] = zero[j];
             }
         }
     }
@@ -167,30 +275,23 @@ template <int GS, int CP, int PASS> __global__ __launch_bounds__(kQThreads) void
     }
 }
 
-// the iteration count of the host loop: it updates zero, then stops at the first iteration whose error (taken before
-// the update) is not below the best so far
-__global__ void quantize_stop_kernel(const double *err, int iters, double numel, int *stop)
-{
-    float best = 1e4f;
-    int n = iters;
-    for (int it = 0; it < iters; ++it) {
-        const float e = (float)(err[it] / numel);
-        if (e < best) {
-            best = e;
-        } else {
-            n = it + 1;
-            break;
-        }
-    }
-    *stop = n;
-}
-
-__global__ void quantize_clear_kernel(double *err, int *stop)
+__global__ void quantize_clear_kernel(double *err)
 {
     if (threadIdx.x < kQMaxIters)
         err[threadIdx.x] = 0.0;
-    if (threadIdx.x == 0)
-        *stop = 0;
+}
+
+// The largest residual a of which it is certain that a - (1 / beta) (a + 1e-8)^(p - 1) is not positive, in whatever
+// iteration: the difference grows with a and is zero at a = (1 / beta)^(1 / (2 - p)) but for the 1e-8; two per cent below
+// that it is negative by more than two per cent of a, a thousand times what the 1e-8 and the roundings can add.
+// (p = 0.7, 1 / beta = 0.1: 0.14; a residual is at most half a quantisation step, so trained weights never get there.)
+static float shrink_skip(double beta, double kappa, int iters, float lp)
+{
+    const double last = beta * std::pow(kappa, (double)iters), most = last > beta ? last : beta;
+    if (!(lp >= 0.0f && lp <= 1.0f) || !(beta > 0) || !(last > 0) || !(most < 1e30))
+        return -1.0f; // never skipped
+    const double at = 0.98 * std::pow(1.0 / most, 1.0 / (2.0 - (double)lp));
+    return at > 1e-4 ? (float)at : -1.0f;
 }
 
 // One group for the whole tensor (channel_wise = False).  Three launches: the extremes are cleared, every block
@@ -209,12 +310,30 @@ __global__ void whole_clear_kernel(int *extremes)
     extremes[1] = (int)0x80000000; // max
 }
 
+// Four 16-byte loads a thread and trip where the pointer allows, and few blocks: with one 4-byte load a trip and a block
+// per 2048 values the blocks' atomics on the two words, not the reading, took the time (3.7 M values: 44.5 -> 9.4 us).
 __global__ __launch_bounds__(256) void whole_extremes_kernel(const float *x, int64_t n, int *extremes)
 {
+    typedef float vec4 __attribute__((ext_vector_type(4)));
     __shared__ float mn_s[4], mx_s[4];
-    const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
     float mn = x[first < n ? first : 0], mx = mn;
-    for (int64_t i = first; i < n; i += (int64_t)gridDim.x * 256) {
+    const int64_t quads = (reinterpret_cast<uintptr_t>(x) & 15u) == 0 ? n / 4 : 0;
+    const vec4 *xv = reinterpret_cast<const vec4 *>(x);
+    for (int64_t i = first; i < quads; i += 4 * stride) {
+        vec4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            v[u] = xv[i + u * stride < quads ? i + u * stride : i];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                mn = __builtin_fminf(mn, v[u][e]);
+                mx = __builtin_fmaxf(mx, v[u][e]);
+            }
+    }
+    for (int64_t i = 4 * quads + first; i < n; i += stride) {
         mn = __builtin_fminf(mn, x[i]);
         mx = __builtin_fmaxf(mx, x[i]);
     }
@@ -262,9 +381,10 @@ template <int GS, int CP> int run_groups_cp(const QuantParams &p, hipStream_t s)
         quantize_groups_kernel<GS, CP, 0><<<blocks, kQThreads, 0, s>>>(p);
         return launch_status();
     }
-    quantize_clear_kernel<<<1, 64, 0, s>>>(p.err, p.stop);
-    quantize_groups_kernel<GS, CP, 1><<<blocks, kQThreads, 0, s>>>(p);
-    quantize_stop_kernel<<<1, 1, 0, s>>>(p.err, p.iters, (double)p.rows * (double)p.cols, p.stop);
+    quantize_clear_kernel<<<1, 64, 0, s>>>(p.err);
+    QuantParams q = p;
+    for (q.first = 0; q.first < p.iters; q.first += kQChunk)
+        quantize_groups_kernel<GS, CP, 1><<<blocks, kQThreads, 0, s>>>(q);
     quantize_groups_kernel<GS, CP, 2><<<blocks, kQThreads, 0, s>>>(p);
     return launch_status();
 }
@@ -308,7 +428,7 @@ int launch_quantize_groups(const void *w, int fp32_in, int64_t rows, int64_t col
     p.lp = lp, p.beta = beta, p.kappa = kappa;
     p.codes = codes, p.inv_scale = inv_scale, p.zero = zero;
     p.err = static_cast<double *>(ws);
-    p.stop = reinterpret_cast<int *>(static_cast<char *>(ws) + kQMaxIters * sizeof(double));
+    p.skip = shrink_skip(beta, kappa, iters, lp);
     switch (rows) {
     case 8: return run_groups<8>(p, s);
     case 16: return run_groups<16>(p, s);
@@ -330,7 +450,8 @@ int launch_quantize_whole(const float *x, int64_t n, int nbits, uint8_t *codes, 
     int64_t blocks = (n + 256 * 8 - 1) / (256 * 8);
     blocks = blocks < 1 ? 1 : (blocks > 2048 ? 2048 : blocks);
     whole_clear_kernel<<<1, 1, 0, s>>>(extremes);
-    whole_extremes_kernel<<<(unsigned)blocks, 256, 0, s>>>(x, n, extremes);
+    const int64_t few = blocks < 256 ? blocks : 256;
+    whole_extremes_kernel<<<(unsigned)few, 256, 0, s>>>(x, n, extremes);
     whole_codes_kernel<<<(unsigned)blocks, 256, 0, s>>>(x, n, (float)((1 << nbits) - 1), extremes, codes, inv_scale, zero);
     return launch_status();
 }

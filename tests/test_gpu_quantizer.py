@@ -114,3 +114,32 @@ def test_layer_quantised_on_the_gpu_equals_the_oracle_layer():
             for f in ("scale", "zero"):
                 got = layer.meta[t][f].cpu().numpy().reshape(-1)
                 assert np.array_equal(got.view(np.uint16), np.asarray(want[t][f], dtype=np.float16).reshape(-1).view(np.uint16)), (nbits, t, f)
+
+
+@pytest.mark.parametrize("kind", ["wide", "constant", "huge", "offset"])
+@pytest.mark.parametrize("nbits,gs", [(2, 8), (2, 16), (3, 64), (4, 128)])
+def test_solver_where_its_short_cuts_do_not_hold(kind, nbits, gs):
+    """Residuals large enough for the shrinkage to leave something (weights tens wide), groups without a spread, and
+    scales and zeros outside the range in which the quotient is corrected without a division: the tensor-op form's
+    results.  The solver's zero is a mean of gs fp32 terms of size |w| * scale, so another order of that sum moves it by
+    gs * 2^-24 of the largest."""
+    from mixtral_offloading_amd import hip_kernels
+    rng = np.random.default_rng(nbits * 1000 + gs)
+    n, k = gs * 3, 84
+    w = rng.standard_normal((n, k)).astype(np.float32)
+    if kind == "wide":
+        w *= 30
+    elif kind == "constant":
+        w[:, ::3] = 0.25
+    elif kind == "huge":
+        w[:, ::2] *= np.float32(2.0 ** 70)
+    else:
+        w = w * np.float32(1e-3) + 50
+    q, scale, zero = o.hqq_quantize_tensor(w, nbits, gs, optimize=True, round_zero=(nbits == 4), iters=6)
+    gq, gscale, gzero = hip_kernels.quantize_groups(torch.from_numpy(w).cuda(), gs, nbits, round_zero=(nbits == 4), iters=6)
+    gq, gscale, gzero = gq.cpu().numpy(), gscale.cpu().numpy().reshape(-1), gzero.cpu().numpy().reshape(-1)
+    assert np.array_equal(gscale, scale.reshape(-1))
+    terms = np.abs(w.reshape(gs, -1).astype(np.float64) / scale.reshape(1, -1)).max(axis=0) + 2 ** nbits
+    assert (np.abs(gzero - zero.reshape(-1)) <= 1e-4 * 2 ** nbits + 6 * gs * 2.0 ** -24 * terms).all()
+    moved = np.abs(gq.astype(int) - q.astype(int))
+    assert moved.max() <= 1 and (moved != 0).mean() <= (0.02 if kind == "offset" else 2e-3)
