@@ -256,6 +256,15 @@ int hqq_rope_append_rows(void *q_f16, const void *k_f16, const void *v_f16, cons
                          int64_t start, int64_t rows, void *cache_k_f16, void *cache_v_f16, int64_t max_len,
                          int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, void *stream);
 
+/* ---- causal attention of `rows` new tokens at positions start .. start + rows - 1 over their sequence's cache (HF
+ *      transformers' Mixtral attention in the reference): q (rows, n_heads*head_dim) rotated, cache_k / cache_v
+ *      [n_kv_heads][max_len][head_dim] with positions 0 .. start + rows - 1 filled (hqq_rope_append_rows does both);
+ *      token t attends positions 0 .. start + t.  out (rows, n_heads*head_dim), not overlapping the inputs.  Scores,
+ *      softmax and sums in fp32, probabilities enter the product with the values in fp16.  head_dim 64 or 128, n_heads
+ *      a multiple of n_kv_heads, all pointers 16-byte aligned.                                                       */
+int hqq_attention_rows(const void *q_f16, const void *cache_k_f16, const void *cache_v_f16, int64_t start, int64_t rows,
+                       int64_t max_len, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, void *out_f16, void *stream);
+
 /* ---- hqq_add_rmsnorm followed by hqq_router_top2 on its output y, in one launch: the post-attention norm of a
  *      decoder layer and the router that reads it (src/custom_layers.py:276-282).  x and y as hqq_add_rmsnorm gives
  *      them; logits as hqq_router_top2 up to the order of the fp32 sums.                                           */

@@ -633,6 +633,28 @@ def rope_append_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: tor
     return q
 
 
+def attention_rows_supported(q: torch.Tensor, cache_k: torch.Tensor, cache_v: torch.Tensor) -> bool:
+    """Whether ``attention_rows`` takes q (tokens, heads, hd) and caches (kv_heads, max_len, hd) of these forms."""
+    return (q.shape[-1] in (64, 128) and cache_k.shape == cache_v.shape and q.shape[1] % cache_k.shape[0] == 0
+            and all(t.is_cuda and t.dtype == torch.float16 and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for t in (q, cache_k, cache_v)))
+
+
+def attention_rows(q: torch.Tensor, cache_k: torch.Tensor, cache_v: torch.Tensor, start: int) -> torch.Tensor:
+    """Causal attention of the new tokens of one sequence: ``q`` (tokens, heads, hd) rotated, caches (kv_heads, max_len,
+    hd) filled up to position ``start + tokens - 1``.  Returns (tokens, heads * hd)."""
+    T, n_heads, hd = q.shape
+    n_kv, max_len = cache_k.shape[0], cache_k.shape[1]
+    assert attention_rows_supported(q, cache_k, cache_v) and cache_k.shape[2] == hd and 0 <= start and start + T <= max_len
+    out = torch.empty((T, n_heads * hd), dtype=torch.float16, device=q.device)
+    if T:
+        with _on(q.device):
+            _lib.check(_lib.lib.hqq_attention_rows(q.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), int(start), T, max_len,
+                                                   n_heads, n_kv, hd, out.data_ptr(), _lib.current_stream_ptr(q.device)),
+                       "hqq_attention_rows")
+    return out
+
+
 _attention_workspaces = {}  # (device, stream) -> zero-filled bytes for the split attention launch
 
 

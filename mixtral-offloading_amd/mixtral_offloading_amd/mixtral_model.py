@@ -97,6 +97,8 @@ class Attention(nn.Module):
             from . import hip_kernels
 
             hip_kernels.rope_append_rows(q, k, v, rotary.cos, rotary.sin, start, cache_k, cache_v)
+            if hip_kernels.attention_rows_supported(q, cache_k, cache_v):
+                return self.o_proj(hip_kernels.attention_rows(q, cache_k, cache_v, start))
         else:
             positions = torch.arange(start, start + T, device=x.device)
             q, k = rotary.apply(q, k, positions)
