@@ -418,9 +418,20 @@ int hqq_expert_ffn(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear 
                            nullptr, nullptr);
 }
 
+// Whether an expert's FFN at M rows is two launches of the batch kernel, so that several can share them: exactly the
+// calls for which expert_ffn_impl takes that kernel for the gate and for the down projection.
+static bool ffn_runs_batch_kernel(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, int64_t M)
+{
+    return batch_group_class(M) >= 0 && !tuning_flag("HQQ_BATCH_OFF") && validate_linear(w1) == HQQ_OK &&
+           validate_linear(w2) == HQQ_OK && validate_linear(w3) == HQQ_OK && w2->K == w1->N && w2->N == w1->K && !w1->bias &&
+           !w3->bias && batch_gate_supported(w1, w3, M) && batch_supported(w2, M) && pick_family(w1, M) == FAM_SMALLBATCH &&
+           pick_family(w3, M) == FAM_SMALLBATCH && pick_family(w2, M) == FAM_SMALLBATCH;
+}
+
 // ---- the experts of one MoE layer over rows already grouped by expert: hqq_expert_ffn once per group, from one call
-// Workspace of the grouped call: what the largest group needs, then the partial sums of every group whose down
-// projection leaves its finishing pass to the end of the call.
+// Workspace of the grouped call: what the largest group needs, then what outlives a group's own launches: the partial
+// sums of every group whose down projection leaves its finishing pass to the end of the call, and silu(a) * b of every
+// group that shares its launches with others.
 static size_t groups_common_bytes(const hqq_linear *const *w1, const hqq_linear *const *w2, const hqq_linear *const *w3,
                                   int32_t n_groups, const int64_t *row_start, size_t *parts)
 {
@@ -438,6 +449,8 @@ static size_t groups_common_bytes(const hqq_linear *const *w1, const hqq_linear 
         need = one > need ? one : need;
         if (down_finish_deferrable(w2[g], M))
             *parts += tile_partial_bytes(w2[g], M);
+        if (ffn_runs_batch_kernel(w1[g], w2[g], w3[g], M)) // silu(a) * b of an expert that shares launches
+            *parts += align256((size_t)M * (size_t)w1[g]->N * sizeof(f16));
     }
     return align256(need);
 }
@@ -475,9 +488,57 @@ int hqq_expert_groups_ffn(const hqq_linear *const *w1, const hqq_linear *const *
     TileFinish fin[kTileFinishGroupMax];
     int nf = 0;
     char *part_at = static_cast<char *>(workspace) + common;
+    // Groups of 3 to 16 rows, by class of the batch kernel: the gates of a class as one launch, then its down projections
+    // (class by class: with fewer than two members there is nothing to share, and the loop below takes the group).
+    // Every group's rows and results are its own, so the order of the groups does not matter.
+    uint64_t done = 0; // groups finished here; those beyond the 64th are left to the loop below
+    if (defer && x_f16 && y_f16 && (reinterpret_cast<uintptr_t>(workspace) & 255u) == 0 && (reinterpret_cast<uintptr_t>(x_f16) & 15u) == 0) {
+        uint64_t eligible = 0;
+        for (int g = 0; g < n_groups && g < 64; ++g) {
+            const int64_t M = row_start[g + 1] - row_start[g];
+            if (M > 0 && ffn_runs_batch_kernel(w1[g], w2[g], w3[g], M))
+                eligible |= 1ull << g;
+        }
+        for (int lead = 0; lead < n_groups && lead < 64; ++lead) {
+            if (!(eligible >> lead & 1) || (done >> lead & 1))
+                continue;
+            const int64_t lead_rows = row_start[lead + 1] - row_start[lead];
+            const hqq_linear *const first[3] = {w1[lead], w2[lead], w3[lead]};
+            BatchGroupItem gate[64], down[64];
+            uint64_t taken = 0;
+            int n = 0;
+            for (int g = lead; g < n_groups && g < 64; ++g) {
+                const int64_t lo = row_start[g], M = row_start[g + 1] - lo;
+                if (!(eligible >> g & 1) || (done >> g & 1) || batch_group_class(M) != batch_group_class(lead_rows))
+                    continue;
+                const hqq_linear *const l[3] = {w1[g], w2[g], w3[g]};
+                if (!batch_group_ffn_alike(first, l, M))
+                    continue;
+                const f16 *x = static_cast<const f16 *>(x_f16) + lo * w1[g]->K;
+                f16 *y = static_cast<f16 *>(y_f16) + lo * w2[g]->N;
+                gate[n] = BatchGroupItem{w1[g], w3[g], x, M, nullptr, nullptr};
+                down[n] = BatchGroupItem{w2[g], nullptr, nullptr, M, y, row_scale_f16 ? static_cast<const f16 *>(row_scale_f16) + lo : nullptr};
+                taken |= 1ull << g;
+                ++n;
+            }
+            if (n < 2)
+                continue;
+            for (int i = 0; i < n; ++i) {
+                gate[i].y = reinterpret_cast<f16 *>(part_at);
+                down[i].x = gate[i].y;
+                part_at += align256((size_t)gate[i].M * (size_t)gate[i].l0->N * sizeof(f16));
+            }
+            int rc = launch_batch_group(gate, n, true, workspace, common, (hipStream_t)stream);
+            if (rc == HQQ_OK)
+                rc = launch_batch_group(down, n, false, workspace, common, (hipStream_t)stream);
+            if (rc != HQQ_OK)
+                return rc;
+            done |= taken;
+        }
+    }
     for (int g = 0; g < n_groups; ++g) {
         const int64_t lo = row_start[g], M = row_start[g + 1] - lo;
-        if (M == 0)
+        if (M == 0 || (g < 64 && (done >> g & 1)))
             continue;
         const char *x = static_cast<const char *>(x_f16) + (size_t)lo * (size_t)w1[g]->K * 2;
         char *y = static_cast<char *>(y_f16) + (size_t)lo * (size_t)w2[g]->N * 2;

@@ -156,6 +156,18 @@ bool strip_gate_supported(const hqq_linear *w1, const hqq_linear *w3, int64_t M)
 bool batch_supported(const hqq_linear *l, int64_t M);
 bool batch_gate_supported(const hqq_linear *w1, const hqq_linear *w3, int64_t M);
 size_t batch_workspace_bytes(const hqq_linear *l, int64_t M);
+// experts of one MoE layer in common launches: one item per expert, all of one batch_group_class and alike
+struct BatchGroupItem {
+    const hqq_linear *l0, *l1; // l1: the gate's second projection
+    const f16 *x;
+    int64_t M;
+    f16 *y;
+    const f16 *row_scale;
+};
+constexpr int kBatchGroupMax = 16; // members of a launch: their records travel in the kernel arguments
+int batch_group_class(int64_t M); // 0 .. 2, or -1: not a size the batch kernel takes
+bool batch_group_ffn_alike(const hqq_linear *const first[3], const hqq_linear *const l[3], int64_t M);
+int launch_batch_group(const BatchGroupItem *item, int n, bool gate, void *ws, size_t ws_bytes, hipStream_t s);
 int launch_batch_matmul(const hqq_linear *l, const f16 *x, int64_t M, f16 *y, void *ws, size_t ws_bytes,
                         const SmallBatchEpilogue &ep, hipStream_t s, const StripIndex *ix = nullptr);
 int launch_batch_gate_up(const hqq_linear *w1, const hqq_linear *w3, const f16 *x, int64_t M, f16 *h, void *ws,

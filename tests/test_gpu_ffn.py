@@ -224,3 +224,32 @@ def test_expert_groups_at_full_size_leave_the_finishing_passes_to_the_end():
         assert torch.equal(out, each)
         one = hip_kernels.expert_ffn(descs[0][0], descs[0][1], descs[0][2], x[:1].contiguous())
         assert bool(torch.isfinite(one).all())
+
+
+@pytest.mark.parametrize("nbits,gs", [(2, 16), (4, 64)])
+@pytest.mark.parametrize("counts", [[3, 4, 3], [5, 3, 8, 4, 0, 7, 2, 1], [9, 16, 17, 4], [4] * 6 + [8] * 3])
+def test_expert_groups_of_decode_size_share_launches(nbits, gs, counts):
+    """Experts with 3 to 16 rows share the batch kernel's launches, by class of rows (up to four, eight, sixteen) and as
+    many as the accumulation slots of a K split hold (four experts of four rows, two of eight, at 4096 outputs).  Each
+    block sums what it sums alone: bit for bit one call per expert, again on the second call (slots left at zero)."""
+    from mixtral_offloading_amd import hip_kernels
+    from test_gpu_matmul import _full_size_layer
+    hidden, ffn = 4096, 7168  # the down projection splits K over blocks, the gate holds all of it
+    shapes = ((ffn, hidden), (hidden, ffn), (ffn, hidden))
+    descs = [tuple(_full_size_layer(nbits, n, k, gs, seed=3 * e + i) for i, (n, k) in enumerate(shapes)) for e in range(len(counts))]
+    group = hip_kernels.ExpertGroup(descs)
+    starts = np.concatenate(([0], np.cumsum(counts)))
+    rows = int(starts[-1])
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn((rows, hidden), device="cuda", generator=g).half()
+    scale = (torch.rand((rows,), device="cuda", generator=g) * 0.6 + 0.2).half()
+    each = torch.empty((rows, hidden), dtype=torch.float16, device="cuda")
+    for row_scale in (scale, None, scale):
+        for e, (w1, w2, w3) in enumerate(descs):
+            lo, hi = int(starts[e]), int(starts[e + 1])
+            if hi > lo:
+                hip_kernels.expert_ffn(w1, w2, w3, x[lo:hi], out=each[lo:hi],
+                                       row_scale=None if row_scale is None else row_scale[lo:hi])
+        out = torch.full((rows, hidden), 3.0, dtype=torch.float16, device="cuda")
+        hip_kernels.expert_groups_ffn(group, x, starts, row_scale, out)
+        assert bool(torch.isfinite(each).all()) and torch.equal(out, each)
