@@ -224,6 +224,11 @@ int hqq_matmul_group_norm(const hqq_linear *const *layers, int32_t count, const 
 int hqq_router_top2(const void *x_f16, const void *gate_w_f16, int32_t n_experts, int64_t hidden, int32_t *sel_out,
                     void *weights_f16_out, void *logits_f16_out, void *stream);
 
+/* ---- the end of a greedy decode step: the n logits of one token copied to out, the index of the largest (the first of
+ *      equal ones; a NaN counts as larger than any number) to *token, and *position += 1.  logits and out are 16-byte
+ *      aligned and do not overlap; all pointers are device memory.                                                   */
+int hqq_next_token(const void *logits_f16, int64_t n, void *out_f16, int64_t *token, int64_t *position, void *stream);
+
 /* ---- residual add and RMSNorm of one token (the reference takes both from HF transformers' Mixtral decoder layer):
  *      x += delta in fp16 when delta is not NULL (x is written back), y = weight * fp16(x * rsqrt(mean(x^2) + eps)). */
 int hqq_add_rmsnorm(void *x_f16, const void *delta_f16, const void *weight_f16, float eps, void *y_f16, int64_t hidden,

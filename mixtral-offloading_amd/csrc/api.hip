@@ -855,6 +855,13 @@ int hqq_router_top2(const void *x_f16, const void *gate_w_f16, int32_t n_experts
                               (f16 *)weights_f16_out, (f16 *)logits_f16_out, (hipStream_t)stream);
 }
 
+int hqq_next_token(const void *logits_f16, int64_t n, void *out_f16, int64_t *token, int64_t *position, void *stream)
+{
+    if (!logits_f16 || !out_f16 || !token || !position)
+        return HQQ_E_NULL;
+    return launch_next_token((const f16 *)logits_f16, n, (f16 *)out_f16, token, position, (hipStream_t)stream);
+}
+
 int hqq_add_rmsnorm(void *x_f16, const void *delta_f16, const void *weight_f16, float eps, void *y_f16, int64_t hidden,
                     void *stream)
 {

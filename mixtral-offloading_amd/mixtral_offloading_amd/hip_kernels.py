@@ -538,6 +538,16 @@ def router_top2(x: torch.Tensor, gate_weight: torch.Tensor, sel: torch.Tensor, w
                                             _lib.current_stream_ptr(x.device)), "hqq_router_top2")
 
 
+def next_token(logits: torch.Tensor, out: torch.Tensor, token: torch.Tensor, position: torch.Tensor) -> None:
+    """The end of a greedy decode step: ``out = logits`` (one row), ``token = logits.argmax()``, ``position += 1``."""
+    assert logits.dtype == out.dtype == torch.float16 and logits.is_contiguous() and out.is_contiguous()
+    assert logits.numel() == out.numel() and token.dtype == position.dtype == torch.int64
+    assert token.numel() == 1 and position.numel() == 1
+    with _on(logits.device):
+        _lib.check(_lib.lib.hqq_next_token(logits.data_ptr(), logits.numel(), out.data_ptr(), token.data_ptr(),
+                                           position.data_ptr(), _lib.current_stream_ptr(logits.device)), "hqq_next_token")
+
+
 def add_rmsnorm(x: torch.Tensor, delta: Optional[torch.Tensor], weight: torch.Tensor, eps: float,
                 out: torch.Tensor) -> torch.Tensor:
     """``x += delta`` (when given) then ``out = weight * rmsnorm(x)`` for one token."""

@@ -251,9 +251,13 @@ class DecodeGraph:
                 hip_kernels.expert_ffn_indexed(table, self.sel[1:2], self.xn, self.moe, row_scale=self.rw[1:2], accumulate=True)
             delta = self.moe
         hip_kernels.add_rmsnorm(x, delta, m.model.norm.weight, eps, self.xn)
-        self.logits.copy_(m.lm_head(self.xn))
-        self.tok.copy_(self.logits.argmax(-1))
-        self.pos.add_(1)
+        logits = m.lm_head(self.xn)
+        if logits.dtype == torch.float16 and logits.is_contiguous() and logits.data_ptr() % 16 == 0:
+            hip_kernels.next_token(logits, self.logits, self.tok, self.pos)
+        else:  # another head in the model's place
+            self.logits.copy_(logits)
+            self.tok.copy_(self.logits.argmax(-1))
+            self.pos.add_(1)
 
     def capture(self):
         """Warm up on a side stream (workspaces and allocator pools get their final size), then record the step."""
