@@ -252,6 +252,14 @@ int hqq_router_top2_rows(const void *x_f16, const void *gate_w_f16, int32_t n_ex
 int hqq_moe_group_pairs(const int32_t *sel, const void *weights_f16, int64_t tokens, int32_t n_experts, int32_t *counts_out,
                         int64_t *token_of_row_out, void *scale_of_row_f16_out, void *stream);
 
+/* ---- the same, and for every pair p the row it went to (-1: its expert is out of range): row_of_pair_out[2 * tokens];
+ *      and the sum that undoes the grouping (src/custom_layers.py:307-312): y[t] = the rows of token t's two pairs added
+ *      in fp16, first slot first, beginning from zero.  rows and y are 16-byte aligned, hidden a multiple of 8.      */
+int hqq_moe_group_pairs_rows(const int32_t *sel, const void *weights_f16, int64_t tokens, int32_t n_experts,
+                             int32_t *counts_out, int64_t *token_of_row_out, void *scale_of_row_f16_out,
+                             int32_t *row_of_pair_out, void *stream);
+int hqq_moe_combine(const void *rows_f16, const int32_t *row_of_pair, int64_t tokens, int64_t hidden, void *y_f16, void *stream);
+
 /* ---- rotary embedding and KV-cache append of `rows` new tokens at positions start .. start + rows - 1 (HF
  *      transformers' apply_rotary_pos_emb in the reference's Mixtral attention): q (rows, n_heads*head_dim) is rotated
  *      in place, the rotated k (rows, n_kv_heads*head_dim) and v are written to cache_k / cache_v

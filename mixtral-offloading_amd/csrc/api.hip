@@ -896,7 +896,25 @@ int hqq_moe_group_pairs(const int32_t *sel, const void *weights_f16, int64_t tok
         return HQQ_E_NULL;
     return launch_moe_group_pairs(sel, (const f16 *)weights_f16, tokens, n_experts, counts_out,
                                   reinterpret_cast<long long *>(token_of_row_out), (f16 *)scale_of_row_f16_out,
-                                  (hipStream_t)stream);
+                                  nullptr, (hipStream_t)stream);
+}
+
+int hqq_moe_group_pairs_rows(const int32_t *sel, const void *weights_f16, int64_t tokens, int32_t n_experts,
+                             int32_t *counts_out, int64_t *token_of_row_out, void *scale_of_row_f16_out,
+                             int32_t *row_of_pair_out, void *stream)
+{
+    if (!sel || !weights_f16 || !counts_out || !token_of_row_out || !scale_of_row_f16_out || !row_of_pair_out)
+        return HQQ_E_NULL;
+    return launch_moe_group_pairs(sel, (const f16 *)weights_f16, tokens, n_experts, counts_out,
+                                  reinterpret_cast<long long *>(token_of_row_out), (f16 *)scale_of_row_f16_out,
+                                  row_of_pair_out, (hipStream_t)stream);
+}
+
+int hqq_moe_combine(const void *rows_f16, const int32_t *row_of_pair, int64_t tokens, int64_t hidden, void *y_f16, void *stream)
+{
+    if (!rows_f16 || !row_of_pair || !y_f16)
+        return HQQ_E_NULL;
+    return launch_moe_combine((const f16 *)rows_f16, row_of_pair, tokens, hidden, (f16 *)y_f16, (hipStream_t)stream);
 }
 
 int hqq_rope_append_rows(void *q_f16, const void *k_f16, const void *v_f16, const void *cos_f16, const void *sin_f16,

@@ -59,6 +59,8 @@ _SIGNATURES = {
     "hqq_expert_groups_ffn_workspace_bytes": (c_size_t, [c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
     "hqq_expert_groups_ffn": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                       c_size_t, c_void_p]),
+    "hqq_moe_group_pairs_rows": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "hqq_moe_combine": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p]),
     "hqq_moe_group_pairs": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
     "hqq_gate_up_workspace_bytes": (c_size_t, [_P(HqqLinear), _P(HqqLinear), c_int64]),
     "hqq_gate_up": (c_int, [_P(HqqLinear), _P(HqqLinear), c_void_p, c_int64, c_void_p, c_void_p, c_size_t, c_void_p]),
@@ -77,9 +79,9 @@ _SIGNATURES = {
     "hqq_matmul_group_norm": (c_int, [_P(_P(HqqLinear)), c_int32, c_void_p, c_void_p, c_void_p, ctypes.c_float, c_void_p,
                                       _P(c_void_p), c_void_p, c_size_t, c_void_p]),
     "hqq_router_top2": (c_int, [c_void_p, c_void_p, c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "hqq_next_token": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "hqq_add_rmsnorm": (c_int, [c_void_p, c_void_p, c_void_p, ctypes.c_float, c_void_p, c_int64, c_void_p]),
     "hqq_add_rmsnorm_rows": (c_int, [c_void_p, c_void_p, c_void_p, ctypes.c_float, c_void_p, c_int64, c_int64, c_void_p]),
-    "hqq_next_token": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "hqq_router_top2_rows": (c_int, [c_void_p, c_void_p, c_int32, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "hqq_rope_append_rows": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p,
                                      c_int64, c_int32, c_int32, c_int32, c_void_p]),

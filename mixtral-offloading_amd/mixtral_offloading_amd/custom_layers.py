@@ -299,13 +299,13 @@ class SparseMoeWrapper(nn.Module):
             routing_weights = routing_weights.to(hidden_states.dtype)
 
         tokens = hidden_states.shape[0]
-        final_hidden_states = torch.zeros((tokens, hidden_dim), dtype=hidden_states.dtype, device=hidden_states.device)
         if tokens > 1 and selected_experts.dtype == torch.int32 and routing_weights.dtype == torch.float16:
             # Several tokens, router on the device: the (token, slot) pairs are grouped by expert there as well, the
             # rows of every expert are gathered at once, and only then does the host wait, for the experts' row counts
             # alone (reference :288-312 does a where / gather / index_add_ per expert).  Each token receives the same
-            # two fp16 terms in the index_add_ below, and their sum does not depend on the order.
-            counts_dev, top_x, scales = hip_kernels.moe_group_pairs(selected_experts, routing_weights, self.num_experts)
+            # two fp16 terms, and their sum does not depend on the order.
+            counts_dev, top_x, scales, row_of_pair = hip_kernels.moe_group_pairs_rows(selected_experts, routing_weights,
+                                                                                      self.num_experts)
             gathered = hidden_states.index_select(0, top_x)
             weighted = torch.empty_like(gathered)
             group = self._resident_group()
@@ -320,8 +320,9 @@ class SparseMoeWrapper(nn.Module):
                         *((self.layer_id, expert_idx) for expert_idx in active_experts), unordered=True):
                     lo, hi = int(starts[expert_idx]), int(starts[expert_idx + 1])
                     expert_layer(gathered[lo:hi], out=weighted[lo:hi], row_scale=scales[lo:hi])
-            final_hidden_states.index_add_(0, top_x, weighted)
-            return final_hidden_states.reshape(batch_size, sequence_length, hidden_dim), router_logits
+            combined = hip_kernels.moe_combine(weighted, row_of_pair)
+            return combined.reshape(batch_size, sequence_length, hidden_dim), router_logits
+        final_hidden_states = torch.zeros((tokens, hidden_dim), dtype=hidden_states.dtype, device=hidden_states.device)
         sel_host = selected_experts.cpu()  # one host sync per layer: the cache is driven from the host
         if tokens == 1:
             selected = sel_host[0].tolist()

@@ -626,6 +626,34 @@ def moe_group_pairs(sel: torch.Tensor, weights: torch.Tensor, n_experts: int):
     return counts, token_of_row, scale_of_row
 
 
+def moe_group_pairs_rows(sel: torch.Tensor, weights: torch.Tensor, n_experts: int):
+    """``moe_group_pairs`` and, for every pair ``2 * token + slot``, the row it went to (int32, for ``moe_combine``)."""
+    assert sel.dtype == torch.int32 and sel.dim() == 2 and sel.shape[1] == 2 and sel.is_contiguous()
+    assert weights.dtype == torch.float16 and weights.shape == sel.shape and weights.is_contiguous()
+    pairs = sel.numel()
+    counts = torch.empty((n_experts,), dtype=torch.int32, device=sel.device)
+    token_of_row = torch.empty((pairs,), dtype=torch.int64, device=sel.device)
+    scale_of_row = torch.empty((pairs,), dtype=torch.float16, device=sel.device)
+    row_of_pair = torch.empty((pairs,), dtype=torch.int32, device=sel.device)
+    with _on(sel.device):
+        _lib.check(_lib.lib.hqq_moe_group_pairs_rows(sel.data_ptr(), weights.data_ptr(), pairs // 2, n_experts,
+                                                     counts.data_ptr(), token_of_row.data_ptr(), scale_of_row.data_ptr(),
+                                                     row_of_pair.data_ptr(), _lib.current_stream_ptr(sel.device)),
+                   "hqq_moe_group_pairs_rows")
+    return counts, token_of_row, scale_of_row, row_of_pair
+
+
+def moe_combine(rows: torch.Tensor, row_of_pair: torch.Tensor) -> torch.Tensor:
+    """Every token's two grouped rows added up (reference src/custom_layers.py:312 ``index_add_``s them into zeros)."""
+    assert rows.dtype == torch.float16 and rows.dim() == 2 and rows.is_contiguous() and rows.shape[0] == row_of_pair.numel()
+    assert row_of_pair.dtype == torch.int32 and row_of_pair.is_contiguous() and row_of_pair.numel() % 2 == 0
+    out = torch.empty((row_of_pair.numel() // 2, rows.shape[1]), dtype=torch.float16, device=rows.device)
+    with _on(rows.device):
+        _lib.check(_lib.lib.hqq_moe_combine(rows.data_ptr(), row_of_pair.data_ptr(), out.shape[0], out.shape[1],
+                                            out.data_ptr(), _lib.current_stream_ptr(rows.device)), "hqq_moe_combine")
+    return out
+
+
 def rope_append_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, start: int,
                      cache_k: torch.Tensor, cache_v: torch.Tensor) -> torch.Tensor:
     """Rotary embedding of ``q`` (tokens, heads, hd; in place) and ``k`` (tokens, kv_heads, hd) at positions ``start``

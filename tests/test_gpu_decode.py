@@ -509,3 +509,28 @@ def test_rope_append_rows_equals_the_torch_ops(T, heads, kv, hd, start, L):
     assert out is q and torch.equal(q, q_want) and torch.equal(ck, ck_want) and torch.equal(cv, cv_want)
     with pytest.raises(Exception):  # past the end of the cache
         hip_kernels.rope_append_rows(q, k, v, rot.cos, rot.sin, L - T + 1, ck, cv)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,n_experts,hidden", [(1, 8, 8), (2, 8, 4096), (129, 2, 2056), (700, 16, 4096), (2048, 8, 1000)])
+def test_moe_combine_equals_index_add_into_zeros(tokens, n_experts, hidden):
+    """Grouping with the pairs' rows gives what grouping without gives; adding every token's two rows equals the
+    index_add_ of all rows into zeros (reference src/custom_layers.py:312), bit for bit: two fp16 terms, one order.  A
+    pair without an expert adds nothing, whatever the free row at the end holds."""
+    from mixtral_offloading_amd import hip_kernels
+    gen = torch.Generator().manual_seed(tokens)
+    sel = torch.stack([torch.randperm(n_experts, generator=gen)[:2] for _ in range(tokens)]).int().cuda()
+    w = torch.rand((tokens, 2), generator=gen).half().cuda()
+    rows = torch.randn((2 * tokens, hidden), generator=gen).half().cuda()
+    plain = hip_kernels.moe_group_pairs(sel, w, n_experts)
+    *same, row_of_pair = hip_kernels.moe_group_pairs_rows(sel, w, n_experts)
+    assert all(torch.equal(a, b) for a, b in zip(plain, same))
+    order = torch.argsort(sel.reshape(-1).long(), stable=True)
+    assert torch.equal(row_of_pair[order].long(), torch.arange(2 * tokens, device="cuda"))
+    want = torch.zeros((tokens, hidden), dtype=torch.float16, device="cuda").index_add_(0, same[1], rows)
+    assert torch.equal(hip_kernels.moe_combine(rows, row_of_pair), want)
+    sel[0, 0] = n_experts + 3
+    *_, row_of_pair = hip_kernels.moe_group_pairs_rows(sel, w, n_experts)
+    rows[-1] = float("nan")
+    got = hip_kernels.moe_combine(rows, row_of_pair)
+    assert int(row_of_pair[0]) == -1 and torch.equal(got[0], rows[int(row_of_pair[1])]) and bool(torch.isfinite(got).all())
