@@ -311,6 +311,15 @@ int hqq_gate_up(const hqq_linear *w1, const hqq_linear *w3, const void *x_f16, i
     return launch_silu_mul(a, b, h, M * w1->N, s);
 }
 
+// Whether the gate of 3-bit layers at M rows is one launch of the LDS kernel: where each projection would take that
+// kernel, and where the matmul part of the workspace, sized for the widest family of one projection, holds the partial
+// sums of both (it does at 14336x4096, where it is sized for the 4-bit rewrite of the codes).
+static bool lds_gate_preferred(const hqq_linear *w1, const hqq_linear *w3, int64_t M, size_t mm_bytes)
+{
+    return M <= kSmallBatchMax && pick_family(w1, M) == FAM_LDS && pick_family(w3, M) == FAM_LDS &&
+           ldsgemm_gate_supported(w1, w3, M) && mm_bytes >= ldsgemm_gate_workspace_bytes(w1, w3, M);
+}
+
 // whether the down projection of an expert FFN at M rows is a tile launch whose finishing pass can be left to the caller
 static bool down_finish_deferrable(const hqq_linear *w2, int64_t M)
 {
@@ -370,6 +379,9 @@ static int expert_ffn_impl(const hqq_linear *w1, const hqq_linear *w2, const hqq
     } else if (prefer_tile && tile_gate_supported(w1, w3, M)) {
         // both projections in one launch of the tile kernel, silu(a) * b in its finishing pass
         if ((rc = launch_tile_gate_up(w1, w3, x, M, h, mm, mm_bytes, s)) != HQQ_OK)
+            return rc;
+    } else if (lds_gate_preferred(w1, w3, M, mm_bytes)) {
+        if ((rc = launch_ldsgemm_gate(w1, w3, x, M, h, mm, mm_bytes, s)) != HQQ_OK)
             return rc;
     } else {
         if ((rc = run_matmul(w1, x, M, a, mm, mm_bytes, pick_family(w1, M), s)) != HQQ_OK)

@@ -249,6 +249,10 @@ int launch_tile_gate_up(const hqq_linear *w1, const hqq_linear *w3, const f16 *x
 // MFMA with the de-quantised weights staged in LDS (2-, 3- and 4-bit codes): the kernel of wide batches
 bool ldsgemm_supported(const hqq_linear *l, int64_t M);
 size_t ldsgemm_workspace_bytes(const hqq_linear *l, int64_t M);
+bool ldsgemm_gate_supported(const hqq_linear *w1, const hqq_linear *w3, int64_t M);
+size_t ldsgemm_gate_workspace_bytes(const hqq_linear *w1, const hqq_linear *w3, int64_t M);
+int launch_ldsgemm_gate(const hqq_linear *w1, const hqq_linear *w3, const f16 *x, int64_t M, f16 *h, void *ws, size_t ws_bytes,
+                        hipStream_t s);
 int launch_ldsgemm_matmul(const hqq_linear *l, const f16 *x, int64_t M, f16 *y, void *ws, size_t ws_bytes, hipStream_t s,
                           const SmallBatchEpilogue *ep = nullptr);
 bool vec3_supported(const hqq_linear *l, int64_t M);
@@ -278,8 +282,8 @@ int launch_rope_append_rows(f16 *q, const f16 *k, const f16 *v, const f16 *cos_t
                             int head_dim, hipStream_t s);
 int launch_attention_rows(const f16 *q, const f16 *cache_k, const f16 *cache_v, int64_t start, int64_t tokens, int64_t max_len,
                           int n_heads, int n_kv, int head_dim, f16 *out, hipStream_t s);
-int launch_add_rmsnorm_router(f16 *x, const f16 *delta, const f16 *weight, float eps, f16 *y, int64_t hidden,
 int launch_next_token(const f16 *logits, int64_t n, f16 *out, int64_t *token, int64_t *position, hipStream_t s);
+int launch_add_rmsnorm_router(f16 *x, const f16 *delta, const f16 *weight, float eps, f16 *y, int64_t hidden,
                               const f16 *gate_w, int n_experts, int *sel, f16 *weights, f16 *logits, hipStream_t s);
 int launch_attention_decode(const f16 *q, const f16 *k, const f16 *v, const f16 *cos_t, const f16 *sin_t, const int64_t *pos,
                             f16 *cache_k, f16 *cache_v, int64_t max_len, int n_heads, int n_kv_heads, int head_dim, f16 *out,

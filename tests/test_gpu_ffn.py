@@ -253,3 +253,20 @@ def test_expert_groups_of_decode_size_share_launches(nbits, gs, counts):
         out = torch.full((rows, hidden), 3.0, dtype=torch.float16, device="cuda")
         hip_kernels.expert_groups_ffn(group, x, starts, row_scale, out)
         assert bool(torch.isfinite(each).all()) and torch.equal(out, each)
+
+
+@pytest.mark.parametrize("ffn,hidden,gs,quantised", [(14336, 4096, 64, True), (2560, 4096, 64, True), (1280, 768, 64, False)])
+@pytest.mark.parametrize("m", [9, 13, 16])
+def test_3bit_gate_in_one_launch_equals_the_launches_it_replaces(ffn, hidden, gs, quantised, m):
+    """3-bit experts with 9 to 16 rows: both gate projections in one launch and silu(a) * b in its finishing pass round
+    where two matmuls and the activation kernel do (``gate_up``, then ``matmul``): bit for bit."""
+    from mixtral_offloading_amd import hip_kernels
+    from test_gpu_matmul import _full_size_layer
+    if quantised:
+        d1, d2, d3 = (_full_size_layer(3, n, k, gs, seed=i) for i, (n, k) in enumerate(((ffn, hidden), (hidden, ffn), (ffn, hidden))))
+    else:
+        d1, d2, d3 = (desc_of(l) for l in _ffn_case(np.random.default_rng(m), 3, hidden, ffn, gs, False))
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn((m, hidden), device="cuda", generator=g).half()
+    want = hip_kernels.matmul(d2, hip_kernels.gate_up(d1, d3, x))
+    assert bool(torch.isfinite(want).all()) and torch.equal(hip_kernels.expert_ffn(d1, d2, d3, x), want)
