@@ -278,6 +278,16 @@ int hqq_rope_append_rows(void *q_f16, const void *k_f16, const void *v_f16, cons
 int hqq_attention_rows(const void *q_f16, const void *cache_k_f16, const void *cache_v_f16, int64_t start, int64_t rows,
                        int64_t max_len, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, void *out_f16, void *stream);
 
+/* ---- the same with a workspace (256-byte aligned, no initial contents, at least hqq_attention_rows_workspace_bytes()):
+ *      where few new tokens stand behind many positions, the positions are split over as many blocks as fill the chip,
+ *      and a second launch adds the blocks' shares up in fp32, in the order of the positions.  The results agree with
+ *      hqq_attention_rows' within its rounding, not bit for bit.  The workspace query returns 0 where there is no split
+ *      (then both entry points are the same).                                                                        */
+size_t hqq_attention_rows_workspace_bytes(int64_t start, int64_t rows, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim);
+int hqq_attention_rows_ws(const void *q_f16, const void *cache_k_f16, const void *cache_v_f16, int64_t start, int64_t rows,
+                          int64_t max_len, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, void *out_f16,
+                          void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---- hqq_add_rmsnorm followed by hqq_router_top2 on its output y, in one launch: the post-attention norm of a
  *      decoder layer and the router that reads it (src/custom_layers.py:276-282).  x and y as hqq_add_rmsnorm gives
  *      them; logits as hqq_router_top2 up to the order of the fp32 sums.                                           */

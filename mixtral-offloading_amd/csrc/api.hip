@@ -949,6 +949,24 @@ int hqq_attention_rows(const void *q_f16, const void *cache_k_f16, const void *c
                                  n_heads, n_kv_heads, head_dim, (f16 *)out_f16, (hipStream_t)stream);
 }
 
+size_t hqq_attention_rows_workspace_bytes(int64_t start, int64_t rows, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim)
+{
+    return attention_rows_workspace_bytes(start, rows, n_heads, n_kv_heads, head_dim);
+}
+
+int hqq_attention_rows_ws(const void *q_f16, const void *cache_k_f16, const void *cache_v_f16, int64_t start, int64_t rows,
+                          int64_t max_len, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, void *out_f16,
+                          void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (!q_f16 || !cache_k_f16 || !cache_v_f16 || !out_f16)
+        return HQQ_E_NULL;
+    const size_t need = attention_rows_workspace_bytes(start, rows, n_heads, n_kv_heads, head_dim);
+    if (need > 0 && (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255u)))
+        return HQQ_E_WORKSPACE;
+    return launch_attention_rows((const f16 *)q_f16, (const f16 *)cache_k_f16, (const f16 *)cache_v_f16, start, rows, max_len,
+                                 n_heads, n_kv_heads, head_dim, (f16 *)out_f16, (hipStream_t)stream, need ? workspace : nullptr);
+}
+
 int hqq_add_rmsnorm_router(void *x_f16, const void *delta_f16, const void *weight_f16, float eps, void *y_f16,
                            int64_t hidden, const void *gate_w_f16, int32_t n_experts, int32_t *sel_out,
                            void *weights_f16_out, void *logits_f16_out, void *stream)

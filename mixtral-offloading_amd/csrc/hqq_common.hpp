@@ -281,7 +281,8 @@ int launch_rope_append_rows(f16 *q, const f16 *k, const f16 *v, const f16 *cos_t
                             int64_t rows, f16 *cache_k, f16 *cache_v, int64_t max_len, int n_heads, int n_kv_heads,
                             int head_dim, hipStream_t s);
 int launch_attention_rows(const f16 *q, const f16 *cache_k, const f16 *cache_v, int64_t start, int64_t tokens, int64_t max_len,
-                          int n_heads, int n_kv, int head_dim, f16 *out, hipStream_t s);
+                          int n_heads, int n_kv, int head_dim, f16 *out, hipStream_t s, void *ws = nullptr);
+size_t attention_rows_workspace_bytes(int64_t start, int64_t tokens, int n_heads, int n_kv, int head_dim);
 int launch_next_token(const f16 *logits, int64_t n, f16 *out, int64_t *token, int64_t *position, hipStream_t s);
 int launch_add_rmsnorm_router(f16 *x, const f16 *delta, const f16 *weight, float eps, f16 *y, int64_t hidden,
                               const f16 *gate_w, int n_experts, int *sel, f16 *weights, f16 *logits, hipStream_t s);

@@ -87,6 +87,9 @@ _SIGNATURES = {
                                      c_int64, c_int32, c_int32, c_int32, c_void_p]),
     "hqq_attention_rows": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, c_void_p,
                                    c_void_p]),
+    "hqq_attention_rows_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int32, c_int32, c_int32]),
+    "hqq_attention_rows_ws": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, c_void_p,
+                                      c_void_p, c_size_t, c_void_p]),
     "hqq_add_rmsnorm_router": (c_int, [c_void_p, c_void_p, c_void_p, ctypes.c_float, c_void_p, c_int64, c_void_p, c_int32,
                                        c_void_p, c_void_p, c_void_p, c_void_p]),
     "hqq_attention_decode": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,

@@ -687,9 +687,12 @@ def attention_rows(q: torch.Tensor, cache_k: torch.Tensor, cache_v: torch.Tensor
     out = torch.empty((T, n_heads * hd), dtype=torch.float16, device=q.device)
     if T:
         with _on(q.device):
-            _lib.check(_lib.lib.hqq_attention_rows(q.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), int(start), T, max_len,
-                                                   n_heads, n_kv, hd, out.data_ptr(), _lib.current_stream_ptr(q.device)),
-                       "hqq_attention_rows")
+            # few tokens behind many positions: the positions over several blocks, their shares through a scratch tensor
+            need = int(_lib.lib.hqq_attention_rows_workspace_bytes(int(start), T, n_heads, n_kv, hd))
+            ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
+            _lib.check(_lib.lib.hqq_attention_rows_ws(q.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), int(start), T, max_len,
+                                                      n_heads, n_kv, hd, out.data_ptr(), ws.data_ptr() if need else None, need,
+                                                      _lib.current_stream_ptr(q.device)), "hqq_attention_rows_ws")
     return out
 
 

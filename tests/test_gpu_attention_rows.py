@@ -43,14 +43,67 @@ def test_attention_rows(tokens, start, heads, kv, hd):
     assert ((got - want).abs() <= 2 * bound).all()
 
 
-@pytest.mark.parametrize("tokens,spread", [(2048, 1.0), (2100, 6.0)])
-def test_attention_rows_two_tiles_a_wave(tokens, spread):
+@pytest.mark.parametrize("tokens,spread,hd", [(2048, 1.0, 128), (2100, 6.0, 128), (2050, 1.0, 64)])
+def test_attention_rows_two_tiles_a_wave(tokens, spread, hd):
     """From 512 blocks a wave takes two query tiles (32 heads on 8 key/value heads: 2017 tokens)."""
     from mixtral_offloading_amd import hip_kernels
-    q, ck, cv = _case(tokens, 5, 32, 8, 128, seed=tokens, spread=spread)
+    q, ck, cv = _case(tokens, 5, 32, 8, hd, seed=tokens, spread=spread)
     want, bound = _reference(q, ck, cv, 5)
     got = hip_kernels.attention_rows(q, ck, cv, 5).double().cpu()
     assert ((got - want).abs() <= 2 * bound).all()
+
+
+def _parts(tokens, start, heads, kv, hd):
+    """Parts the positions of a call are split into, from the size of the scratch it asks for."""
+    from mixtral_offloading_amd import _lib
+    return max(1, _lib.lib.hqq_attention_rows_workspace_bytes(start, tokens, heads, kv, hd) // (4 * (hd + 2) * heads * tokens))
+
+
+# few tokens behind many positions, each with more than one part; the last part short or one position long, blocks that
+# see less than the last part (several blocks a head: 40 and 64 tokens), as many parts as there may be
+@pytest.mark.parametrize("tokens,start,heads,kv,hd", [
+    (1, 4000, 32, 8, 128), (1, 16001, 32, 8, 128), (5, 2047, 32, 8, 128), (16, 16368, 32, 8, 128), (40, 4090, 32, 8, 128),
+    (64, 8000, 32, 8, 128), (130, 3967, 32, 8, 128), (1, 2112, 4, 2, 64), (33, 6001, 4, 2, 64), (3, 20000, 3, 1, 128),
+    (2, 66000, 2, 1, 64)])
+def test_attention_rows_behind_a_long_cache(tokens, start, heads, kv, hd):
+    """The parts' fp32 shares are added up in fp32: the bound of the one-pass form.  The same call without a scratch
+    (hqq_attention_rows) walks the positions in one block and gives the same within that bound."""
+    from mixtral_offloading_amd import _lib, hip_kernels
+    assert _parts(tokens, start, heads, kv, hd) > 1
+    q, ck, cv = _case(tokens, start, heads, kv, hd, seed=tokens + start, spread=1.5)
+    want, bound = _reference(q, ck, cv, start)
+    for _ in range(2):
+        got = hip_kernels.attention_rows(q, ck, cv, start).double().cpu()
+        assert ((got - want).abs() <= 2 * bound).all()
+    one = torch.empty((tokens, heads * hd), dtype=torch.float16, device="cuda")
+    _lib.check(_lib.lib.hqq_attention_rows(q.data_ptr(), ck.data_ptr(), cv.data_ptr(), start, tokens, ck.shape[1], heads, kv, hd,
+                                           one.data_ptr(), _lib.current_stream_ptr(q.device)), "hqq_attention_rows")
+    assert ((one.double().cpu() - want).abs() <= 2 * bound).all()
+
+
+@pytest.mark.parametrize("tokens,start", [(70, 100), (20, 5000)])  # one part; several
+def test_attention_rows_infinities_and_nan_in_visible_positions(tokens, start):
+    """What softmax gives in 64 bits: a key that is NaN or scores +inf makes the rows that see it NaN and leaves the
+    others alone, one that scores -inf has no weight; an infinite or NaN value reaches its column of the rows that see it."""
+    from mixtral_offloading_amd import hip_kernels
+    heads, kv, hd = 8, 2, 128
+    assert (_parts(tokens, start, heads, kv, hd) > 1) == (start == 5000)
+    clean = _case(tokens, start, heads, kv, hd, seed=3)
+    at = start + tokens // 2  # the second half of the tokens see it
+    for value in (float("nan"), float("inf"), float("-inf")):
+        q, ck, cv = (t.clone() for t in clean)
+        ck[0, at, 5] = value
+        want, bound = _reference(q, ck, cv, start)
+        got = hip_kernels.attention_rows(q, ck, cv, start).double().cpu()
+        assert torch.equal(got.isnan(), want.isnan()) and bool(want.isnan().any()) and bool((~want.isnan()[tokens // 2:]).any())
+        seen = ~want.isnan()
+        assert ((got - want).abs() <= 2 * bound)[seen].all()
+        q, ck, cv = (t.clone() for t in clean)
+        cv[0, 7, 5] = value  # every row sees it
+        want, _ = _reference(q, ck, cv, start)
+        got = hip_kernels.attention_rows(q, ck, cv, start).double().cpu()
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        assert torch.equal(got[got.isinf()], want[want.isinf()]) and bool((got.isinf() | got.isnan()).any())
 
 
 def test_attention_rows_refuses_what_it_does_not_take():

@@ -105,6 +105,37 @@ def test_kernel_family_by_batch_size_is_host_logic():
     assert lib.hqq_matmul_workspace_bytes(ctypes.byref(up), 640) >= fp16_weights
 
 
+def test_attention_behind_a_long_cache_is_split_until_the_chip_is_full():
+    """A block of the prompt attention takes 64 (token, head of a group) rows and walks their positions in series: where
+    the rows alone make fewer blocks than the 256 compute units, the positions are split (the scratch query tells the
+    parts: heads * tokens rows of head_dim outputs, a maximum and a sum each)."""
+    from mixtral_offloading_amd import _lib
+    query = _lib.lib.hqq_attention_rows_workspace_bytes
+
+    def parts(tokens, start, heads=32, kv=8, hd=128):
+        size = query(start, tokens, heads, kv, hd)
+        assert size % (4 * (hd + 2) * heads * tokens) == 0
+        return size // (4 * (hd + 2) * heads * tokens)
+
+    for tokens in (1, 4, 16, 64):
+        for start in (4000, 16000, 32000):
+            blocks = 8 * -(-4 * tokens // 64)
+            steps = -(-(start + tokens) // 64)
+            assert parts(tokens, start) >= 2 and parts(tokens, start) * blocks <= 512
+            assert parts(tokens, start) * blocks >= 256 or steps / parts(tokens, start) < 6
+    assert parts(1999, 0) == parts(1, 0) == parts(700, 0) == parts(4096, 30000) == 0  # enough rows, or few positions
+    assert parts(1, 100000, heads=1, kv=1, hd=64) <= 256
+    for bad in ((-1, 4, 32, 8, 128), (0, 0, 32, 8, 128), (0, 4, 30, 8, 128), (0, 4, 32, 0, 128), (0, 4, 32, 8, 96)):
+        assert query(*bad) == 0
+    lib, some = _lib.lib, [1 << 20, 2 << 20, 3 << 20]
+    out = 4 << 20
+    assert lib.hqq_attention_rows_ws(*some, 16000, 4, 20000, 32, 8, 128, out, None, 0, None) == -5  # no workspace
+    assert lib.hqq_attention_rows_ws(*some, 16000, 4, 20000, 32, 8, 128, out, 5 << 20, 4096, None) == -5  # too small
+    assert lib.hqq_attention_rows_ws(*some, 16000, 4, 20000, 32, 8, 128, out, (5 << 20) + 16, 1 << 30, None) == -5  # misaligned
+    assert lib.hqq_attention_rows_ws(*some, 16000, 4, 16003, 32, 8, 128, out, 5 << 20, 1 << 30, None) == -3  # past the cache
+    assert lib.hqq_attention_rows_ws(None, *some[1:], 0, 4, 16, 32, 8, 128, out, None, 0, None) == -1
+
+
 def _plan(lib, c, experts):
     n = len(experts)
     arr = (ctypes.c_int32 * n)(*experts)
