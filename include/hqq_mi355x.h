@@ -114,7 +114,9 @@ int hqq_matmul_transpose(const hqq_linear *l, const void *x_f16, int64_t M, void
 /* ---- y = w2( silu(w1 x) * (w3 x) ): replaces MixtralBLockSparseTop2MLP_HQQ.forward, src/custom_layers.py:253-256.
  *      x fp16 (M, hidden), y fp16 (M, hidden).  When `row_scale_f16` is not NULL, row m of the result is multiplied by
  *      row_scale_f16[m] (the routing weight, src/custom_layers.py:308) and when `accumulate` is non-zero the result is
- *      added to y in fp16 instead of stored (the index_add_ at :312 for a single row block).                          */
+ *      added to y in fp16 instead of stored (the index_add_ at :312 for a single row block).
+ *      The workspace query counts the partial sums of a 3-bit gate that runs both projections in one launch (9 to 16
+ *      rows); a workspace that holds everything else is taken too, and the projections then run one by one (same bits). */
 size_t hqq_expert_ffn_workspace_bytes(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, int64_t M);
 int hqq_expert_ffn(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, const void *x_f16, int64_t M,
                    void *y_f16, const void *row_scale_f16, int accumulate, void *workspace, size_t workspace_bytes,
@@ -139,7 +141,7 @@ int hqq_expert_groups_ffn(const hqq_linear *const *w1, const hqq_linear *const *
  *      serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The workspace is an
  *      array of HQQ_STATIC_SCRATCH_BYTES built into the library's device code (every GPU the library runs on holds it
  *      until the process ends); the call allocates nothing and returns HQQ_E_WORKSPACE when
- *      hqq_expert_ffn_workspace_bytes(w1, w2, w3, M) exceeds that size (Mixtral-8x7B experts: batches up to 4 rows at
+ *      the least workspace hqq_expert_ffn takes for w1, w2, w3 and M exceeds that size (Mixtral-8x7B experts: batches up to 4 rows at
  *      any code width, up to 16 rows for 2-bit codes).  Results are hqq_expert_ffn's, bit for bit.  All calls on one
  *      GPU share the array: calls that overlap in time on one GPU race (order them on one stream, or with events).
  *      The first call on a GPU records one extra small fill kernel on `stream`.                                    */

@@ -237,11 +237,39 @@ static size_t ffn_matmul_scratch(const hqq_linear *w1, const hqq_linear *w2, con
     return align256(mm);
 }
 
+// Whether the gate of 3-bit layers at M rows is one launch of the LDS kernel: where each projection would take that kernel
+static bool lds_gate_preferred(const hqq_linear *w1, const hqq_linear *w3, int64_t M)
+{
+    return w1->nbits == 3 && M <= kSmallBatchMax && pick_family(w1, M) == FAM_LDS && pick_family(w3, M) == FAM_LDS &&
+           ldsgemm_gate_supported(w1, w3, M);
+}
+
+// The matmul part with the partial sums of both gate projections.  What one projection's widest family needs holds them at
+// 14336x4096 (it is sized for the 4-bit rewrite of the codes), but not where the tile kernel does not take the shape: the
+// query counts them, and a call with a workspace that lacks them runs the projections one after the other.
+static size_t ffn_gate_scratch(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, int64_t M)
+{
+    const size_t mm = ffn_matmul_scratch(w1, w2, w3, M);
+    const size_t g = lds_gate_preferred(w1, w3, M) ? align256(ldsgemm_gate_workspace_bytes(w1, w3, M)) : 0;
+    return g > mm ? g : mm;
+}
+
+static size_t ffn_rows_bytes(const hqq_linear *w1, const hqq_linear *w2, int64_t M)
+{
+    return 3 * align256((size_t)M * w1->N * 2) + align256((size_t)M * w2->N * 2);
+}
+
+// the least a call is taken with
+static size_t ffn_least_bytes(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, int64_t M)
+{
+    return ffn_matmul_scratch(w1, w2, w3, M) + ffn_rows_bytes(w1, w2, M);
+}
+
 size_t hqq_expert_ffn_workspace_bytes(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, int64_t M)
 {
     if (validate_linear(w1) != HQQ_OK || validate_linear(w2) != HQQ_OK || validate_linear(w3) != HQQ_OK || M <= 0)
         return 0;
-    return ffn_matmul_scratch(w1, w2, w3, M) + 3 * align256((size_t)M * w1->N * 2) + align256((size_t)M * w2->N * 2);
+    return ffn_gate_scratch(w1, w2, w3, M) + ffn_rows_bytes(w1, w2, M);
 }
 
 // workspace of the gate: [matmul scratch, counters first][a, b: M x N fp16 each (unfused paths only)]
@@ -311,15 +339,6 @@ int hqq_gate_up(const hqq_linear *w1, const hqq_linear *w3, const void *x_f16, i
     return launch_silu_mul(a, b, h, M * w1->N, s);
 }
 
-// Whether the gate of 3-bit layers at M rows is one launch of the LDS kernel: where each projection would take that
-// kernel, and where the matmul part of the workspace, sized for the widest family of one projection, holds the partial
-// sums of both (it does at 14336x4096, where it is sized for the 4-bit rewrite of the codes).
-static bool lds_gate_preferred(const hqq_linear *w1, const hqq_linear *w3, int64_t M, size_t mm_bytes)
-{
-    return M <= kSmallBatchMax && pick_family(w1, M) == FAM_LDS && pick_family(w3, M) == FAM_LDS &&
-           ldsgemm_gate_supported(w1, w3, M) && mm_bytes >= ldsgemm_gate_workspace_bytes(w1, w3, M);
-}
-
 // whether the down projection of an expert FFN at M rows is a tile launch whose finishing pass can be left to the caller
 static bool down_finish_deferrable(const hqq_linear *w2, int64_t M)
 {
@@ -341,13 +360,19 @@ static int expert_ffn_impl(const hqq_linear *w1, const hqq_linear *w2, const hqq
         return HQQ_OK;
     if (!x_f16 || !y_f16)
         return HQQ_E_NULL;
-    const size_t need = hqq_expert_ffn_workspace_bytes(w1, w2, w3, M);
-    if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255u))
+    const size_t rows_bytes = ffn_rows_bytes(w1, w2, M);
+    size_t mm_bytes = ffn_matmul_scratch(w1, w2, w3, M);
+    if (!workspace || workspace_bytes < mm_bytes + rows_bytes || (reinterpret_cast<uintptr_t>(workspace) & 255u))
         return HQQ_E_WORKSPACE;
+    bool lds_gate = lds_gate_preferred(w1, w3, M);
+    if (lds_gate) {
+        const size_t g = ffn_gate_scratch(w1, w2, w3, M);
+        lds_gate = workspace_bytes >= g + rows_bytes;
+        mm_bytes = lds_gate ? g : mm_bytes;
+    }
     hipStream_t s = (hipStream_t)stream;
     char *p = static_cast<char *>(workspace);
     const size_t mid = align256((size_t)M * w1->N * 2), outb = align256((size_t)M * w2->N * 2);
-    const size_t mm_bytes = ffn_matmul_scratch(w1, w2, w3, M);
     void *mm = p; // first, so that hqq_workspace_init finds the counters at the head of the workspace
     f16 *h = (f16 *)(p + mm_bytes);
     f16 *t = (f16 *)(p + mm_bytes + mid);
@@ -380,7 +405,7 @@ static int expert_ffn_impl(const hqq_linear *w1, const hqq_linear *w2, const hqq
         // both projections in one launch of the tile kernel, silu(a) * b in its finishing pass
         if ((rc = launch_tile_gate_up(w1, w3, x, M, h, mm, mm_bytes, s)) != HQQ_OK)
             return rc;
-    } else if (lds_gate_preferred(w1, w3, M, mm_bytes)) {
+    } else if (lds_gate) {
         if ((rc = launch_ldsgemm_gate(w1, w3, x, M, h, mm, mm_bytes, s)) != HQQ_OK)
             return rc;
     } else {
@@ -617,7 +642,7 @@ int hqq_expert_ffn_static(const hqq_linear *w1, const hqq_linear *w2, const hqq_
         return HQQ_E_SHAPE;
     if (M == 0)
         return HQQ_OK;
-    if (hqq_expert_ffn_workspace_bytes(w1, w2, w3, M) > kStaticScratchBytes)
+    if (ffn_least_bytes(w1, w2, w3, M) > kStaticScratchBytes)
         return HQQ_E_WORKSPACE; // beyond the built-in scratch: use hqq_expert_ffn with a workspace of the caller's
     void *ws = nullptr;
     if ((rc = static_scratch(&ws)) != HQQ_OK)
@@ -657,7 +682,7 @@ int hqq_expert_ffn_indexed(const hqq_linear *w1, const hqq_linear *w2, const hqq
     const bool three = w1->nbits == 3 && vec3_ffn_supported(w1, w2, w3, M, 1);
     if (!three && (!strip_supported(w1, M) || !strip_supported(w3, M) || !strip_supported(w2, M)))
         return HQQ_E_UNSUPPORTED;
-    const size_t need = hqq_expert_ffn_workspace_bytes(w1, w2, w3, M);
+    const size_t need = ffn_least_bytes(w1, w2, w3, M);
     if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255u))
         return HQQ_E_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;

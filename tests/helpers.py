@@ -45,3 +45,22 @@ def assert_matmul_close(y_gpu: np.ndarray, y_ref: np.ndarray, atol: np.ndarray, 
     assert not bad.any(), (f"{int(bad.sum())} of {bad.size} outputs out of tolerance; worst err {err.max():.4g}, "
                            f"worst err/bound {(err / bound).max():.3g}")
     return float((err / bound).max())
+
+
+def launches(call):
+    """How many nodes a HIP graph recorded from ``call()`` has: which route a call takes, where the routes' results are the
+    same.  Recorded only, never replayed; a first call on the recording stream makes the stream's workspace."""
+    import ctypes
+    import re
+    hip = ctypes.CDLL(re.search(r"\S*libamdhip64\.so\S*", open("/proc/self/maps").read()).group(0))
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=stream):
+        call()
+    count = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    return count.value

@@ -1,10 +1,12 @@
 """GPU parity tests of the expert FFN entry point (reference src/custom_layers.py:253-256, :308-312) against the
 numpy oracle at small sizes, and against de-quantise-then-matmul on the GPU at Mixtral size."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from helpers import assert_matmul_close, desc_of, to_dev
+from helpers import assert_matmul_close, desc_of, launches, to_dev
 from oracle import hqq_oracle as o
 
 pytestmark = pytest.mark.gpu
@@ -270,3 +272,31 @@ def test_3bit_gate_in_one_launch_equals_the_launches_it_replaces(ffn, hidden, gs
     x = torch.randn((m, hidden), device="cuda", generator=g).half()
     want = hip_kernels.matmul(d2, hip_kernels.gate_up(d1, d3, x))
     assert bool(torch.isfinite(want).all()) and torch.equal(hip_kernels.expert_ffn(d1, d2, d3, x), want)
+
+
+# short: what one projection's widest family needs does not hold the partial sums of both
+@pytest.mark.parametrize("ffn,hidden,gs,m,short", [(14336, 4096, 64, 9, False), (2560, 4096, 64, 16, False), (1280, 768, 64, 16, False),
+                                                   (5760, 768, 64, 16, True), (4992, 256, 64, 12, True), (2304, 512, 128, 12, True)])
+def test_3bit_gate_in_one_launch_wherever_the_kernel_takes_it(ffn, hidden, gs, m, short):
+    """The route itself, by launches: the joint gate and its finishing pass, then the down projection as it is alone, against
+    the gate's two matmuls and the activation kernel; the same bits by either.  A workspace without room for the joint
+    gate's sums is still taken, and a smaller one refused."""
+    from mixtral_offloading_amd import _lib, hip_kernels
+    from test_gpu_matmul import _full_size_layer
+    d1, d2, d3 = (_full_size_layer(3, n, k, gs, seed=i) for i, (n, k) in enumerate(((ffn, hidden), (hidden, ffn), (ffn, hidden))))
+    x = torch.randn((m, hidden), device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).half()
+    h = hip_kernels.gate_up(d1, d3, x)
+    want = hip_kernels.matmul(d2, h)
+    assert bool(torch.isfinite(want).all()) and torch.equal(hip_kernels.expert_ffn(d1, d2, d3, x), want)
+    down = launches(lambda: hip_kernels.matmul(d2, h))
+    assert launches(lambda: hip_kernels.expert_ffn(d1, d2, d3, x)) == 2 + down
+    assert launches(lambda: hip_kernels.gate_up(d1, d3, x)) >= 3
+    if short:
+        up256 = lambda v: (v + 255) // 256 * 256  # noqa: E731
+        least = max(_lib.lib.hqq_matmul_workspace_bytes(d.ref, m) for d in (d1, d2)) + 3 * up256(2 * m * ffn) + up256(2 * m * hidden)
+        assert least < _lib.lib.hqq_expert_ffn_workspace_bytes(d1.ref, d2.ref, d3.ref, m)
+        ws, out = torch.zeros(least, dtype=torch.uint8, device="cuda"), torch.zeros((m, hidden), dtype=torch.float16, device="cuda")
+        call = lambda size: _lib.lib.hqq_expert_ffn(d1.ref, d2.ref, d3.ref, x.data_ptr(), m, out.data_ptr(), None, 0, ws.data_ptr(),  # noqa: E731
+                                                    size, _lib.current_stream_ptr(x.device))
+        assert call(least - 256) == -5 and call(least) == 0 and torch.equal(out, want)
+        assert launches(lambda: call(least)) > 2 + down

@@ -105,6 +105,30 @@ def test_kernel_family_by_batch_size_is_host_logic():
     assert lib.hqq_matmul_workspace_bytes(ctypes.byref(up), 640) >= fp16_weights
 
 
+def test_ffn_scratch_holds_the_sums_of_a_joint_3bit_gate():
+    """9 to 16 rows of 3-bit experts run both gate projections in one launch, which leaves the partial sums of both (per K
+    block and row, 4 bytes an output).  The query counts them, also where one projection alone needs less."""
+    from mixtral_offloading_amd import _lib
+    lib = _lib.lib
+
+    def layer(n, k, gs):
+        lin = _lib.HqqLinear()
+        lin.nbits, lin.group_size, lin.N, lin.K, lin.codes = 3, gs, n, k, 1 << 30
+        for t, at in ((lin.scale, 2 << 30), (lin.zero, 3 << 30)):
+            t.data, t.kind = at, _lib.HQQ_TABLE_U8
+            t.meta_scale, t.meta_zero = at + (1 << 28), at + (1 << 29)
+        lin.scale.meta_cols, lin.zero.meta_cols = n // gs * k // 128, 1
+        return lin
+
+    head, up256 = 576 * 1024, lambda v: (v + 255) // 256 * 256  # noqa: E731
+    for n, k, gs, m, blocks in ((14336, 4096, 64, 16, 4), (5760, 768, 64, 16, 1), (4992, 256, 64, 12, 1), (2304, 512, 128, 12, 1)):
+        up, down = layer(n, k, gs), layer(k, n, gs)
+        assert lib.hqq_matmul_kernel_family(ctypes.byref(up), m) == _lib.FAM_LDS
+        sums = up256(head + 2 * blocks * m * n * 4)
+        have = lib.hqq_expert_ffn_workspace_bytes(ctypes.byref(up), ctypes.byref(down), ctypes.byref(up), m)
+        assert have >= sums + 3 * up256(2 * m * n) + up256(2 * m * k)
+
+
 def test_attention_behind_a_long_cache_is_split_until_the_chip_is_full():
     """A block of the prompt attention takes 64 (token, head of a group) rows and walks their positions in series: where
     the rows alone make fewer blocks than the 256 compute units, the positions are split (the scratch query tells the
