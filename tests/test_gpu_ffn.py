@@ -228,15 +228,15 @@ def test_expert_groups_at_full_size_leave_the_finishing_passes_to_the_end():
         assert bool(torch.isfinite(one).all())
 
 
-@pytest.mark.parametrize("nbits,gs", [(2, 16), (4, 64)])
+@pytest.mark.parametrize("nbits,gs,ffn", [(2, 16, 14336), (4, 64, 7168)])
 @pytest.mark.parametrize("counts", [[3, 4, 3], [5, 3, 8, 4, 0, 7, 2, 1], [9, 16, 17, 4], [4] * 6 + [8] * 3])
-def test_expert_groups_of_decode_size_share_launches(nbits, gs, counts):
+def test_expert_groups_of_decode_size_share_launches(nbits, gs, ffn, counts):
     """Experts with 3 to 16 rows share the batch kernel's launches, by class of rows (up to four, eight, sixteen) and as
     many as the accumulation slots of a K split hold (four experts of four rows, two of eight, at 4096 outputs).  Each
     block sums what it sums alone: bit for bit one call per expert, again on the second call (slots left at zero)."""
     from mixtral_offloading_amd import hip_kernels
     from test_gpu_matmul import _full_size_layer
-    hidden, ffn = 4096, 7168  # the down projection splits K over blocks, the gate holds all of it
+    hidden = 4096  # the down projection splits K over blocks, the gate (224 tiles) holds all of it
     shapes = ((ffn, hidden), (hidden, ffn), (ffn, hidden))
     descs = [tuple(_full_size_layer(nbits, n, k, gs, seed=3 * e + i) for i, (n, k) in enumerate(shapes)) for e in range(len(counts))]
     group = hip_kernels.ExpertGroup(descs)
@@ -255,6 +255,42 @@ def test_expert_groups_of_decode_size_share_launches(nbits, gs, counts):
         out = torch.full((rows, hidden), 3.0, dtype=torch.float16, device="cuda")
         hip_kernels.expert_groups_ffn(group, x, starts, row_scale, out)
         assert bool(torch.isfinite(each).all()) and torch.equal(out, each)
+
+
+@pytest.mark.parametrize("nbits,gs,ffn", [(2, 16, 14336), (4, 64, 7168)])
+@pytest.mark.parametrize("counts", [[3, 4, 3], [5, 3, 8, 4, 0, 7, 2, 1], [9, 16, 17, 4], [4] * 6 + [8] * 3])
+def test_expert_groups_of_decode_size_take_as_few_launches_as_their_slots_allow(nbits, gs, ffn, counts):
+    """The route itself, by launches: a class with two members or more runs its gates in one launch and its down
+    projections in as many as the slots hold members of it; every other expert as it runs alone.  A workspace of the
+    largest expert's need is still taken, with one call per expert (same bits), and a smaller one refused."""
+    from mixtral_offloading_amd import _lib, hip_kernels
+    from test_gpu_matmul import _full_size_layer
+    hidden = 4096
+    shapes = ((ffn, hidden), (hidden, ffn), (ffn, hidden))
+    one = tuple(_full_size_layer(nbits, n, k, gs, seed=i) for i, (n, k) in enumerate(shapes))
+    group = hip_kernels.ExpertGroup([one] * len(counts))
+    starts = np.concatenate(([0], np.cumsum(counts)))
+    rows = int(starts[-1])
+    x = torch.randn((rows, hidden), device="cuda", generator=torch.Generator(device="cuda").manual_seed(rows)).half()
+    out = torch.full((rows, hidden), 3.0, dtype=torch.float16, device="cuda")
+    members = {4: [], 8: [], 16: []}  # rows of a class -> its experts
+    for m in counts:
+        if 3 <= m <= 16:
+            members[4 if m <= 4 else 8 if m <= 8 else 16].append(m)
+    shared = {m: n for m, n in members.items() if len(n) >= 2}
+    alone = sum(launches(lambda: hip_kernels.expert_ffn(*one, x[:m])) for m in counts if m and not any(m in n for n in shared.values()))
+    every = sum(launches(lambda: hip_kernels.expert_ffn(*one, x[:m])) for m in counts if m)
+    together = sum(1 + -(-len(n) // (16 // m)) for m, n in shared.items())
+    assert launches(lambda: hip_kernels.expert_groups_ffn(group, x, starts, None, out)) == together + alone < every
+    hip_kernels.expert_groups_ffn(group, x, starts, None, out)
+    held = (ctypes.c_int64 * len(starts))(*[int(v) for v in starts])
+    least = max(_lib.lib.hqq_expert_ffn_workspace_bytes(*(d.ref for d in one), m) for m in counts if m)
+    assert least < _lib.lib.hqq_expert_groups_ffn_workspace_bytes(group.w1, group.w2, group.w3, group.n, held)
+    ws, got = torch.zeros(least, dtype=torch.uint8, device="cuda"), torch.full_like(out, 5.0)
+    call = lambda size: _lib.lib.hqq_expert_groups_ffn(group.w1, group.w2, group.w3, group.n, held, x.data_ptr(), got.data_ptr(),  # noqa: E731
+                                                       None, ws.data_ptr(), size, _lib.current_stream_ptr(x.device))
+    assert call(least - 256) == -5 and call(least) == 0 and bool(torch.isfinite(out).all()) and torch.equal(got, out)
+    assert launches(lambda: call(least)) == every
 
 
 @pytest.mark.parametrize("ffn,hidden,gs,quantised", [(14336, 4096, 64, True), (2560, 4096, 64, True), (1280, 768, 64, False)])
