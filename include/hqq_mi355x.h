@@ -128,9 +128,10 @@ int hqq_expert_ffn(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear 
  *      y[row] = row_scale_f16[row] * expert(x[row]) (row_scale_f16 may be NULL).  row_start is a HOST array of
  *      n_groups + 1 entries starting at 0; groups without rows may have NULL layers.  One call issues every group's
  *      launches in order on `stream` with one workspace of hqq_expert_groups_ffn_workspace_bytes(..) bytes (the
- *      largest group's need, then the partial sums of the down projections that split K: their finishing passes run
- *      as one launch at the end of the call; head zeroed as for hqq_matmul_transpose).  Results are
- *      hqq_expert_ffn's, bit for bit.                                                                              */
+ *      largest group's need, then the partial sums of the down projections that split K, whose finishing passes run
+ *      as one launch at the end of the call, and silu(a) * b of the groups of 3 to 16 rows, which share launches;
+ *      head zeroed as for hqq_matmul_transpose).  A workspace of the largest group's need alone is taken too, with
+ *      the groups one by one.  Results are hqq_expert_ffn's, bit for bit.                                          */
 size_t hqq_expert_groups_ffn_workspace_bytes(const hqq_linear *const *w1, const hqq_linear *const *w2,
                                              const hqq_linear *const *w3, int32_t n_groups, const int64_t *row_start);
 int hqq_expert_groups_ffn(const hqq_linear *const *w1, const hqq_linear *const *w2, const hqq_linear *const *w3,
@@ -140,11 +141,10 @@ int hqq_expert_groups_ffn(const hqq_linear *const *w1, const hqq_linear *const *
 /* ---- hqq_expert_ffn for callers that cannot allocate or carry a workspace (code under HIP graph capture, tight
  *      serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The workspace is an
  *      array of HQQ_STATIC_SCRATCH_BYTES built into the library's device code (every GPU the library runs on holds it
- *      until the process ends); the call allocates nothing and returns HQQ_E_WORKSPACE when
- *      the least workspace hqq_expert_ffn takes for w1, w2, w3 and M exceeds that size (Mixtral-8x7B experts: batches up to 4 rows at
- *      any code width, up to 16 rows for 2-bit codes).  Results are hqq_expert_ffn's, bit for bit.  All calls on one
- *      GPU share the array: calls that overlap in time on one GPU race (order them on one stream, or with events).
- *      The first call on a GPU records one extra small fill kernel on `stream`.                                    */
+ *      until the process ends); the call allocates nothing and returns HQQ_E_WORKSPACE when the least workspace
+ *      hqq_expert_ffn takes for w1, w2, w3 and M exceeds that size (Mixtral-8x7B experts: batches up to 4 rows at any
+ *      code width, up to 16 rows for 2-bit codes).  Results are hqq_expert_ffn's, bit for bit.  All calls on one GPU
+ *      share the array: calls that overlap in time on one GPU race (order them on one stream, or with events).     */
 #define HQQ_STATIC_SCRATCH_BYTES ((size_t)16 << 20)
 int hqq_expert_ffn_static(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, const void *x_f16, int64_t M,
                           void *y_f16, const void *row_scale_f16, int accumulate, void *stream);

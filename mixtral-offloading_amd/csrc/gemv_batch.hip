@@ -435,7 +435,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_batch_kernel(BatchParams p)
     gemv_batch_block<NBITS, PH, MS, SKIND, ZKIND, EPI, WAVES, true>(p, p.layer[0], p.layer[1], blockIdx.z);
 }
 
-// One launch over the experts of a MoE layer that have up to four (PH 4) or five to eight (PH 2) rows.
+// One launch over the experts of a MoE layer that have three or four rows (PH 4), five to eight (PH 2) or nine to sixteen
+// (PH 2, MS 2).
 // A launch per expert has a block for at most 224 of the 256 compute units and pays its start and its tail each time;
 // together the experts fill the chip and the next expert's blocks start while the last one's finish.
 // 14336x4096 2-bit in groups of 16, cache-cold: the gates of four experts of 3 and 4 rows 60.3 -> 54.6 us, their down
