@@ -293,6 +293,34 @@ def test_expert_groups_of_decode_size_take_as_few_launches_as_their_slots_allow(
     assert launches(lambda: call(least)) == every
 
 
+def test_expert_groups_share_launches_only_with_experts_alike():
+    """Seventy groups (shared launches are made up among the first 64) whose experts differ in code width, group size,
+    FFN width, table kind and the bias of the down projection: bit for bit one call per expert."""
+    from mixtral_offloading_amd import hip_kernels
+    rng = np.random.default_rng(70)
+    hidden = 512
+    kinds = [(2, 4096, 16, True, False), (2, 4096, 16, False, False), (2, 4096, 32, True, False), (4, 4096, 64, True, False),
+             (2, 4096, 16, True, True), (2, 2048, 16, True, False)]
+    descs = []
+    for nbits, ffn, gs, tables, bias in kinds:
+        w1, w2, w3 = _ffn_case(rng, nbits, hidden, ffn, gs, tables)
+        descs.append((desc_of(w1), desc_of(w2, bias=rng.standard_normal(hidden).astype(np.float16) if bias else None), desc_of(w3)))
+    counts = [int(v) for v in rng.choice([3, 4, 5, 8, 9, 16, 1, 0, 20], size=70)]
+    experts = [descs[int(v)] for v in rng.choice(len(kinds), size=70)]
+    starts = np.concatenate(([0], np.cumsum(counts)))
+    rows = int(starts[-1])
+    x, scale = to_dev(rng.standard_normal((rows, hidden)).astype(np.float16)), to_dev(rng.uniform(0.2, 0.8, rows).astype(np.float16))
+    group = hip_kernels.ExpertGroup(experts)
+    out, each = (torch.full((rows, hidden), v, dtype=torch.float16, device="cuda") for v in (3.0, 5.0))
+    for _ in range(2):
+        hip_kernels.expert_groups_ffn(group, x, starts, scale, out)
+        for e, m in enumerate(counts):
+            lo = int(starts[e])
+            if m:
+                hip_kernels.expert_ffn(*experts[e], x[lo:lo + m], out=each[lo:lo + m], row_scale=scale[lo:lo + m])
+        assert bool(torch.isfinite(each).all()) and torch.equal(out, each)
+
+
 @pytest.mark.parametrize("ffn,hidden,gs,quantised", [(14336, 4096, 64, True), (2560, 4096, 64, True), (1280, 768, 64, False)])
 @pytest.mark.parametrize("m", [9, 13, 16])
 def test_3bit_gate_in_one_launch_equals_the_launches_it_replaces(ffn, hidden, gs, quantised, m):
