@@ -17,11 +17,11 @@
 // host loop would have stopped, and returns if so; the last pass repeats the iterations of the one pass the stop fell
 // into and writes the result.  All arithmetic is fp32 with separate multiplies and adds, as the tensor ops it replaces.
 //
-// Bound by the vector units: an iteration is sixteen or so operations a value.  It was over a hundred: the shrinkage's
-// power took most of them and a full division the next, and all iterations ran before the stop was looked for.  The
-// power is evaluated only where its term can be other than zero (shrink_skip), the division is a reciprocal corrected
-// to the same rounding (divide_by).  14336 x 4096, 2-bit in groups of 16, stopped within the third of five passes: all
-// passes together 2185 -> 520 us, with the same bits; about 30 us an iteration.
+// An iteration is a dozen operations a value.  It was over a hundred: the shrinkage's power took most of them and a full
+// division the next, and all iterations ran before the stop was looked for.  The power is evaluated only where its term
+// can be other than zero (shrink_skip), the division is a product by the reciprocal in two floats (divide_by; sixteen
+// operations a value with a correction by the residual, 614 -> 576 us).  A 14336 x 4096 layer to 2 bits in groups of 16,
+// stopped within the third of five passes: 2238 -> 576 us, with the same bits.
 #include "hqq_common.hpp"
 
 #include <cmath>
@@ -77,35 +77,34 @@ __device__ __forceinline__ float shrink_lp(float x, float inv_beta, float pm1)
     return x > 0.f ? r : (x < 0.f ? -r : 0.f);
 }
 
-// x / s correctly rounded, from inv = 1 / s correctly rounded: the first two steps bring the quotient to within an ulp,
-// and one more correction by the exact residual rounds it as a division does (Markstein 1990), five operations for about
-// twice as many slots.  For |s| and |x| where neither residual nor quotient leaves the normal range: see divide_safe.
-__device__ __forceinline__ float divide_by(float x, float s, float inv)
-{
-    float q = x * inv;
-    q = __builtin_fmaf(__builtin_fmaf(-s, q, x), inv, q);
-    return __builtin_fmaf(__builtin_fmaf(-s, q, x), inv, q);
-}
+// x / s from 1 / s as the sum hi + lo of two floats.  The sum is within 2^-46 of 1 / s, so before its one rounding the
+// quotient is within 2^-45 of its size: it is rounded as a division rounds it unless it lies that near the middle
+// between two floats (one quotient in some millions, and then the other of the two neighbours).  Two operations, where
+// correcting x * hi by the exact residual takes five.  Only the errors that decide the stop are made with it; neither
+// zero points nor codes are.  For |s| and |x| where nothing leaves the normal range: see divide_safe.
+__device__ __forceinline__ float divide_by(float x, float hi, float lo) { return __builtin_fmaf(x, hi, x * lo); }
 // x = q - zero with q whole: zero itself, or not below the distance of neighbouring floats around a whole number
+// (2^-24, or 2^-40 where zero is that small); hi above 2^-40 and lo, if not 0, above 2^-48 of it leave x * lo above
+// 2^-128, 2^-48 of the quotient, where a denormal result still has all the bits that count
 __device__ __forceinline__ bool divide_safe(float scale, float zero)
 {
     const float a = __builtin_fabsf(zero);
-    return scale > 0x1p-60f && scale < 0x1p60f && (a == 0.f || (a > 0x1p-60f && a < 0x1p60f));
+    return scale > 0x1p-40f && scale < 0x1p40f && (a == 0.f || (a > 0x1p-40f && a < 0x1p40f));
 }
 
 // One iteration of the solver on a column: its zero point moves, its error is returned.  The plain sums are made again
 // with divisions and the shrinkage in them where a lane of the wave may need either.
 template <int GS, int CP>
-__device__ __forceinline__ float solver_step(const QuantParams &p, const float (&w)[GS][CP], int j, float scale, float inv,
-                                             float inv_beta, float &zero)
+__device__ __forceinline__ float solver_step(const QuantParams &p, const float (&w)[GS][CP], int j, float scale, float hi,
+                                             float lo, float inv_beta, float &zero)
 {
     float e = 0.f, acc = 0.f, top = 0.f;
 #pragma unroll
     for (int r = 0; r < GS; ++r) {
         const float ws = w[r][j] * scale;
-        float q = __builtin_rintf(ws + zero);
-        q = __builtin_fminf(__builtin_fmaxf(q, 0.f), p.max_v);
-        const float a = __builtin_fabsf(w[r][j] - divide_by(q - zero, scale, inv));
+        // the middle of the three is the clamped value in one operation (0 for a NaN, as of the two)
+        const float q = __builtin_amdgcn_fmed3f(__builtin_rintf(ws + zero), 0.f, p.max_v);
+        const float a = __builtin_fabsf(w[r][j] - divide_by(q - zero, hi, lo));
         e += a;
         top = __builtin_fmaxf(top, a);
         acc += q - ws;
@@ -204,10 +203,12 @@ template <int GS, int CP, int PASS> __global__ __launch_bounds__(kQThreads) void
         double beta = p.beta; // the host loop keeps beta as a double and hands 1 / beta to fp32 tensor ops
         for (int it = 0; it < first; ++it)
             beta *= p.kappa;
-        float inv[CP];
+        float hi[CP], lo[CP]; // 1 / scale
 #pragma unroll
-        for (int j = 0; j < CP; ++j)
-            inv[j] = 1.0f / scale[j];
+        for (int j = 0; j < CP; ++j) {
+            hi[j] = 1.0f / scale[j];
+            lo[j] = __builtin_fmaf(-scale[j], hi[j], 1.0f) * hi[j];
+        }
 #pragma unroll 1
         for (int it = first; it < last; ++it) {
             const float inv_beta = (float)(1.0 / beta);
@@ -216,7 +217,7 @@ template <int GS, int CP, int PASS> __global__ __launch_bounds__(kQThreads) void
             for (int j = 0; j < CP; ++j) {
                 float sc = scale[j];
                 asm volatile("" : "+v"(sc)); // keeps w * scale out of registers of its own across iterations
-                e += solver_step<GS, CP>(p, w, j, sc, inv[j], inv_beta, zero[j]);
+                e += solver_step<GS, CP>(p, w, j, sc, hi[j], lo[j], inv_beta, zero[j]);
             }
             beta *= p.kappa;
             if constexpr (PASS == 1) {
