@@ -11,8 +11,8 @@
 // One thread owns CP neighbouring groups (4, 2 or 1, by what the registers hold) and keeps their values in registers,
 // so every iteration of the solver is register arithmetic; consecutive threads read consecutive pieces of a row, so
 // every row is a coalesced streaming read of 4 to 16 bytes per thread.  The solver
-// stops for the WHOLE tensor at once: passes of kQChunk iterations add up the error of every iteration (fp64 atomics)
-// and leave the zero points they reached in one of the two output vectors (the next pass reads it and writes the
+// stops for the WHOLE tensor at once: passes of kQChunk iterations add up the error of every iteration (fp64 atomics,
+// on several sums side by side) and leave the zero points they reached in one of the two output vectors (the next pass reads it and writes the
 // other, so both ends of a pass are at hand); every block of a later pass finds from the errors so far whether the
 // host loop would have stopped, and returns if so; the last pass repeats the iterations of the one pass the stop fell
 // into and writes the result.  All arithmetic is fp32 with separate multiplies and adds, as the tensor ops it replaces.
@@ -20,8 +20,9 @@
 // An iteration is a dozen operations a value.  It was over a hundred: the shrinkage's power took most of them and a full
 // division the next, and all iterations ran before the stop was looked for.  The power is evaluated only where its term
 // can be other than zero (shrink_skip), the division is a product by the reciprocal in two floats (divide_by; sixteen
-// operations a value with a correction by the residual, 614 -> 576 us).  A 14336 x 4096 layer to 2 bits in groups of 16,
-// stopped within the third of five passes: 2238 -> 576 us, with the same bits.
+// operations a value with a correction by the residual, 614 -> 576 us), and the blocks' error sums do not queue for one
+// line of memory (kQSums; 576 -> 510 us).  Times are of a 14336 x 4096 layer taken to 2 bits in groups of 16, stopped
+// within the third of five passes; it began at 2238 us, with the same bits.
 #include "hqq_common.hpp"
 
 #include <cmath>
@@ -32,6 +33,9 @@ namespace {
 constexpr int kQThreads = 256;
 constexpr int kQMaxIters = 64;
 constexpr int kQChunk = 4; // iterations between two looks at the stop: a pass more costs one read of the tensor
+// Sums of an iteration's error, blocks taking them in turn: atomics on one line follow each other at some 10 ns, so that
+// on a single sum the four of each of 3584 blocks (58.7 M values) take longer than the pass's arithmetic.
+constexpr int kQSums = 32;
 
 struct QuantParams {
     const void *w;
@@ -41,13 +45,14 @@ struct QuantParams {
     int round_zero;
     int iters;
     float lp;
-    double beta, kappa; // doubles, as in the host loop they restate
     uint8_t *codes;   // (rows, cols)
     float *inv_scale; // (cols)
     float *zero;      // (cols)
-    double *err;      // [kQMaxIters] sums of |w - w_r| per iteration
+    double *err;      // [sums][kQMaxIters]: |w - w_r| added up per iteration, each block in one of the sums
+    int sums;
     int first;        // solver pass: its first iteration
     float skip;       // shrink_skip(): residuals up to this one shrink to zero
+    float inv_beta[kQMaxIters]; // 1 / beta of every iteration
 };
 
 // CP consecutive values starting at element `at` (a multiple of CP)
@@ -132,10 +137,25 @@ __device__ __forceinline__ float solver_step(const QuantParams &p, const float (
 // threads of the block call it.
 __device__ __forceinline__ int solver_stop(const QuantParams &p, int known)
 {
+    static_assert(kQMaxIters == 64, "a wave's lanes are the iterations");
+    __shared__ double part[kQThreads / 64][kQMaxIters];
     __shared__ float mean[kQMaxIters];
     __shared__ int stop;
-    if ((int)threadIdx.x < known)
-        mean[threadIdx.x] = (float)(p.err[threadIdx.x] / ((double)p.rows * (double)p.cols));
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane < known) {
+        double t = 0.0;
+        for (int i = wave; i < p.sums; i += kQThreads / 64)
+            t += p.err[i * kQMaxIters + lane];
+        part[wave][lane] = t;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < known) {
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < kQThreads / 64; ++i)
+            t += part[i][threadIdx.x];
+        mean[threadIdx.x] = (float)(t / ((double)p.rows * (double)p.cols));
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         float best = 1e4f;
@@ -199,10 +219,7 @@ template <int GS, int CP, int PASS> __global__ __launch_bounds__(kQThreads) void
             for (int j = 0; j < CP; ++j)
                 zero[j] = from[cc + j];
         }
-        __shared__ double red[kQChunk][kQThreads / 64];
-        double beta = p.beta; // the host loop keeps beta as a double and hands 1 / beta to fp32 tensor ops
-        for (int it = 0; it < first; ++it)
-            beta *= p.kappa;
+        __shared__ float err_lds[kQChunk][kQThreads];
         float hi[CP], lo[CP]; // 1 / scale
 #pragma unroll
         for (int j = 0; j < CP; ++j) {
@@ -211,7 +228,7 @@ template <int GS, int CP, int PASS> __global__ __launch_bounds__(kQThreads) void
         }
 #pragma unroll 1
         for (int it = first; it < last; ++it) {
-            const float inv_beta = (float)(1.0 / beta);
+            const float inv_beta = p.inv_beta[it];
             float e = 0.f;
 #pragma unroll
             for (int j = 0; j < CP; ++j) {
@@ -219,23 +236,23 @@ template <int GS, int CP, int PASS> __global__ __launch_bounds__(kQThreads) void
                 asm volatile("" : "+v"(sc)); // keeps w * scale out of registers of its own across iterations
                 e += solver_step<GS, CP>(p, w, j, sc, hi[j], lo[j], inv_beta, zero[j]);
             }
-            beta *= p.kappa;
-            if constexpr (PASS == 1) {
-                double s = on ? (double)e : 0.0;
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1)
-                    s += __shfl_xor(s, off, 64);
-                if ((threadIdx.x & 63) == 0)
-                    red[it - first][threadIdx.x >> 6] = s;
-            }
+            if constexpr (PASS == 1)
+                err_lds[it - first][threadIdx.x] = on ? e : 0.f;
         }
         if constexpr (PASS == 1) {
+            // the block's errors, one wave an iteration, once all iterations are through: none waits for lane exchanges
             __syncthreads();
-            if ((int)threadIdx.x < last - first) {
+            const int lane = threadIdx.x & 63;
+            for (int it = threadIdx.x >> 6; it < last - first; it += kQThreads / 64) {
                 double t = 0.0;
+#pragma unroll
                 for (int i = 0; i < kQThreads / 64; ++i)
-                    t += red[threadIdx.x][i];
-                atomicAdd(&p.err[first + threadIdx.x], t);
+                    t += (double)err_lds[it][64 * i + lane];
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1)
+                    t += __shfl_xor(t, off, 64);
+                if (lane == 0)
+                    atomicAdd(&p.err[(int)(blockIdx.x % (unsigned)p.sums) * kQMaxIters + first + it], t);
             }
             if (on) {
                 float *to = odd ? p.inv_scale : p.zero;
@@ -276,10 +293,10 @@ template <int GS, int CP, int PASS> __global__ __launch_bounds__(kQThreads) void
     }
 }
 
-__global__ void quantize_clear_kernel(double *err)
+__global__ __launch_bounds__(kQThreads) void quantize_clear_kernel(double *err, int n)
 {
-    if (threadIdx.x < kQMaxIters)
-        err[threadIdx.x] = 0.0;
+    for (int i = threadIdx.x; i < n; i += kQThreads)
+        err[i] = 0.0;
 }
 
 // The largest residual a of which it is certain that a - (1 / beta) (a + 1e-8)^(p - 1) is not positive, in whatever
@@ -385,7 +402,7 @@ template <int GS, int CP> int run_groups_cp(const QuantParams &p, hipStream_t s)
         quantize_groups_kernel<GS, CP, 0><<<blocks, kQThreads, 0, s>>>(p);
         return launch_status();
     }
-    quantize_clear_kernel<<<1, 64, 0, s>>>(p.err);
+    quantize_clear_kernel<<<1, kQThreads, 0, s>>>(p.err, p.sums * kQMaxIters);
     QuantParams q = p;
     for (q.first = 0; q.first < p.iters; q.first += kQChunk)
         quantize_groups_kernel<GS, CP, 1><<<blocks, kQThreads, 0, s>>>(q);
@@ -414,7 +431,8 @@ template <int GS> int run_groups(const QuantParams &p, hipStream_t s)
 
 } // namespace
 
-size_t quantize_workspace_bytes() { return kQMaxIters * sizeof(double) + 64; }
+constexpr size_t kQSumBytes = kQMaxIters * sizeof(double); // four lines of memory: no two sums share one
+size_t quantize_workspace_bytes() { return kQSums * kQSumBytes + 64; }
 
 int launch_quantize_groups(const void *w, int fp32_in, int64_t rows, int64_t cols, int nbits, int round_zero, int iters,
                            float lp, double beta, double kappa, uint8_t *codes, float *inv_scale, float *zero, void *ws,
@@ -424,14 +442,20 @@ int launch_quantize_groups(const void *w, int fp32_in, int64_t rows, int64_t col
         return HQQ_E_SHAPE;
     if (cols >= (1ll << 31) * (int64_t)kQThreads)
         return HQQ_E_UNSUPPORTED;
-    if (iters > 0 && (!ws || ws_bytes < quantize_workspace_bytes() || (reinterpret_cast<uintptr_t>(ws) & 7u)))
+    // (one sum is enough to go on with)
+    if (iters > 0 && (!ws || ws_bytes < kQSumBytes + 64 || (reinterpret_cast<uintptr_t>(ws) & 7u)))
         return HQQ_E_WORKSPACE;
     QuantParams p = {};
     p.w = w, p.fp32_in = fp32_in, p.rows = rows, p.cols = cols;
     p.max_v = (float)((1 << nbits) - 1), p.round_zero = round_zero, p.iters = iters;
-    p.lp = lp, p.beta = beta, p.kappa = kappa;
+    p.lp = lp;
+    double b = beta; // the host loop keeps beta as a double and hands 1 / beta to fp32 tensor ops
+    for (int it = 0; it < iters; ++it, b *= kappa)
+        p.inv_beta[it] = (float)(1.0 / b);
     p.codes = codes, p.inv_scale = inv_scale, p.zero = zero;
     p.err = static_cast<double *>(ws);
+    const size_t room = (ws_bytes - (iters > 0 ? 64 : 0)) / kQSumBytes;
+    p.sums = room < (size_t)kQSums ? (int)room : kQSums;
     p.skip = shrink_skip(beta, kappa, iters, lp);
     switch (rows) {
     case 8: return run_groups<8>(p, s);
@@ -448,7 +472,7 @@ int launch_quantize_whole(const float *x, int64_t n, int nbits, uint8_t *codes, 
 {
     if (n < 1 || nbits < 1 || nbits > 8)
         return HQQ_E_SHAPE;
-    if (!ws || ws_bytes < quantize_workspace_bytes() || (reinterpret_cast<uintptr_t>(ws) & 7u))
+    if (!ws || ws_bytes < kQSumBytes + 64 || (reinterpret_cast<uintptr_t>(ws) & 7u))
         return HQQ_E_WORKSPACE;
     int *extremes = static_cast<int *>(ws);
     int64_t blocks = (n + 256 * 8 - 1) / (256 * 8);
