@@ -21,8 +21,11 @@
 // division the next, and all iterations ran before the stop was looked for.  The power is evaluated only where its term
 // can be other than zero (shrink_skip), the division is a product by the reciprocal in two floats (divide_by; sixteen
 // operations a value with a correction by the residual, 614 -> 576 us), and the blocks' error sums do not queue for one
-// line of memory (kQSums; 576 -> 510 us).  Times are of a 14336 x 4096 layer taken to 2 bits in groups of 16, stopped
-// within the third of five passes; it began at 2238 us, with the same bits.
+// line of memory (kQSums; 576 -> 510 us).  Registers set how many waves share a unit: sums that the compiler moved past a
+// branch kept two values of every weight alive with it (16 x 4 values a thread: 156 -> 113 registers, four waves for
+// three, 510 -> 462 us; 64 x 2: 496 -> 215, two waves for one, 3-bit 1876 -> 1057 us and 4-bit 1863 -> 1047 us by all
+// three steps).  Times are of a 14336 x 4096 layer, taken to 2 bits in groups of 16 where nothing else is said and then
+// stopped within the third of five passes; that one began at 2238 us, with the same bits.  Vector operations bound it.
 #include "hqq_common.hpp"
 
 #include <cmath>
@@ -113,6 +116,11 @@ __device__ __forceinline__ float solver_step(const QuantParams &p, const float (
         e += a;
         top = __builtin_fmaxf(top, a);
         acc += q - ws;
+        if (r % 16 == 15 || r == GS - 1) {
+            // the sums are made here, not past the branch below, where every q and ws would have to be kept until then
+            asm volatile("" : "+v"(e), "+v"(acc), "+v"(top));
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     if (__any(top > p.skip || !divide_safe(scale, zero))) {
         const float pm1 = p.lp - 1.0f;

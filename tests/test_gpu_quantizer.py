@@ -143,3 +143,26 @@ def test_solver_where_its_short_cuts_do_not_hold(kind, nbits, gs):
     assert (np.abs(gzero - zero.reshape(-1)) <= 1e-4 * 2 ** nbits + 6 * gs * 2.0 ** -24 * terms).all()
     moved = np.abs(gq.astype(int) - q.astype(int))
     assert moved.max() <= 1 and (moved != 0).mean() <= (0.02 if kind == "offset" else 2e-3)
+
+
+@pytest.mark.parametrize("nbits,gs,cols", [(2, 16, 4 * 256 * 5 + 4), (3, 64, 2 * 256 * 3 + 2), (4, 64, 1), (2, 8, 1021)])
+def test_solver_with_room_for_fewer_error_sums(nbits, gs, cols):
+    """The solver's error is added up in as many places as the workspace holds, down to one: the stop, and with it every
+    output, is the same (the sums are fp64, and the stop compares their fp32 means)."""
+    from mixtral_offloading_amd import _lib, hip_kernels
+    gen = torch.Generator(device="cuda").manual_seed(cols)
+    w = (torch.randn((gs, cols), device="cuda", generator=gen) * 0.02).half()
+    want = hip_kernels.quantize_groups(w, gs, nbits, iters=20)
+    full = int(_lib.lib.hqq_quantize_workspace_bytes())
+    for nbytes in (64 * 8 + 64, 2 * 64 * 8 + 64, 7 * 64 * 8 + 100, full):
+        ws = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+        got = [torch.empty_like(t) for t in want]
+        rc = _lib.lib.hqq_quantize_groups(w.data_ptr(), 0, gs, cols, nbits, 0, 20, 0.7, 10.0, 1.01, got[0].data_ptr(),
+                                          got[1].data_ptr(), got[2].data_ptr(), ws.data_ptr(), nbytes,
+                                          _lib.current_stream_ptr(w.device))
+        assert rc == 0
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), nbytes
+        assert bool((ws[nbytes:] == 0xA5).all())  # nothing past the end it was told of
+    assert _lib.lib.hqq_quantize_groups(w.data_ptr(), 0, gs, cols, nbits, 0, 20, 0.7, 10.0, 1.01, got[0].data_ptr(),
+                                        got[1].data_ptr(), got[2].data_ptr(), ws.data_ptr(), 64 * 8 + 63,
+                                        _lib.current_stream_ptr(w.device)) == -5
