@@ -37,8 +37,12 @@ constexpr int kQThreads = 256;
 constexpr int kQMaxIters = 64;
 constexpr int kQChunk = 4; // iterations between two looks at the stop: a pass more costs one read of the tensor
 // Sums of an iteration's error, blocks taking them in turn: atomics on one line follow each other at some 10 ns, so that
-// on a single sum the four of each of 3584 blocks (58.7 M values) take longer than the pass's arithmetic.
+// on a single sum the four of each of 3584 blocks (58.7 M values) take longer than the pass's arithmetic.  But every block
+// of every pass reads all sums, so a tensor of few blocks takes one for 32 of its blocks (groups of 8, 20 iterations, us
+// with one sum / 32 blocks a sum / 32 sums: 16 blocks 33.5 / 33.5 / 40.0, 256 blocks 56.0 / 38.4 / 41.0, 1024 blocks
+// 138.6 / 58.6 / 58.6; groups of 16 and 64 alike).
 constexpr int kQSums = 32;
+constexpr int kQBlocksPerSum = 32;
 
 struct QuantParams {
     const void *w;
@@ -52,7 +56,7 @@ struct QuantParams {
     float *inv_scale; // (cols)
     float *zero;      // (cols)
     double *err;      // [sums][kQMaxIters]: |w - w_r| added up per iteration, each block in one of the sums
-    int sums;
+    int sums;         // as many as the workspace has room for; launched with no more than the blocks are worth
     int first;        // solver pass: its first iteration
     float skip;       // shrink_skip(): residuals up to this one shrink to zero
     float inv_beta[kQMaxIters]; // 1 / beta of every iteration
@@ -410,11 +414,13 @@ template <int GS, int CP> int run_groups_cp(const QuantParams &p, hipStream_t s)
         quantize_groups_kernel<GS, CP, 0><<<blocks, kQThreads, 0, s>>>(p);
         return launch_status();
     }
-    quantize_clear_kernel<<<1, kQThreads, 0, s>>>(p.err, p.sums * kQMaxIters);
     QuantParams q = p;
+    const int worth = blocks / kQBlocksPerSum > 0 ? (int)(blocks / kQBlocksPerSum) : 1;
+    q.sums = worth < p.sums ? worth : p.sums;
+    quantize_clear_kernel<<<1, kQThreads, 0, s>>>(q.err, q.sums * kQMaxIters);
     for (q.first = 0; q.first < p.iters; q.first += kQChunk)
         quantize_groups_kernel<GS, CP, 1><<<blocks, kQThreads, 0, s>>>(q);
-    quantize_groups_kernel<GS, CP, 2><<<blocks, kQThreads, 0, s>>>(p);
+    quantize_groups_kernel<GS, CP, 2><<<blocks, kQThreads, 0, s>>>(q);
     return launch_status();
 }
 

@@ -166,3 +166,22 @@ def test_solver_with_room_for_fewer_error_sums(nbits, gs, cols):
     assert _lib.lib.hqq_quantize_groups(w.data_ptr(), 0, gs, cols, nbits, 0, 20, 0.7, 10.0, 1.01, got[0].data_ptr(),
                                         got[1].data_ptr(), got[2].data_ptr(), ws.data_ptr(), 64 * 8 + 63,
                                         _lib.current_stream_ptr(w.device)) == -5
+
+
+@pytest.mark.parametrize("gs,cols,sums", [(8, 1021, 1), (16, 4 * 256 * 63, 1), (16, 4 * 256 * 63 + 4, 2), (64, 2 * 256 * 96, 3)])
+def test_tensors_of_few_blocks_use_few_error_sums(gs, cols, sums):
+    """Every block of every pass reads all sums, so a tensor takes one for 32 of its blocks: the others are neither
+    cleared nor added to."""
+    from mixtral_offloading_amd import _lib, hip_kernels
+    gen = torch.Generator(device="cuda").manual_seed(cols)
+    w = (torch.randn((gs, cols), device="cuda", generator=gen) * 0.02).half()
+    want = hip_kernels.quantize_groups(w, gs, 2, iters=20)
+    got = [torch.empty_like(t) for t in want]
+    ws = torch.full((int(_lib.lib.hqq_quantize_workspace_bytes()),), 0x7F, dtype=torch.uint8, device="cuda")
+    assert _lib.lib.hqq_quantize_groups(w.data_ptr(), 0, gs, cols, 2, 0, 20, 0.7, 10.0, 1.01, got[0].data_ptr(),
+                                        got[1].data_ptr(), got[2].data_ptr(), ws.data_ptr(), ws.numel(),
+                                        _lib.current_stream_ptr(w.device)) == 0
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    err = ws[:sums * 512].view(torch.float64).view(sums, 64)
+    assert bool((err[:, 0] > 0).all()) and bool((err < w.numel()).all())  # cleared, and each added to
+    assert bool((ws[sums * 512:] == 0x7F).all())
