@@ -145,24 +145,25 @@ def test_solver_where_its_short_cuts_do_not_hold(kind, nbits, gs):
     assert moved.max() <= 1 and (moved != 0).mean() <= (0.02 if kind == "offset" else 2e-3)
 
 
-@pytest.mark.parametrize("nbits,gs,cols", [(2, 16, 4 * 256 * 5 + 4), (3, 64, 2 * 256 * 3 + 2), (4, 64, 1), (2, 8, 1021)])
+@pytest.mark.parametrize("nbits,gs,cols", [(2, 16, 4 * 256 * 1030 + 4), (3, 64, 2 * 256 * 70 + 2), (4, 64, 1), (2, 8, 256 * 1060 + 5)])
 def test_solver_with_room_for_fewer_error_sums(nbits, gs, cols):
-    """The solver's error is added up in as many places as the workspace holds, down to one: the stop, and with it every
-    output, is the same (the sums are fp64, and the stop compares their fp32 means)."""
+    """The solver's error is added up in as many places as the workspace holds and the blocks (1031, 71, 1 and 1061, one
+    sum for 32 of them) are worth, down to one: the stop, and with it every output, is the same (the sums are fp64, and
+    the stop compares their fp32 means).  The workspace starts as doubles of 1e306: a sum that is not cleared shows."""
     from mixtral_offloading_amd import _lib, hip_kernels
     gen = torch.Generator(device="cuda").manual_seed(cols)
     w = (torch.randn((gs, cols), device="cuda", generator=gen) * 0.02).half()
     want = hip_kernels.quantize_groups(w, gs, nbits, iters=20)
     full = int(_lib.lib.hqq_quantize_workspace_bytes())
     for nbytes in (64 * 8 + 64, 2 * 64 * 8 + 64, 7 * 64 * 8 + 100, full):
-        ws = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+        ws = torch.full((nbytes + 64,), 0x7F, dtype=torch.uint8, device="cuda")
         got = [torch.empty_like(t) for t in want]
         rc = _lib.lib.hqq_quantize_groups(w.data_ptr(), 0, gs, cols, nbits, 0, 20, 0.7, 10.0, 1.01, got[0].data_ptr(),
                                           got[1].data_ptr(), got[2].data_ptr(), ws.data_ptr(), nbytes,
                                           _lib.current_stream_ptr(w.device))
         assert rc == 0
         assert all(torch.equal(a, b) for a, b in zip(got, want)), nbytes
-        assert bool((ws[nbytes:] == 0xA5).all())  # nothing past the end it was told of
+        assert bool((ws[nbytes:] == 0x7F).all())  # nothing past the end it was told of
     assert _lib.lib.hqq_quantize_groups(w.data_ptr(), 0, gs, cols, nbits, 0, 20, 0.7, 10.0, 1.01, got[0].data_ptr(),
                                         got[1].data_ptr(), got[2].data_ptr(), ws.data_ptr(), 64 * 8 + 63,
                                         _lib.current_stream_ptr(w.device)) == -5
@@ -185,3 +186,43 @@ def test_tensors_of_few_blocks_use_few_error_sums(gs, cols, sums):
     err = ws[:sums * 512].view(torch.float64).view(sums, 64)
     assert bool((err[:, 0] > 0).all()) and bool((err < w.numel()).all())  # cleared, and each added to
     assert bool((ws[sums * 512:] == 0x7F).all())
+
+
+@pytest.mark.parametrize("last", [5, 31])
+def test_every_block_of_every_error_sum_counts_for_the_stop(last):
+    """1061 blocks on 32 sums, so that most sums take a block of each of the 33 rounds.  The error lies in every 32nd
+    block, all of one sum: with them the solver runs all 20 iterations, and what the other sums hold would stop it within
+    10, which a fiftieth of the groups shows.  A rounding of the power or of a group's mean flips a code of a group now and
+    then: a value has to lie within some 2^-21 of one of the three boundaries, in one of 8 x 20 looks, less than 1e-3 of
+    the groups."""
+    from mixtral_offloading_amd import _lib, hip_kernels
+    gs, cols = 8, 256 * 1060 + 5  # odd: one group a thread
+    rng = np.random.default_rng(last)
+    w = rng.standard_normal((gs, cols)) * 0.02
+    heavy = np.arange(cols) // 256 % 32 == last
+    w[:, heavy] = rng.random((gs, int(heavy.sum()))) * 2
+    w = w.astype(np.float16)
+    q, scale, zero = o.hqq_quantize_tensor(w, 2, gs, optimize=True)
+    # on the oracle: the other blocks alone stop within 10 iterations, and the tensor stopped there is another
+    early = o.hqq_quantize_tensor(w[:, ~heavy], 2, gs, optimize=True, iters=10)[2]
+    assert np.array_equal(early, o.hqq_quantize_tensor(w[:, ~heavy], 2, gs, optimize=True)[2])
+    for iters in (10, 19):
+        stopped = o.hqq_quantize_tensor(w, 2, gs, optimize=True, iters=iters)[2]
+        assert (np.abs(stopped - zero) > 4e-4).mean() > 1e-2
+    x = torch.from_numpy(w).cuda()
+    gq, gscale, gzero = hip_kernels.quantize_groups(x, gs, 2, iters=20)
+    assert np.array_equal(gscale.cpu().numpy(), scale.reshape(1, -1))
+    assert (np.abs(gzero.cpu().numpy() - zero.reshape(1, -1)) > 4e-4).mean() <= 1e-3
+    assert (gq.cpu().numpy() != q).mean() <= 1e-3
+    # the first iteration's error, sum by sum, from the oracle's codes before it: block b in sum b % 32
+    q0, s0, z0 = o.hqq_quantize_tensor(w, 2, gs)
+    s0 = np.float32(1) / s0  # (the outputs hold 1 / scale; the error is made with scale, an ulp beside)
+    err = np.abs(w.astype(np.float64) - (q0.astype(np.float64) - z0) / s0).sum(axis=0)
+    want = np.bincount(np.arange(cols) // 256 % 32, weights=err, minlength=32)
+    ws = torch.full((int(_lib.lib.hqq_quantize_workspace_bytes()),), 0x7F, dtype=torch.uint8, device="cuda")
+    assert _lib.lib.hqq_quantize_groups(x.data_ptr(), 0, gs, cols, 2, 0, 20, 0.7, 10.0, 1.01, gq.data_ptr(), gscale.data_ptr(),
+                                        gzero.data_ptr(), ws.data_ptr(), ws.numel(), _lib.current_stream_ptr(x.device)) == 0
+    sums = ws[:32 * 512].view(torch.float64).view(32, 64)[:, 0].cpu().numpy()
+    # a difference is good to some 2^-22 of its group's largest value, which is below ten times the mean difference, and
+    # the roundings of 8 that are added may all go one way (a lost block would be a 33rd)
+    assert np.allclose(sums, want, rtol=8 * 10 * 2.0 ** -22, atol=0)
