@@ -348,9 +348,11 @@ int hqq_attention_chain(const hqq_linear *q, const hqq_linear *k, const hqq_line
  *      loop, so that beta takes the same sequence of values; the solver stops for the whole tensor when the mean
  *      absolute error no longer falls), then q = clamp(round(w * scale + zero), 0, 2^nbits - 1).  Outputs: codes
  *      uint8 (rows, cols), unpacked; inv_scale fp32 (cols) = 1 / scale; zero fp32 (cols).  The workspace (8-byte
- *      aligned, hqq_quantize_workspace_bytes()) is only needed when iters > 0.  hqq_quantize_whole is the one-group
- *      form (channel_wise = False, the zero table's 8-bit meta): min and max over all n fp32 values; it always needs
- *      the workspace.                                                                                              */
+ *      aligned; its contents do not matter) is only needed when iters > 0.  hqq_quantize_workspace_bytes() holds all 32
+ *      of the sums on which a large tensor adds up its errors; from 576 bytes on (64, and 512 for each sum) a call goes
+ *      on with as many as there is room for, to the same outputs in more time (14336 x 4096 in groups of 16: 345 us with
+ *      32 sums, 778 with one), and less is HQQ_E_WORKSPACE.  hqq_quantize_whole is the one-group form (channel_wise =
+ *      False, the zero table's 8-bit meta): min and max over all n fp32 values; it always needs 576 bytes.          */
 size_t hqq_quantize_workspace_bytes(void);
 int hqq_quantize_groups(const void *w, int32_t w_is_fp32, int64_t rows, int64_t cols, int32_t nbits, int32_t round_zero,
                         int32_t iters, float lp_norm, double beta, double kappa, void *codes_u8, void *inv_scale_f32,

@@ -15,7 +15,8 @@
 // on several sums side by side) and leave the zero points they reached in one of the two output vectors (the next pass reads it and writes the
 // other, so both ends of a pass are at hand); every block of a later pass finds from the errors so far whether the
 // host loop would have stopped, and returns if so; the last pass repeats the iterations of the one pass the stop fell
-// into and writes the result.  All arithmetic is fp32 with separate multiplies and adds, as the tensor ops it replaces.
+// into and writes the result.  All arithmetic is fp32 with separate multiplies and adds, as the tensor ops it replaces;
+// only the quotients in the errors that decide the stop are made another way (divide_by).
 //
 // An iteration is a dozen operations a value.  It was over a hundred: the shrinkage's power took most of them and a full
 // division the next, and all iterations ran before the stop was looked for.  The power is evaluated only where its term
@@ -25,7 +26,12 @@
 // branch kept two values of every weight alive with it (16 x 4 values a thread: 156 -> 113 registers, four waves for
 // three, 510 -> 462 us; 64 x 2: 496 -> 215, two waves for one, 3-bit 1876 -> 1057 us and 4-bit 1863 -> 1047 us by all
 // three steps).  Times are of a 14336 x 4096 layer, taken to 2 bits in groups of 16 where nothing else is said and then
-// stopped within the third of five passes; that one began at 2238 us, with the same bits.  Vector operations bound it.
+// stopped within the third of five passes; that one began at 2238 us, with the same bits.
+//
+// What bounds it, by counters: in groups of 16 the vector units, whose instructions (50.6 M, four cycles each, on 1024
+// units) are 88 to 98 % of a pass of 86 to 98 us.  In groups of 64, with two waves to a unit, they are 49 % of 157 us, and
+// a wave waits for 54 % of its time: its 128 values arrive before it begins, and one other wave is there to cover that
+// (the same reads and no iteration: 67 us).
 #include "hqq_common.hpp"
 
 #include <cmath>
@@ -91,7 +97,8 @@ __device__ __forceinline__ float shrink_lp(float x, float inv_beta, float pm1)
 
 // x / s from 1 / s as the sum hi + lo of two floats.  The sum is within 2^-46 of 1 / s, so before its one rounding the
 // quotient is within 2^-45 of its size: it is rounded as a division rounds it unless it lies that near the middle
-// between two floats (one quotient in some millions, and then the other of the two neighbours).  Two operations, where
+// between two floats, and then to the other of two neighbours that are as good as equally far (25 of 8 * 10^9 quotients
+// of this kind, off by 0.50000004 of an ulp at most; the mean error is a division's, 0.25 ulp).  Two operations, where
 // correcting x * hi by the exact residual takes five.  Only the errors that decide the stop are made with it; neither
 // zero points nor codes are.  For |s| and |x| where nothing leaves the normal range: see divide_safe.
 __device__ __forceinline__ float divide_by(float x, float hi, float lo) { return __builtin_fmaf(x, hi, x * lo); }
@@ -445,7 +452,7 @@ template <int GS> int run_groups(const QuantParams &p, hipStream_t s)
 
 } // namespace
 
-constexpr size_t kQSumBytes = kQMaxIters * sizeof(double); // four lines of memory: no two sums share one
+constexpr size_t kQSumBytes = kQMaxIters * sizeof(double); // an iteration's words in the sums lie four lines of memory apart
 size_t quantize_workspace_bytes() { return kQSums * kQSumBytes + 64; }
 
 int launch_quantize_groups(const void *w, int fp32_in, int64_t rows, int64_t cols, int nbits, int round_zero, int iters,

@@ -120,8 +120,8 @@ def test_layer_quantised_on_the_gpu_equals_the_oracle_layer():
 @pytest.mark.parametrize("nbits,gs", [(2, 8), (2, 16), (3, 64), (4, 128)])
 def test_solver_where_its_short_cuts_do_not_hold(kind, nbits, gs):
     """Residuals large enough for the shrinkage to leave something (weights tens wide), groups without a spread, and
-    scales and zeros outside the range in which the quotient is corrected without a division: the tensor-op form's
-    results.  The solver's zero is a mean of gs fp32 terms of size |w| * scale, so another order of that sum moves it by
+    scales and zeros outside the range in which a quotient is a product by the reciprocal in two floats: the tensor-op
+    form's results.  The solver's zero is a mean of gs fp32 terms of size |w| * scale, so another order of that sum moves it by
     gs * 2^-24 of the largest."""
     from mixtral_offloading_amd import hip_kernels
     rng = np.random.default_rng(nbits * 1000 + gs)
