@@ -29,7 +29,7 @@
 // stopped within the third of five passes; that one began at 2238 us, with the same bits.
 //
 // What bounds it, by counters: in groups of 16 the vector units, whose instructions (50.6 M, four cycles each, on 1024
-// units) are 88 to 98 % of a pass of 86 to 98 us.  In groups of 64, with two waves to a unit, they are 49 % of 157 us, and
+// units) are 87 to 98 % of a pass of 86 to 98 us.  In groups of 64, with two waves to a unit, they are 49 % of 157 us, and
 // a wave waits for 54 % of its time: its 128 values arrive before it begins, and one other wave is there to cover that
 // (the same reads and no iteration: 67 us).
 #include "hqq_common.hpp"
