@@ -138,6 +138,18 @@ int hqq_expert_groups_ffn(const hqq_linear *const *w1, const hqq_linear *const *
                           int32_t n_groups, const int64_t *row_start, const void *x_f16, void *y_f16,
                           const void *row_scale_f16, void *workspace, size_t workspace_bytes, void *stream);
 
+/* ---- the same loop planned as a whole: every group's gate in one launch and every down projection in another (and a
+ *      finishing pass where K is split), whatever the groups' sizes.  A group whose layers are all NULL is left out of
+ *      the launches, and its rows of y alone, but the K split is planned for all rows: a row's result does not depend
+ *      on which groups come in the same call.  Results are hqq_expert_ffn's to rounding.  Layers of different shapes,
+ *      shapes that the kernel does not take (3-bit codes among them) and plans of too few blocks to fill the chip run
+ *      as hqq_expert_groups_ffn, the groups that are there.                                                        */
+size_t hqq_expert_rows_ffn_workspace_bytes(const hqq_linear *const *w1, const hqq_linear *const *w2,
+                                           const hqq_linear *const *w3, int32_t n_groups, const int64_t *row_start);
+int hqq_expert_rows_ffn(const hqq_linear *const *w1, const hqq_linear *const *w2, const hqq_linear *const *w3,
+                        int32_t n_groups, const int64_t *row_start, const void *x_f16, void *y_f16,
+                        const void *row_scale_f16, void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---- hqq_expert_ffn for callers that cannot allocate or carry a workspace (code under HIP graph capture, tight
  *      serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The workspace is an
  *      array of HQQ_STATIC_SCRATCH_BYTES built into the library's device code (every GPU the library runs on holds it

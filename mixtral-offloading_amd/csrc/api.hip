@@ -244,6 +244,26 @@ static bool lds_gate_preferred(const hqq_linear *w1, const hqq_linear *w3, int64
            ldsgemm_gate_supported(w1, w3, M);
 }
 
+// Whether the rows kernel takes an expert's FFN at M rows: both gate projections as one launch, the down projection as
+// another (and a finishing pass where K is split)
+static bool ffn_rows_supported(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, int64_t M)
+{
+    return !w1->bias && !w3->bias && rows_supported(w1, M) && rows_supported(w3, M) && rows_supported(w2, M) && rows_alike(w1, w3);
+}
+
+// Alone, an expert needs some hundreds of rows to fill the chip that way (2-bit Mixtral expert, the other kernels against
+// this one: 256 rows 137 / 165 us, 333 rows 223 / 160, 500 rows 247 / 200)
+static bool ffn_runs_rows_kernel(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, int64_t M)
+{
+    return M > 288 && ffn_rows_supported(w1, w2, w3, M);
+}
+
+static TileFinish rows_finish(const RowsItem &it, int kpb)
+{
+    return TileFinish{it.part, kpb, (int)it.M, (int)it.l0->N, 8 / it.l0->nbits, static_cast<const f16 *>(it.l0->bias), it.y,
+                      it.row_scale, it.accumulate};
+}
+
 // The matmul part with the partial sums of both gate projections.  What one projection's widest family needs holds them at
 // 14336x4096 (it is sized for the 4-bit rewrite of the codes), but not where the tile kernel does not take the shape: the
 // query counts them, and a call with a workspace that lacks them runs the projections one after the other.
@@ -251,7 +271,9 @@ static size_t ffn_gate_scratch(const hqq_linear *w1, const hqq_linear *w2, const
 {
     const size_t mm = ffn_matmul_scratch(w1, w2, w3, M);
     const size_t g = lds_gate_preferred(w1, w3, M) ? align256(ldsgemm_gate_workspace_bytes(w1, w3, M)) : 0;
-    return g > mm ? g : mm;
+    const size_t r = ffn_runs_rows_kernel(w1, w2, w3, M) ? workspace_head_bytes() + rows_partial_bytes(w2, M, rows_k_blocks(w2, M, rows_blocks(w2, M, false))) : 0;
+    const size_t most = g > r ? g : r;
+    return most > mm ? most : mm;
 }
 
 static size_t ffn_rows_bytes(const hqq_linear *w1, const hqq_linear *w2, int64_t M)
@@ -381,6 +403,22 @@ static int expert_ffn_impl(const hqq_linear *w1, const hqq_linear *w2, const hqq
     const f16 *x = (const f16 *)x_f16;
     f16 *y = (f16 *)y_f16;
 
+    // 17 rows and more: both gate projections in one launch, silu(a) * b in its blocks, then the down projection
+    if (ffn_runs_rows_kernel(w1, w2, w3, M) && aligned16(x)) {
+        const int kpb = rows_k_blocks(w2, M, rows_blocks(w2, M, false));
+        const size_t bytes = rows_partial_bytes(w2, M, kpb);
+        if (workspace_bytes >= ffn_gate_scratch(w1, w2, w3, M) + rows_bytes) // else the kernels that need no more than the least
+            mm_bytes = ffn_gate_scratch(w1, w2, w3, M), h = (f16 *)(p + mm_bytes);
+        if (workspace_head_bytes() + bytes <= mm_bytes) {
+            float *part = bytes ? reinterpret_cast<float *>(p + workspace_head_bytes()) : nullptr;
+            const RowsItem gate = {w1, w3, x, M, h, nullptr, nullptr, 0};
+            const RowsItem down = {w2, nullptr, h, M, y, part, (const f16 *)row_scale_f16, accumulate};
+            if ((rc = launch_rows(&gate, &kpb, 1, true, s)) != HQQ_OK || (rc = launch_rows(&down, &kpb, 1, false, s)) != HQQ_OK || !part)
+                return rc;
+            const TileFinish fin = rows_finish(down, kpb);
+            return launch_tile_finish_group(&fin, 1, s);
+        }
+    }
     // 3-bit decode batches: both gate projections in one launch, silu(a) * b folded into the down projection's loads
     if (pick_family(w1, M) == FAM_VEC3 && pick_family(w2, M) == FAM_VEC3 && vec3_ffn_supported(w1, w2, w3, M, 1)) {
         if ((rc = launch_vec3_gate(w1, w3, x, M, a, (int64_t)(mid / 2), 1, mm, mm_bytes, s)) != HQQ_OK)
@@ -594,6 +632,159 @@ int hqq_expert_groups_ffn(const hqq_linear *const *w1, const hqq_linear *const *
         }
     }
     return nf ? launch_tile_finish_group(fin, nf, (hipStream_t)stream) : HQQ_OK;
+}
+
+// ---- the same for the rows of a prompt or a decode batch, planned as a whole: every gate in one launch and every down
+// projection in another, whatever the groups' sizes.  Groups without layers are left out of the launches, not of the plan.
+// The first group that has layers, or null where the rows kernel does not take all of them together.
+static const hqq_linear *const *expert_rows_lead(const hqq_linear *const *w1, const hqq_linear *const *w2, const hqq_linear *const *w3,
+                                                 int32_t n_groups, const int64_t *row_start)
+{
+    const hqq_linear *const *lead = nullptr; // of w2
+    for (int g = 0; g < n_groups; ++g) {
+        const int64_t M = row_start[g + 1] - row_start[g];
+        if (M <= 0 || (!w1[g] && !w2[g] && !w3[g]))
+            continue;
+        if (validate_linear(w1[g]) != HQQ_OK || validate_linear(w2[g]) != HQQ_OK || validate_linear(w3[g]) != HQQ_OK ||
+            w2[g]->K != w1[g]->N || w2[g]->N != w1[g]->K || !ffn_rows_supported(w1[g], w2[g], w3[g], M))
+            return nullptr;
+        lead = lead ? lead : w2 + g;
+        if (!rows_alike(w1[lead - w2], w1[g]) || !rows_alike(*lead, w2[g]))
+            return nullptr;
+    }
+    if (!lead)
+        return nullptr;
+    // Few experts, or few rows of one, leave the chip idle: the kernels that split K further are faster then (2-bit Mixtral
+    // experts, one by one / together: four with a row each 80 / 92 us, eight 169 / 172, eight with two 202 / 168).
+    int64_t blocks = 0;
+    bool wide = false;
+    for (int g = 0; g < n_groups; ++g)
+        if (row_start[g + 1] > row_start[g]) {
+            blocks += rows_blocks(w1[lead - w2], row_start[g + 1] - row_start[g], true);
+            wide = wide || row_start[g + 1] - row_start[g] > 32;
+        }
+    return blocks >= (wide ? 160 : 512) ? lead : nullptr;
+}
+
+// blocks of all groups' down projections, K not split
+static int64_t expert_rows_blocks(const hqq_linear *w2, int32_t n_groups, const int64_t *row_start)
+{
+    int64_t blocks = 0;
+    for (int g = 0; g < n_groups; ++g)
+        if (row_start[g + 1] > row_start[g])
+            blocks += rows_blocks(w2, row_start[g + 1] - row_start[g], false);
+    return blocks;
+}
+
+// whether every group that has rows has layers
+static bool expert_rows_all(const hqq_linear *const *w1, const hqq_linear *const *w2, const hqq_linear *const *w3, int32_t n_groups,
+                            const int64_t *row_start)
+{
+    for (int g = 0; g < n_groups; ++g)
+        if (row_start[g + 1] > row_start[g] && (!w1[g] || !w2[g] || !w3[g]))
+            return false;
+    return true;
+}
+
+static size_t expert_rows_apart_bytes(const hqq_linear *const *w1, const hqq_linear *const *w2, const hqq_linear *const *w3,
+                                      int32_t n_groups, const int64_t *row_start)
+{
+    size_t need = 0;
+    for (int g = 0; g < n_groups; ++g) {
+        const int64_t M = row_start[g + 1] - row_start[g];
+        const size_t one = M > 0 && w1[g] && w2[g] && w3[g] ? hqq_expert_ffn_workspace_bytes(w1[g], w2[g], w3[g], M) : 0;
+        need = one > need ? one : need;
+    }
+    return need;
+}
+
+size_t hqq_expert_rows_ffn_workspace_bytes(const hqq_linear *const *w1, const hqq_linear *const *w2, const hqq_linear *const *w3,
+                                           int32_t n_groups, const int64_t *row_start)
+{
+    if (!w1 || !w2 || !w3 || !row_start || n_groups <= 0)
+        return 0;
+    const hqq_linear *const *lead = expert_rows_lead(w1, w2, w3, n_groups, row_start);
+    if (!lead)
+        return expert_rows_all(w1, w2, w3, n_groups, row_start) ? hqq_expert_groups_ffn_workspace_bytes(w1, w2, w3, n_groups, row_start)
+                                                                : expert_rows_apart_bytes(w1, w2, w3, n_groups, row_start);
+    const int64_t blocks = expert_rows_blocks(*lead, n_groups, row_start);
+    size_t need = workspace_head_bytes();
+    for (int g = 0; g < n_groups; ++g) {
+        const int64_t M = row_start[g + 1] - row_start[g];
+        if (M > 0 && w1[g])
+            need += align256((size_t)M * (size_t)w1[g]->N * sizeof(f16)) + rows_partial_bytes(w2[g], M, rows_k_blocks(w2[g], M, blocks));
+    }
+    return need;
+}
+
+int hqq_expert_rows_ffn(const hqq_linear *const *w1, const hqq_linear *const *w2, const hqq_linear *const *w3, int32_t n_groups,
+                        const int64_t *row_start, const void *x_f16, void *y_f16, const void *row_scale_f16, void *workspace,
+                        size_t workspace_bytes, void *stream)
+{
+    if (!w1 || !w2 || !w3 || !row_start)
+        return HQQ_E_NULL;
+    if (n_groups < 0 || row_start[0] != 0)
+        return HQQ_E_SHAPE;
+    for (int g = 0; g < n_groups; ++g)
+        if (row_start[g + 1] < row_start[g])
+            return HQQ_E_SHAPE;
+    const hqq_linear *const *lead = aligned16(x_f16) ? expert_rows_lead(w1, w2, w3, n_groups, row_start) : nullptr;
+    if (!lead && expert_rows_all(w1, w2, w3, n_groups, row_start))
+        return hqq_expert_groups_ffn(w1, w2, w3, n_groups, row_start, x_f16, y_f16, row_scale_f16, workspace, workspace_bytes, stream);
+    if (!lead) { // the same bits
+        for (int g = 0; g < n_groups; ++g) {
+            const int64_t lo = row_start[g], M = row_start[g + 1] - lo;
+            if (M == 0 || (!w1[g] && !w2[g] && !w3[g]))
+                continue;
+            if (!w1[g] || !w2[g] || !w3[g] || !x_f16 || !y_f16)
+                return HQQ_E_NULL;
+            const int rc = hqq_expert_ffn(w1[g], w2[g], w3[g], static_cast<const f16 *>(x_f16) + lo * w1[g]->K, M,
+                                          static_cast<f16 *>(y_f16) + lo * w2[g]->N,
+                                          row_scale_f16 ? static_cast<const f16 *>(row_scale_f16) + lo : nullptr, 0, workspace,
+                                          workspace_bytes, stream);
+            if (rc != HQQ_OK)
+                return rc;
+        }
+        return HQQ_OK;
+    }
+    if (!x_f16 || !y_f16)
+        return HQQ_E_NULL;
+    if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u) ||
+        workspace_bytes < hqq_expert_rows_ffn_workspace_bytes(w1, w2, w3, n_groups, row_start))
+        return HQQ_E_WORKSPACE;
+    hipStream_t s = (hipStream_t)stream;
+    const int64_t blocks = expert_rows_blocks(*lead, n_groups, row_start);
+    char *at = static_cast<char *>(workspace) + workspace_head_bytes(); // the head holds other kernels' counters
+    RowsItem gate[kTileFinishGroupMax], down[kTileFinishGroupMax];
+    TileFinish fin[kTileFinishGroupMax];
+    int kpb[kTileFinishGroupMax], n = 0, rc;
+    const auto flush = [&]() -> int {
+        int nf = 0;
+        for (int i = 0; i < n; ++i)
+            if (down[i].part)
+                fin[nf++] = rows_finish(down[i], kpb[i]);
+        if (n == 0 || (rc = launch_rows(gate, kpb, n, true, s)) != HQQ_OK || (rc = launch_rows(down, kpb, n, false, s)) != HQQ_OK)
+            return n ? rc : HQQ_OK;
+        n = 0;
+        return nf ? launch_tile_finish_group(fin, nf, s) : HQQ_OK;
+    };
+    for (int g = 0; g < n_groups; ++g) {
+        const int64_t lo = row_start[g], M = row_start[g + 1] - lo;
+        if (M == 0 || !w1[g])
+            continue;
+        if (n == kTileFinishGroupMax && (rc = flush()) != HQQ_OK)
+            return rc;
+        f16 *h = reinterpret_cast<f16 *>(at);
+        at += align256((size_t)M * (size_t)w1[g]->N * sizeof(f16));
+        kpb[n] = rows_k_blocks(w2[g], M, blocks);
+        const size_t bytes = rows_partial_bytes(w2[g], M, kpb[n]);
+        gate[n] = RowsItem{w1[g], w3[g], static_cast<const f16 *>(x_f16) + lo * w1[g]->K, M, h, nullptr, nullptr, 0};
+        down[n] = RowsItem{w2[g], nullptr, h, M, static_cast<f16 *>(y_f16) + lo * w2[g]->N, bytes ? reinterpret_cast<float *>(at) : nullptr,
+                           row_scale_f16 ? static_cast<const f16 *>(row_scale_f16) + lo : nullptr, 0};
+        at += bytes;
+        ++n;
+    }
+    return flush();
 }
 
 // ---- the expert FFN for callers that cannot allocate.  The workspace is a file-scope device array; each GPU holds

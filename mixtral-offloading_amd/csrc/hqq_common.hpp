@@ -291,6 +291,22 @@ int launch_attention_decode(const f16 *q, const f16 *k, const f16 *v, const f16 
                             hipStream_t s, void *ws = nullptr, size_t ws_bytes = 0);
 int attention_parts(int64_t max_len); // blocks per head of the attention launch
 size_t attention_workspace_bytes(int64_t max_len, int n_heads, int head_dim);
+// rows_tile.hip: batches of 17 rows and more, the experts of a MoE layer in common launches
+struct RowsItem {
+    const hqq_linear *l0, *l1; // l1: the gate's second projection
+    const f16 *x;
+    int64_t M;
+    f16 *y;
+    float *part;               // rows_k_blocks(...) > 1: that many partial sums per output, finished by launch_tile_finish_group
+    const f16 *row_scale;
+    int accumulate;
+};
+bool rows_supported(const hqq_linear *l, int64_t M);
+bool rows_alike(const hqq_linear *a, const hqq_linear *b);
+int64_t rows_blocks(const hqq_linear *l, int64_t M, bool gate); // of a launch whose K is not split
+int rows_k_blocks(const hqq_linear *l, int64_t M, int64_t blocks); // blocks: of all members of the launch
+size_t rows_partial_bytes(const hqq_linear *l, int64_t M, int kpb);
+int launch_rows(const RowsItem *item, const int *kpb, int n, bool gate, hipStream_t s);
 // dequant_gemm.hip: wide batches as hqq_dequantize into the workspace + one library GEMM
 bool dqgemm_supported(const hqq_linear *l, int64_t M);
 bool dqgemm_preferred(const hqq_linear *l, int64_t M);

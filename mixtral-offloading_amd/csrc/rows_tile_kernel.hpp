@@ -1,0 +1,480 @@
+// Batch rows through the quantised layers of several experts in one launch, on the matrix cores (2- and 4-bit codes; included by
+// one translation unit per code width).
+//
+// A block is eight wavefronts on one tile of at most 128 (4-bit: 96) batch rows.  A wave owns the 64 output rows of one packed
+// row that share table rows (2-bit: 16 rows r of four fields; 4-bit: 32 rows of two), so its lanes hold 16 code bytes of a row
+// and every weight is rebuilt in registers, once per block: mask-and-insert, subtract, fma with the scale and minus scale * zero.
+// Per 128 columns the block reads its x tile straight into LDS (operand order, one barrier), each wave de-quantises its own
+// table entries into LDS, and a wave issues 16 groups of ct MFMAs; see the loop for how they overlap.
+//   * scale * zero is rounded once, from 32 bits, and the weight once: against 64 bits the FFN of a 2-bit expert is off by
+//     0.92e-3, with the reference's five roundings of a weight by 1.45e-3 (4-bit 1.07e-3, 1.23e-3).
+//   * Up to 64 rows there are few MFMAs to hide behind: the block's waves split its columns in two halves and meet in LDS, and up
+//     to 32 rows 128 registers let two blocks share a unit.  There the loads of a step (codes, tables, their meta, x) bound the
+//     launch: eight 2-bit Mixtral experts with 1 to 16 rows each take 170 us (3.1 TB/s), with 32 rows 208 us; the launches of one
+//     expert after the other 172 to 256 and 411 us.
+//   * From 65 rows on the matrix cores' issue does: 3.1 vector instructions an MFMA, two waves to a SIMD.  Eight experts with
+//     128 rows 402 us (897 TFLOP/s), with 500 rows 1332 us (1058 TFLOP/s); one after the other 788 and 1929 us.  What that took,
+//     at 500 rows: the tables read two groups ahead 1522 -> 1437 us, x straight to LDS and the vector instructions spread between
+//     the MFMAs (their own registers are then free for the operands of the next step) 1437 -> 1376, loads from a uniform base
+//     1376 -> 1332.
+#pragma once
+
+#include "gemv_parts.hpp"
+#include "rows_tile.hpp"
+
+namespace hqq {
+namespace rows {
+namespace {
+
+using gemv::gload;
+// The arguments stay where the launch put them: read through a pointer to them, not copied to be indexed.
+#define HQQ_KERNARG __attribute__((address_space(4)))
+#define HQQ_LDS __attribute__((address_space(3)))
+
+// A load from a base that is the same for the whole wave and a 32-bit byte offset of the lane
+template <typename T> __device__ __forceinline__ T load_at(const void *base, uint32_t offset)
+{
+    return *(const T __attribute__((address_space(1))) *)((const char __attribute__((address_space(1))) *)base + offset);
+}
+
+__device__ __forceinline__ float uniform(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
+constexpr int kWaitLoads = 0x0F70; // vmcnt(0), the other counters left alone
+
+template <int BITS> struct Codes {
+    static constexpr int F = 8 / BITS;       // output rows per packed row
+    static constexpr int RBW = 4 / F;        // row blocks of sixteen a wave takes (they share its table rows)
+    static constexpr int RT = F * RBW;       // 16-row tiles per wave
+    static constexpr int pos(int f) { return BITS * (F - 1 - f); }
+    static constexpr uint32_t mask(int f) { return (((1u << BITS) - 1u) * 0x00010001u) << pos(f); }
+    // a field masked in place and OR-ed into the mantissa of 2^(10 - pos) reads as 2^(10 - pos) + code
+    static constexpr uint32_t expo(int f) { return (uint32_t)((10 - pos(f) + 15) << 10) * 0x00010001u; }
+};
+
+__device__ __forceinline__ f16x2 h2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
+__device__ __forceinline__ uint32_t u2(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+
+template <int BITS, int CT, bool GATE, int KW, bool F16T>
+__device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member HQQ_KERNARG &g, int unit, int kp, int col, char *lds)
+{
+    typedef Codes<BITS> C;
+    constexpr int F = C::F, RBW = C::RBW, RT = C::RT;
+    constexpr int NWK = kBlockWaves / KW;           // waves per K half
+    constexpr int JW = NWK / (GATE ? 2 : 1);        // packed rows per block
+    constexpr int XTILE = 4 * CT * 64 * 16;         // bytes of one x tile: [q][row tile][lane] 16-byte operands
+    constexpr int TTILE = 4 * F * 4 * 32;           // bytes of one wave's tables: [q][field][k group] 8 scales, 8 zeros
+    constexpr int XCH = (4 * CT + NWK - 1) / NWK;   // operands a lane stages per step
+    char *const x_lds = lds, *const t_lds = lds + 2 * KW * XTILE;
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kh = KW == 1 ? 0 : wave / NWK, wk = KW == 1 ? wave : wave % NWK;
+    const int proj = GATE ? wk & 1 : 0, jl = GATE ? wk >> 1 : wk;
+    const int jblk = unit / p.RBU, rbu = unit - jblk * p.RBU;
+    const int jw = jblk * JW + jl;
+    const bool live = jw < p.GP;
+    const int jp = live ? jw : p.GP - 1;
+    const uint8_t *const l_codes = g.l[proj].codes, *const l_sq = g.l[proj].sq, *const l_zq = g.l[proj].zq;
+    const f16 *const l_sms = g.l[proj].s_ms, *const l_smz = g.l[proj].s_mz;
+    const int rr = lane & 15, kg = lane >> 4;
+    const int K = p.K, M = g.M;
+    const int m0 = col * (CT * 16);
+
+    const int b0 = kp * g.spp, b1 = b0 + g.spp < p.steps ? b0 + g.spp : p.steps;
+    const int nh = (b1 - b0 + KW - 1) / KW;                   // iterations of every wave of the block
+    const int from = b0 + kh * nh, s0 = from < b1 ? from : b1 - 1;
+    const int mine = from >= b1 ? 0 : (b1 - from < nh ? b1 - from : nh); // steps of this wave's K half
+    const int last = mine > 0 ? mine - 1 : 0;
+
+    uint32_t co[RBW];
+#pragma unroll
+    for (int w = 0; w < RBW; ++w)
+        co[w] = (uint32_t)(jp + (16 * (rbu * RBW + w) + rr) * p.GP) * (uint32_t)K + 16u * kg;
+    // a lane de-quantises TE entries of one of the wave's table rows per step: columns tk .. tk + TE - 1 of row ti
+    constexpr int TE = 2 * F;
+    const int ti = lane / (kStep / TE), tk = TE * (lane % (kStep / TE));
+    const uint32_t trow = (uint32_t)(F * jp + ti) * (uint32_t)K + (uint32_t)tk;
+    uint32_t cm0 = 0;
+    float zneg = 0.f, zoff = 0.f; // -zero = zoff + code * zneg
+    if constexpr (!F16T) {
+        zneg = uniform(-(float)gload<f16>(g.l[proj].z_ms));
+        zoff = uniform(-(float)gload<f16>(g.l[proj].z_mz) * zneg);
+        const uint32_t c = trow + (uint32_t)s0 * kStep;
+        cm0 = c - __umulhi(c, p.s_inv) * p.s_cols; // c mod columns: the quotient estimate is at most 2 short
+        cm0 -= cm0 >= p.s_cols ? p.s_cols : 0;
+        cm0 -= cm0 >= p.s_cols ? p.s_cols : 0;
+    }
+    // The x tile goes to LDS without passing the registers, sixteen bytes a lane in operand order.  (By hand: the compiler
+    // would wait for the transfer before the next LDS read, whichever half of the buffer that reads.)
+    const f16 *xb = g.x + (size_t)m0 * K + (size_t)s0 * kStep;
+    uint32_t xo[XCH], xd[XCH]; // byte offsets: a lane's in x, the wave's in LDS
+#pragma unroll
+    for (int c = 0; c < XCH; ++c) {
+        int pi = wk + NWK * c;
+        pi = pi < 4 * CT ? pi : 4 * CT - 1;
+        const int q = pi & 3, b = pi >> 2;
+        const int m = m0 + 16 * b + rr < M ? 16 * b + rr : M - 1 - m0;
+        xo[c] = 2 * ((uint32_t)m * (uint32_t)K + 64 * (q >> 1) + 16 * kg + 8 * (q & 1));
+        xd[c] = (uint32_t)(uintptr_t)(HQQ_LDS char *)x_lds + kh * XTILE + (q * CT + b) * 1024;
+    }
+
+    // With two row blocks the codes of the next step are read into the registers of this one's as these fall free, a slab
+    // of 64 columns at a time; with one they have registers of their own and the whole step to arrive.
+    constexpr bool LATE = RBW == 2;
+    typedef uint32_t Halves __attribute__((ext_vector_type(TE / 2)));
+    typedef uint32_t Bytes __attribute__((ext_vector_type(TE / 4)));
+    struct Next {
+        u32x4 cw[LATE ? 1 : RBW][2];
+        Halves a, b; // meta of the scale / fp16 scales, fp16 zeros
+        Bytes sq, zq;
+    };
+    auto codes_at = [&](int w, uint32_t k) __attribute__((always_inline)) { return load_at<u32x4>(l_codes + k, co[w]); };
+    auto issue = [&](Next &r, int it, int buf) __attribute__((always_inline)) {
+        const int st = it < last ? it : last;
+        const uint32_t k0 = (uint32_t)(s0 + st) * kStep;
+        const f16 *const xs = xb + (size_t)st * kStep;
+#pragma unroll
+        for (int c = 0; c < XCH; ++c) // (past the end: the last operand once more, the same bytes to the same place)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                         : : "v"(xo[c]), "s"(xs), "s"(xd[c] + buf * (KW * XTILE)) : "memory");
+        if constexpr (F16T) {
+            r.a = load_at<Halves>(l_sq + 2 * (size_t)k0, 2 * trow);
+            r.b = load_at<Halves>(l_zq + 2 * (size_t)k0, 2 * trow);
+        } else {
+            r.sq = load_at<Bytes>(l_sq + k0, trow);
+            r.zq = load_at<Bytes>(l_zq + k0, trow);
+            uint32_t cm = cm0 + (uint32_t)st * kStep; // less than K + columns
+            cm -= __umulhi(cm, p.s_inv) * p.s_cols;
+            cm -= cm >= p.s_cols ? p.s_cols : 0;
+            cm -= cm >= p.s_cols ? p.s_cols : 0;
+            r.a = load_at<Halves>(l_sms, 2 * cm);
+            r.b = load_at<Halves>(l_smz, 2 * cm);
+        }
+        if constexpr (!LATE) {
+            r.cw[0][0] = codes_at(0, k0);
+            r.cw[0][1] = codes_at(0, k0 + 64);
+        }
+    };
+    // where they go: slab tk / 64, k group (tk / 16) % 4, half (tk / 8) % 2
+    char *const t_w = t_lds + wave * TTILE + (((((tk >> 6) * 2 + ((tk >> 3) & 1)) * F + ti) * 4 + ((tk >> 4) & 3)) * 32) + 2 * (tk & 7);
+    auto stage = [&](const Next &r, int buf) __attribute__((always_inline)) {
+        Halves S, Z;
+#pragma unroll
+        for (int e = 0; e < TE / 2; ++e) {
+            if constexpr (F16T) {
+                S[e] = r.a[e];
+                Z[e] = u2(-(h2(r.b[e]) * h2(r.a[e])));
+            } else {
+                f16x2 sv, zv;
+#pragma unroll
+                for (int o = 0; o < 2; ++o) {
+                    uint32_t sw, zw;
+                    if constexpr (TE == 8)
+                        sw = r.sq[e >> 1], zw = r.zq[e >> 1];
+                    else
+                        sw = r.sq[0], zw = r.zq[0];
+                    const int sh = 8 * ((2 * e + o) & 3);
+                    const float sc = (float)((sw >> sh) & 0xFFu), zc = (float)((zw >> sh) & 0xFFu);
+                    const float d = __builtin_fmaf((float)h2(r.b[e])[o], -1.0f, sc);
+                    sv[o] = (f16)__builtin_fmaf(d, (float)h2(r.a[e])[o], 0.0f);
+                    zv[o] = (f16)__builtin_fmaf(__builtin_fmaf(zc, zneg, zoff), (float)sv[o], 0.0f);
+                }
+                S[e] = u2(sv), Z[e] = u2(zv);
+            }
+        }
+        char *const d = t_w + buf * (kBlockWaves * TTILE);
+        *reinterpret_cast<Halves *>(d) = S;
+        *reinterpret_cast<Halves *>(d + 16) = Z;
+    };
+
+    f32x4 acc[RT][CT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int b = 0; b < CT; ++b)
+            acc[i][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    uint32_t expo[F]; // in vector registers: with a second scalar operand the insertion would be two instructions
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        expo[f] = C::expo(f);
+        asm volatile("" : "+v"(expo[f]));
+    }
+    Next nx;
+    u32x4 cw[RBW][2];
+    issue(nx, 0, 0);
+#pragma unroll
+    for (int w = 0; w < RBW; ++w)
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+            cw[w][o] = LATE ? codes_at(w, (uint32_t)s0 * kStep + 64 * o) : nx.cw[0][o];
+    stage(nx, 0);
+    __builtin_amdgcn_s_waitcnt(kWaitLoads);
+    __syncthreads();
+    for (int it = 0; it < nh; ++it) {
+        const int buf = it & 1;
+        issue(nx, it + 1, buf ^ 1);
+        if (KW == 1 || it < mine) {
+            const char *xr = x_lds + (buf * KW + kh) * XTILE + lane * 16;
+            const char *tr = t_lds + buf * (kBlockWaves * TTILE) + wave * TTILE + kg * 32;
+            // Groups of CT MFMAs: while those of group g run, the weights of group g + 1 are built and the tables of
+            // group g + 2 are read (the compiler's own order reads them where they are used, and waits).
+            constexpr int NG = 4 * RT;
+            u32x4 S[2], Z[2], A[2];
+            f16x8 B[CT];
+            uint32_t P[4];
+            auto tables = [&](int h) __attribute__((always_inline)) { // h = q * F + field
+                S[h & 1] = *reinterpret_cast<const u32x4 *>(tr + h * 128);
+                Z[h & 1] = *reinterpret_cast<const u32x4 *>(tr + h * 128 + 16);
+            };
+            auto operand = [&](int q, int b) __attribute__((always_inline)) {
+                return *reinterpret_cast<const f16x8 *>(xr + (q * CT + b) * 1024);
+            };
+            auto build = [&](int gi) __attribute__((always_inline)) { // group gi = (q * RBW + row block) * F + field
+                const int f = gi % F, w = gi / F % RBW, q = gi / RT, h = q * F + f;
+                if (f == 0)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        P[t] = __builtin_amdgcn_perm(0u, cw[w][q >> 1][2 * (q & 1) + (t >> 1)], t & 1 ? 0x0c030c02u : 0x0c010c00u);
+                const f16 offv = (f16)(float)(1 << (10 - C::pos(f)));
+                const f16x2 off = {offv, offv};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const f16x2 v = h2((P[t] & C::mask(f)) | expo[f]) - off; // the exact code
+                    A[gi & 1][t] = u2(__builtin_elementwise_fma(v, h2(S[h & 1][t]), h2(Z[h & 1][t])));
+                }
+            };
+            tables(0);
+#pragma unroll
+            for (int b = 0; b < CT; ++b)
+                B[b] = operand(0, b);
+            tables(1);
+            build(0);
+#pragma unroll
+            for (int gi = 0; gi < NG; ++gi) {
+                const int f = gi % F, w = gi / F % RBW, q = gi / RT;
+                __builtin_amdgcn_sched_barrier(0);
+                if (gi + 1 < NG)
+                    build(gi + 1);
+                // the tables two fields on, once the last row block that uses those in their place has been built
+                constexpr int LAST = (RBW - 1) * F;
+                if (gi > 0 && (gi + 1) % RT >= LAST && (gi + 1) / RT * F + (gi + 1) % F + 2 < 4 * F && RBW > 1)
+                    tables((gi + 1) / RT * F + (gi + 1) % F + 2);
+                else if (RBW == 1 && gi + 2 < NG && gi + 2 >= 2)
+                    tables(gi + 2);
+                if (LATE && (q & 1) && f == 0) // (a slab's last codes are taken apart when its second half begins)
+                    cw[w][q >> 1] = codes_at(w, (uint32_t)(s0 + (it < last ? it + 1 : last)) * kStep + 64 * (q >> 1));
+                const bool turn = f == F - 1 && w == RBW - 1 && q + 1 < 4; // the last MFMAs on these operands
+#pragma unroll
+                for (int b = 0; b < CT; ++b) {
+                    acc[w * F + f][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, A[gi & 1]), B[b],
+                                                                               acc[w * F + f][b], 0, 0, 0);
+                    if (turn)
+                        B[b] = operand(q + 1, b);
+                }
+                // an MFMA, what its operand's register is read into next, and the vector instructions that it hides
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (12 + CT - 1) / CT, 0);
+#pragma unroll
+                for (int b = 1; b < CT; ++b) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, (12 + CT - 1) / CT, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (it + 1 < nh) {
+            stage(nx, buf ^ 1);
+            if constexpr (!LATE)
+                cw[0][0] = nx.cw[0][0], cw[0][1] = nx.cw[0][1];
+        }
+        __builtin_amdgcn_s_waitcnt(kWaitLoads); // the x tile has arrived
+        __syncthreads();
+    }
+
+    // The K halves' sums meet in LDS; the first half finishes the tiles below CB, the second one the others.  (Which
+    // values a wave keeps is selected value by value: with one branch per half the accumulators would be addressed.)
+    constexpr int CB = KW == 1 ? CT : (CT + 1) / 2;
+    f32x4 sum[RT][CB];
+    if constexpr (KW == 2) {
+        f32x4 *const kx = reinterpret_cast<f32x4 *>(lds) + lane; // [wk][K half][tile][row tile][lane]
+#pragma unroll
+        for (int j = 0; j < CB; ++j)
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const f32x4 hi = acc[i][CB + j < CT ? CB + j : j];
+                sum[i][j] = kh ? hi : acc[i][j];
+                kx[(((wk * 2 + kh) * CB + j) * RT + i) * 64] = kh ? acc[i][j] : hi;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CB; ++j)
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+                sum[i][j] += kx[(((wk * 2 + 1 - kh) * CB + j) * RT + i) * 64];
+        if constexpr (GATE)
+            __syncthreads();
+    } else {
+#pragma unroll
+        for (int j = 0; j < CB; ++j)
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+                sum[i][j] = acc[i][j];
+    }
+    // sum[i][j][v]: batch row 16 * (kh * CB + j) + rr of the block's, field i % F, row 4 * kg + v of row block i / F
+    auto row_group = [&](int w, int v) __attribute__((always_inline)) {
+        return (uint32_t)jp + (uint32_t)(16 * (rbu * RBW + w) + 4 * kg + v) * (uint32_t)p.GP;
+    };
+    if constexpr (GATE) {
+        // both projections' waves hold the same outputs: each sends the other the tiles that it finishes
+        constexpr int M0 = (CB + 1) / 2; // the first projection's waves finish the tiles below M0
+        uint32_t *const gx = reinterpret_cast<uint32_t *>(lds) + lane; // [wave][tile][8 pairs][lane]
+        f32x4 own[RT][M0];
+#pragma unroll
+        for (int j = 0; j < M0; ++j)
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const f32x4 hi = sum[i][M0 + j < CB ? M0 + j : j], lo = sum[i][j], out = proj ? lo : hi;
+                own[i][j] = proj ? hi : lo;
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    gx[((wave * M0 + j) * (2 * RT) + 2 * i + h) * 64] = u2((f16x2){(f16)out[2 * h], (f16)out[2 * h + 1]});
+            }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < M0; ++j) {
+            const int jb = proj * M0 + j, tb = kh * CB + jb, m = m0 + 16 * tb + rr;
+            if (jb >= CB || tb >= CT || m >= M || !live)
+                continue;
+            f16 o[RT][4];
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const f16x2 other = h2(gx[(((wave ^ 1) * M0 + j) * (2 * RT) + 2 * i + h) * 64]);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const f16 mine16 = (f16)own[i][j][2 * h + e];
+                        const float u = (float)(proj ? other[e] : mine16);
+                        const f16 up = proj ? mine16 : other[e];
+                        o[i][2 * h + e] = (f16)(u / (1.0f + __expf(-u))) * up; // rounded thrice, as the reference's three operations
+                    }
+                }
+#pragma unroll
+            for (int w = 0; w < RBW; ++w)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    f16 *dst = g.y + (size_t)m * p.N + (size_t)F * row_group(w, v);
+                    if constexpr (F == 4)
+                        *reinterpret_cast<f16x4 *>(dst) = (f16x4){o[0][v], o[1][v], o[2][v], o[3][v]};
+                    else
+                        *reinterpret_cast<f16x2 *>(dst) = (f16x2){o[w * F][v], o[w * F + 1][v]};
+                }
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            const int tb = kh * CB + j, m = m0 + 16 * tb + rr;
+            if (tb >= CT || m >= M || !live)
+                continue;
+#pragma unroll
+            for (int w = 0; w < RBW; ++w)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const uint32_t rg = row_group(w, v);
+                    if (g.part) {
+                        float *dst = g.part + (((size_t)kp * (p.N / F) + rg) * M + m) * F;
+                        if constexpr (F == 4)
+                            *reinterpret_cast<f32x4 *>(dst) = (f32x4){sum[0][j][v], sum[1][j][v], sum[2][j][v], sum[3][j][v]};
+                        else
+                            *reinterpret_cast<float2 *>(dst) = make_float2(sum[w * F][j][v], sum[w * F + 1][j][v]);
+                        continue;
+                    }
+                    f16 o[F];
+                    f16 *dst = g.y + (size_t)m * p.N + (size_t)F * rg;
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        o[f] = (f16)sum[w * F + f][j][v];
+                        if (g.bias)
+                            o[f] = o[f] + g.bias[F * rg + f];
+                        if (g.row_scale)
+                            o[f] = o[f] * g.row_scale[m];
+                        if (g.accumulate)
+                            o[f] = dst[f] + o[f];
+                    }
+                    if constexpr (F == 4)
+                        *reinterpret_cast<f16x4 *>(dst) = (f16x4){o[0], o[1], o[2], o[3]};
+                    else
+                        *reinterpret_cast<f16x2 *>(dst) = (f16x2){o[0], o[1]};
+                }
+        }
+    }
+}
+
+template <int BITS> constexpr size_t lds_bytes(int max_ct, int kw)
+{
+    return (size_t)2 * kw * 4 * max_ct * 1024 + (size_t)2 * kBlockWaves * 4 * Codes<BITS>::F * 128;
+}
+
+// WIDE: members of any number of rows; else of at most 32, whose few accumulators let two blocks share a compute unit
+template <int BITS, bool GATE, bool WIDE, bool F16T>
+__global__ __launch_bounds__(kBlockWaves * 64, WIDE ? 2 : 4) void rows_tile_kernel(Params)
+{
+    const Params HQQ_KERNARG &p = *(const Params HQQ_KERNARG *)__builtin_amdgcn_kernarg_segment_ptr();
+    __shared__ __attribute__((aligned(16))) char lds[WIDE ? lds_bytes<BITS>(8, 1) : lds_bytes<BITS>(2, 2)];
+    // eight consecutive blocks run on eight dies: entry e of the list stands for a row block of each
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    int k = 0;
+    while (k + 1 < p.n && p.m[k + 1].first <= slot)
+        ++k;
+    const Member HQQ_KERNARG &g = p.m[k];
+    const int local = slot - g.first, rr = local / g.ncol, col = local - rr * g.ncol;
+    const int ru = rr * 8 + xcd;
+    if (ru >= g.units * g.kpb)
+        return;
+    const int kp = ru / g.units, unit = ru - kp * g.units;
+    if constexpr (WIDE) {
+        switch (g.ct) {
+        case 1: return tile<BITS, 1, GATE, 2, F16T>(p, g, unit, kp, col, lds);
+        case 2: return tile<BITS, 2, GATE, 2, F16T>(p, g, unit, kp, col, lds);
+        case 3: return tile<BITS, 3, GATE, 2, F16T>(p, g, unit, kp, col, lds);
+        case 4: return tile<BITS, 4, GATE, 2, F16T>(p, g, unit, kp, col, lds);
+        case 5: return tile<BITS, 5, GATE, 1, F16T>(p, g, unit, kp, col, lds);
+        case 6: return tile<BITS, 6, GATE, 1, F16T>(p, g, unit, kp, col, lds);
+        default: break;
+        }
+        if constexpr (max_tiles(BITS) == 8) {
+            if (g.ct == 7)
+                tile<BITS, 7, GATE, 1, F16T>(p, g, unit, kp, col, lds);
+            else
+                tile<BITS, 8, GATE, 1, F16T>(p, g, unit, kp, col, lds);
+        }
+    } else {
+        if (g.ct == 1)
+            tile<BITS, 1, GATE, 2, F16T>(p, g, unit, kp, col, lds);
+        else
+            tile<BITS, 2, GATE, 2, F16T>(p, g, unit, kp, col, lds);
+    }
+}
+
+template <int BITS>
+void launch(const Params &p, bool gate, bool wide, bool f16_tables, unsigned blocks, hipStream_t s)
+{
+    const dim3 block(kBlockWaves * 64);
+#define HQQ_ROWS(G, W, T) rows_tile_kernel<BITS, G, W, T><<<blocks, block, 0, s>>>(p)
+    if (gate)
+        wide ? (f16_tables ? HQQ_ROWS(true, true, true) : HQQ_ROWS(true, true, false))
+             : (f16_tables ? HQQ_ROWS(true, false, true) : HQQ_ROWS(true, false, false));
+    else
+        wide ? (f16_tables ? HQQ_ROWS(false, true, true) : HQQ_ROWS(false, true, false))
+             : (f16_tables ? HQQ_ROWS(false, false, true) : HQQ_ROWS(false, false, false));
+#undef HQQ_ROWS
+}
+
+} // namespace
+} // namespace rows
+} // namespace hqq

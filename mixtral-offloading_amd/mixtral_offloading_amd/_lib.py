@@ -59,6 +59,9 @@ _SIGNATURES = {
     "hqq_expert_groups_ffn_workspace_bytes": (c_size_t, [c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
     "hqq_expert_groups_ffn": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                       c_size_t, c_void_p]),
+    "hqq_expert_rows_ffn_workspace_bytes": (c_size_t, [c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
+    "hqq_expert_rows_ffn": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                    c_size_t, c_void_p]),
     "hqq_moe_group_pairs_rows": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "hqq_moe_combine": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p]),
     "hqq_moe_group_pairs": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),

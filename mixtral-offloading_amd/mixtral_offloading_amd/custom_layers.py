@@ -249,18 +249,23 @@ class SparseMoeWrapper(nn.Module):
         self.gate = gate
         self.experts = expert_cache
 
+    @staticmethod
+    def _expert_descs(module):
+        """The descriptors (w1, w2, w3) of an expert that the library's fused calls take, else None."""
+        ffn = module._expert[0] if hasattr(module, "_expert") else module
+        if getattr(ffn, "hidden_act", "silu") != "silu" or not all(hasattr(ffn, n) for n in ("w1", "w2", "w3")):
+            return None
+        return ffn.w1._desc(), ffn.w2._desc(), ffn.w3._desc()
+
     def _resident_group(self):
         """The layer's experts as ``hip_kernels.ExpertGroup`` when all of them are resident and none can be evicted
         (their device modules then never move), else None."""
         modules = self.experts.resident_group(self.layer_id) if hasattr(self.experts, "resident_group") else None
         if modules is None or len(modules) != self.num_experts:
             return None
-        layers = []
-        for m in modules:
-            ffn = m._expert[0] if hasattr(m, "_expert") else m
-            if getattr(ffn, "hidden_act", "silu") != "silu" or not all(hasattr(ffn, n) for n in ("w1", "w2", "w3")):
-                return None
-            layers.append((ffn.w1._desc(), ffn.w2._desc(), ffn.w3._desc()))
+        layers = [self._expert_descs(m) for m in modules]
+        if None in layers:
+            return None
         key = tuple(id(d) for t in layers for d in t)
         if getattr(self, "_group_cache", None) is None or self._group_cache[0] != key:
             self._group_cache = (key, hip_kernels.ExpertGroup(layers))
@@ -313,13 +318,18 @@ class SparseMoeWrapper(nn.Module):
             starts = np.concatenate(([0], np.cumsum(counts)))
             if group is not None:
                 # every expert of the layer is resident for good: all of them from one library call
-                hip_kernels.expert_groups_ffn(group, gathered, starts, scales, weighted)
+                hip_kernels.expert_rows_ffn(group, gathered, starts, scales, weighted)
             else:
                 active_experts = [e for e in range(self.num_experts) if counts[e] > 0]
                 for (_layer_index, expert_idx), expert_layer in self.experts.load_experts(
                         *((self.layer_id, expert_idx) for expert_idx in active_experts), unordered=True):
-                    lo, hi = int(starts[expert_idx]), int(starts[expert_idx + 1])
-                    expert_layer(gathered[lo:hi], out=weighted[lo:hi], row_scale=scales[lo:hi])
+                    one = self._expert_descs(expert_layer)
+                    if one is not None:  # planned with the other experts' rows: the same bits as all of them at once
+                        only = [one if e == expert_idx else None for e in range(self.num_experts)]
+                        hip_kernels.expert_rows_ffn(hip_kernels.ExpertGroup(only), gathered, starts, scales, weighted)
+                    else:
+                        lo, hi = int(starts[expert_idx]), int(starts[expert_idx + 1])
+                        expert_layer(gathered[lo:hi], out=weighted[lo:hi], row_scale=scales[lo:hi])
             combined = hip_kernels.moe_combine(weighted, row_of_pair)
             return combined.reshape(batch_size, sequence_length, hidden_dim), router_logits
         final_hidden_states = torch.zeros((tokens, hidden_dim), dtype=hidden_states.dtype, device=hidden_states.device)

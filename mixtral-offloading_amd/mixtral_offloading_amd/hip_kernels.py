@@ -221,24 +221,22 @@ def expert_ffn(w1: LinearDesc, w2: LinearDesc, w3: LinearDesc, x: torch.Tensor, 
 
 
 class ExpertGroup:
-    """The layers of a MoE layer's experts as the pointer arrays ``expert_groups_ffn`` takes (built once per layer;
-    the descriptors are kept alive here)."""
+    """The layers of a MoE layer's experts as the pointer arrays ``expert_groups_ffn`` and ``expert_rows_ffn`` take (built
+    once per layer; the descriptors are kept alive here).  For ``expert_rows_ffn`` an expert may be None: its rows are left
+    alone."""
 
     def __init__(self, experts):
-        self.descs = [tuple(e) for e in experts]  # (w1, w2, w3) LinearDesc per expert
+        self.descs = [None if e is None else tuple(e) for e in experts]  # (w1, w2, w3) LinearDesc per expert
         n = len(self.descs)
         arr = ctypes.c_void_p * n
-        self.w1 = arr(*[ctypes.addressof(d[0].c) for d in self.descs])
-        self.w2 = arr(*[ctypes.addressof(d[1].c) for d in self.descs])
-        self.w3 = arr(*[ctypes.addressof(d[2].c) for d in self.descs])
+        self.w1, self.w2, self.w3 = (arr(*[None if d is None else ctypes.addressof(d[i].c) for d in self.descs]) for i in range(3))
         self.n = n
-        self.K, self.N = self.descs[0][0].K, self.descs[0][1].N
+        first = next(d for d in self.descs if d is not None)
+        self.K, self.N = first[0].K, first[1].N
 
 
-def expert_groups_ffn(group: ExpertGroup, x: torch.Tensor, row_start, row_scale: Optional[torch.Tensor],
-                      out: torch.Tensor) -> torch.Tensor:
-    """Rows ``row_start[g] .. row_start[g + 1] - 1`` of ``x`` through expert ``g``, scaled per row, into ``out``: the
-    expert loop of the reference's ``SparseMoeWrapper.forward`` (src/custom_layers.py:298-312) as one library call."""
+def _run_groups(entry: str, group: ExpertGroup, x: torch.Tensor, row_start, row_scale: Optional[torch.Tensor],
+                out: torch.Tensor) -> torch.Tensor:
     assert x.dtype == torch.float16 and x.is_contiguous() and x.shape[-1] == group.K
     rows = x.numel() // group.K
     assert out.dtype == torch.float16 and out.is_contiguous() and out.numel() == rows * group.N
@@ -246,15 +244,29 @@ def expert_groups_ffn(group: ExpertGroup, x: torch.Tensor, row_start, row_scale:
     assert row_scale is None or (row_scale.dtype == torch.float16 and row_scale.is_contiguous() and row_scale.numel() == rows)
     starts = (ctypes.c_int64 * (group.n + 1))(*[int(v) for v in row_start])
     with _on(x.device):
-        need = _lib.lib.hqq_expert_groups_ffn_workspace_bytes(group.w1, group.w2, group.w3, group.n, starts)
+        need = getattr(_lib.lib, entry + "_workspace_bytes")(group.w1, group.w2, group.w3, group.n, starts)
         if rows and need == 0:
-            raise _lib.HqqError(-6, "hqq_expert_groups_ffn_workspace_bytes")
+            raise _lib.HqqError(-6, entry + "_workspace_bytes")
         ws = workspace(x.device, max(need, 1))
-        _lib.check(_lib.lib.hqq_expert_groups_ffn(group.w1, group.w2, group.w3, group.n, starts, x.data_ptr(), out.data_ptr(),
-                                                  row_scale.data_ptr() if row_scale is not None else None,
-                                                  ws.data_ptr(), ws.numel(), _lib.current_stream_ptr(x.device)),
-                   "hqq_expert_groups_ffn")
+        _lib.check(getattr(_lib.lib, entry)(group.w1, group.w2, group.w3, group.n, starts, x.data_ptr(), out.data_ptr(),
+                                            row_scale.data_ptr() if row_scale is not None else None,
+                                            ws.data_ptr(), ws.numel(), _lib.current_stream_ptr(x.device)), entry)
     return out
+
+
+def expert_groups_ffn(group: ExpertGroup, x: torch.Tensor, row_start, row_scale: Optional[torch.Tensor],
+                      out: torch.Tensor) -> torch.Tensor:
+    """Rows ``row_start[g] .. row_start[g + 1] - 1`` of ``x`` through expert ``g``, scaled per row, into ``out``: the
+    expert loop of the reference's ``SparseMoeWrapper.forward`` (src/custom_layers.py:298-312) as one library call, bit for
+    bit one ``expert_ffn`` per expert."""
+    return _run_groups("hqq_expert_groups_ffn", group, x, row_start, row_scale, out)
+
+
+def expert_rows_ffn(group: ExpertGroup, x: torch.Tensor, row_start, row_scale: Optional[torch.Tensor],
+                    out: torch.Tensor) -> torch.Tensor:
+    """The same loop with all gates in one launch and all down projections in another.  A row's result depends on the
+    groups' sizes, not on which of the experts ``group`` holds."""
+    return _run_groups("hqq_expert_rows_ffn", group, x, row_start, row_scale, out)
 
 
 STATIC_SCRATCH_BYTES = 16 << 20  # HQQ_STATIC_SCRATCH_BYTES of include/hqq_mi355x.h
