@@ -142,7 +142,7 @@ int hqq_expert_groups_ffn(const hqq_linear *const *w1, const hqq_linear *const *
  *      finishing pass where K is split), whatever the groups' sizes.  A group whose layers are all NULL is left out of
  *      the launches, and its rows of y alone, but the K split is planned for all rows: a row's result does not depend
  *      on which groups come in the same call.  Results are hqq_expert_ffn's to rounding.  Layers of different shapes,
- *      shapes that the kernel does not take (3-bit codes among them) and plans of too few blocks to fill the chip run
+ *      shapes that the kernel does not take and plans of too few blocks to fill the chip run
  *      as hqq_expert_groups_ffn, the groups that are there.                                                        */
 size_t hqq_expert_rows_ffn_workspace_bytes(const hqq_linear *const *w1, const hqq_linear *const *w2,
                                            const hqq_linear *const *w3, int32_t n_groups, const int64_t *row_start);

@@ -260,7 +260,7 @@ static bool ffn_runs_rows_kernel(const hqq_linear *w1, const hqq_linear *w2, con
 
 static TileFinish rows_finish(const RowsItem &it, int kpb)
 {
-    return TileFinish{it.part, kpb, (int)it.M, (int)it.l0->N, 8 / it.l0->nbits, static_cast<const f16 *>(it.l0->bias), it.y,
+    return TileFinish{it.part, kpb, (int)it.M, (int)it.l0->N, rows_outputs_together(it.l0), static_cast<const f16 *>(it.l0->bias), it.y,
                       it.row_scale, it.accumulate};
 }
 
@@ -271,7 +271,7 @@ static size_t ffn_gate_scratch(const hqq_linear *w1, const hqq_linear *w2, const
 {
     const size_t mm = ffn_matmul_scratch(w1, w2, w3, M);
     const size_t g = lds_gate_preferred(w1, w3, M) ? align256(ldsgemm_gate_workspace_bytes(w1, w3, M)) : 0;
-    const size_t r = ffn_runs_rows_kernel(w1, w2, w3, M) ? workspace_head_bytes() + rows_partial_bytes(w2, M, rows_k_blocks(w2, M, rows_blocks(w2, M, false))) : 0;
+    const size_t r = ffn_runs_rows_kernel(w1, w2, w3, M) ? workspace_head_bytes() + rows_partial_bytes(w2, M, rows_k_blocks(w2, rows_blocks(w2, M, false), M > 32)) : 0;
     const size_t most = g > r ? g : r;
     return most > mm ? most : mm;
 }
@@ -405,7 +405,7 @@ static int expert_ffn_impl(const hqq_linear *w1, const hqq_linear *w2, const hqq
 
     // 17 rows and more: both gate projections in one launch, silu(a) * b in its blocks, then the down projection
     if (ffn_runs_rows_kernel(w1, w2, w3, M) && aligned16(x)) {
-        const int kpb = rows_k_blocks(w2, M, rows_blocks(w2, M, false));
+        const int kpb = rows_k_blocks(w2, rows_blocks(w2, M, false), M > 32);
         const size_t bytes = rows_partial_bytes(w2, M, kpb);
         if (workspace_bytes >= ffn_gate_scratch(w1, w2, w3, M) + rows_bytes) // else the kernels that need no more than the least
             mm_bytes = ffn_gate_scratch(w1, w2, w3, M), h = (f16 *)(p + mm_bytes);
@@ -663,17 +663,20 @@ static const hqq_linear *const *expert_rows_lead(const hqq_linear *const *w1, co
             blocks += rows_blocks(w1[lead - w2], row_start[g + 1] - row_start[g], true);
             wide = wide || row_start[g + 1] - row_start[g] > 32;
         }
-    return blocks >= (wide ? 160 : 512) ? lead : nullptr;
+    return blocks >= (wide || (*lead)->nbits == 3 ? 160 : 512) ? lead : nullptr;
 }
 
-// blocks of all groups' down projections, K not split
-static int64_t expert_rows_blocks(const hqq_linear *w2, int32_t n_groups, const int64_t *row_start)
+// blocks along K of the groups' down projections
+static int expert_rows_k_blocks(const hqq_linear *w2, int32_t n_groups, const int64_t *row_start)
 {
     int64_t blocks = 0;
+    bool wide = false;
     for (int g = 0; g < n_groups; ++g)
-        if (row_start[g + 1] > row_start[g])
+        if (row_start[g + 1] > row_start[g]) {
             blocks += rows_blocks(w2, row_start[g + 1] - row_start[g], false);
-    return blocks;
+            wide = wide || row_start[g + 1] - row_start[g] > 32;
+        }
+    return rows_k_blocks(w2, blocks, wide);
 }
 
 // whether every group that has rows has layers
@@ -707,12 +710,12 @@ size_t hqq_expert_rows_ffn_workspace_bytes(const hqq_linear *const *w1, const hq
     if (!lead)
         return expert_rows_all(w1, w2, w3, n_groups, row_start) ? hqq_expert_groups_ffn_workspace_bytes(w1, w2, w3, n_groups, row_start)
                                                                 : expert_rows_apart_bytes(w1, w2, w3, n_groups, row_start);
-    const int64_t blocks = expert_rows_blocks(*lead, n_groups, row_start);
+    const int kb = expert_rows_k_blocks(*lead, n_groups, row_start);
     size_t need = workspace_head_bytes();
     for (int g = 0; g < n_groups; ++g) {
         const int64_t M = row_start[g + 1] - row_start[g];
         if (M > 0 && w1[g])
-            need += align256((size_t)M * (size_t)w1[g]->N * sizeof(f16)) + rows_partial_bytes(w2[g], M, rows_k_blocks(w2[g], M, blocks));
+            need += align256((size_t)M * (size_t)w1[g]->N * sizeof(f16)) + rows_partial_bytes(w2[g], M, kb);
     }
     return need;
 }
@@ -753,7 +756,7 @@ int hqq_expert_rows_ffn(const hqq_linear *const *w1, const hqq_linear *const *w2
         workspace_bytes < hqq_expert_rows_ffn_workspace_bytes(w1, w2, w3, n_groups, row_start))
         return HQQ_E_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
-    const int64_t blocks = expert_rows_blocks(*lead, n_groups, row_start);
+    const int kb = expert_rows_k_blocks(*lead, n_groups, row_start);
     char *at = static_cast<char *>(workspace) + workspace_head_bytes(); // the head holds other kernels' counters
     RowsItem gate[kTileFinishGroupMax], down[kTileFinishGroupMax];
     TileFinish fin[kTileFinishGroupMax];
@@ -776,7 +779,7 @@ int hqq_expert_rows_ffn(const hqq_linear *const *w1, const hqq_linear *const *w2
             return rc;
         f16 *h = reinterpret_cast<f16 *>(at);
         at += align256((size_t)M * (size_t)w1[g]->N * sizeof(f16));
-        kpb[n] = rows_k_blocks(w2[g], M, blocks);
+        kpb[n] = kb;
         const size_t bytes = rows_partial_bytes(w2[g], M, kpb[n]);
         gate[n] = RowsItem{w1[g], w3[g], static_cast<const f16 *>(x_f16) + lo * w1[g]->K, M, h, nullptr, nullptr, 0};
         down[n] = RowsItem{w2[g], nullptr, h, M, static_cast<f16 *>(y_f16) + lo * w2[g]->N, bytes ? reinterpret_cast<float *>(at) : nullptr,

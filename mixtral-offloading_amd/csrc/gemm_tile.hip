@@ -685,7 +685,7 @@ __device__ __forceinline__ void tile_finish_block(const float *__restrict__ part
                                                   const f16 *__restrict__ row_scale, int accumulate)
 {
     __shared__ f16 t_lds[16][16][F];
-    const int NG = N / F;
+    const int NG = (N + F - 1) / F; // (3-bit codes: the last group may be short)
     const int g0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
     {
         const int m = m0 + (threadIdx.x & 15), gl = threadIdx.x >> 4, g = g0 + gl;
@@ -709,7 +709,7 @@ __device__ __forceinline__ void tile_finish_block(const float *__restrict__ part
                 if constexpr (GATE) {
                     const float u = (float)v;
                     v = (f16)(u / (1.0f + __expf(-u))) * (f16)b[i];
-                } else if (bias) {
+                } else if (bias && (F != 10 || F * g + i < N)) {
                     v = v + bias[F * g + i];
                 }
                 if (row_scale)
@@ -725,7 +725,8 @@ __device__ __forceinline__ void tile_finish_block(const float *__restrict__ part
             f16 *dst = y + (int64_t)m * N + F * g;
 #pragma unroll
             for (int i = 0; i < F; ++i)
-                dst[i] = accumulate ? (f16)(dst[i] + t_lds[threadIdx.x >> 4][gl][i]) : t_lds[threadIdx.x >> 4][gl][i];
+                if (F != 10 || F * g + i < N)
+                    dst[i] = accumulate ? (f16)(dst[i] + t_lds[threadIdx.x >> 4][gl][i]) : t_lds[threadIdx.x >> 4][gl][i];
         }
     }
 }
@@ -747,7 +748,7 @@ struct TileFinishGroup {
 template <int F> __global__ __launch_bounds__(256) void tile_finish_group_kernel(TileFinishGroup g)
 {
     const TileFinish &d = g.f[blockIdx.z];
-    if ((int)blockIdx.x * 16 >= d.N / F || (int)blockIdx.y * 16 >= d.M)
+    if ((int)blockIdx.x * 16 >= (d.N + F - 1) / F || (int)blockIdx.y * 16 >= d.M)
         return;
     tile_finish_block<F, false>(d.part, d.KSP, d.M, d.N, d.bias, d.y, 0, d.row_scale, d.accumulate);
 
@@ -1075,7 +1076,7 @@ int launch_tile_matmul_deferred(const hqq_linear *l, const f16 *x, int64_t M, f1
 // the finishing passes of up to kTileFinishGroupMax deferred launches in one launch per code width
 int launch_tile_finish_group(const TileFinish *f, int n, hipStream_t s)
 {
-    for (int F = 2; F <= 4; F += 2) {
+    for (const int F : {2, 4, 10}) {
         TileFinishGroup g = {};
         int cnt = 0, gx = 0, gy = 0;
         for (int i = 0; i < n; ++i) {
@@ -1084,7 +1085,7 @@ int launch_tile_finish_group(const TileFinish *f, int n, hipStream_t s)
             if (cnt == kTileFinishGroupMax)
                 return HQQ_E_UNSUPPORTED;
             g.f[cnt++] = f[i];
-            const int x = (f[i].N / F + 15) / 16, y = (f[i].M + 15) / 16;
+            const int x = ((f[i].N + F - 1) / F + 15) / 16, y = (f[i].M + 15) / 16;
             gx = x > gx ? x : gx, gy = y > gy ? y : gy;
         }
         if (!cnt)
@@ -1092,6 +1093,8 @@ int launch_tile_finish_group(const TileFinish *f, int n, hipStream_t s)
         const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)cnt);
         if (F == 4)
             tile_finish_group_kernel<4><<<grid, 256, 0, s>>>(g);
+        else if (F == 10)
+            tile_finish_group_kernel<10><<<grid, 256, 0, s>>>(g);
         else
             tile_finish_group_kernel<2><<<grid, 256, 0, s>>>(g);
         const int rc = launch_status();

@@ -304,7 +304,8 @@ struct RowsItem {
 bool rows_supported(const hqq_linear *l, int64_t M);
 bool rows_alike(const hqq_linear *a, const hqq_linear *b);
 int64_t rows_blocks(const hqq_linear *l, int64_t M, bool gate); // of a launch whose K is not split
-int rows_k_blocks(const hqq_linear *l, int64_t M, int64_t blocks); // blocks: of all members of the launch
+int rows_k_blocks(const hqq_linear *l, int64_t blocks, bool wide); // blocks: of all members; wide: one has more than 32 rows
+int rows_outputs_together(const hqq_linear *l);                    // F of a finishing pass
 size_t rows_partial_bytes(const hqq_linear *l, int64_t M, int kpb);
 int launch_rows(const RowsItem *item, const int *kpb, int n, bool gate, hipStream_t s);
 // dequant_gemm.hip: wide batches as hqq_dequantize into the workspace + one library GEMM

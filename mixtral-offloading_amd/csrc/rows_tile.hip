@@ -4,16 +4,16 @@
 #include "gemv_parts.hpp"
 
 #include <algorithm>
+#include <numeric>
 
 namespace hqq {
 using namespace rows;
 
 namespace {
 
-constexpr int64_t kFixedSplitRows = 64;
-
 struct Shape {
     int F, GP, RBU, steps;
+    int words, G, dstep, inv; // 3-bit codes
     bool f16_tables;
 };
 
@@ -21,16 +21,27 @@ bool ptr_aligned(const void *p, unsigned n) { return (reinterpret_cast<uintptr_t
 
 bool shape_of(const hqq_linear *l, Shape &sh)
 {
-    if (l->nbits != 2 && l->nbits != 4)
+    const int64_t G = l->N / l->group_size;
+    sh = Shape{};
+    if (l->K % kStep != 0 || G * l->K >= (1ll << 31) || l->K >= (1 << 24) || l->N >= (1ll << 30) || !ptr_aligned(l->codes, 16))
         return false;
-    sh.F = 8 / l->nbits;
-    const int64_t G = l->N / l->group_size, rbw = 4 / sh.F;
-    if (l->group_size % (16 * rbw) != 0 || G % sh.F != 0 || l->K % kStep != 0 || l->N / l->group_size * l->K >= (1ll << 31) ||
-        l->N / sh.F * l->K >= (1ll << 32) || l->K >= (1 << 24)) // 32-bit offsets within a layer
-        return false;
-    sh.GP = (int)(G / sh.F), sh.RBU = (int)(l->group_size / (16 * rbw)), sh.steps = (int)(l->K / kStep);
-    if (!ptr_aligned(l->codes, 16))
-        return false;
+    sh.steps = (int)(l->K / kStep);
+    if (l->nbits == 3) {
+        const int64_t d = std::gcd((int64_t)10, G), P = G / d, words = (l->N + 9) / 10;
+        // table rows of a block: at most 24, once round G at most; a window: at most sixteen word rows
+        if (d > kMaxStep3 || G < 10 + kMaxStep3 * (kBlockWaves - 1) || (words + P - 1) / P > 16 || l->N % 2 != 0 ||
+            words * l->K * 4 >= (1ll << 32) || P >= (1 << 15))
+            return false;
+        sh.F = 10, sh.GP = (int)P, sh.RBU = 1, sh.words = (int)words, sh.G = (int)G, sh.dstep = (int)d;
+        while (sh.inv < P && 10 / d * sh.inv % P != 1 % P)
+            ++sh.inv;
+    } else {
+        sh.F = 8 / l->nbits;
+        const int64_t rbw = 4 / sh.F;
+        if (l->group_size % (16 * rbw) != 0 || G % sh.F != 0 || l->N / sh.F * l->K >= (1ll << 32)) // 32-bit offsets within a layer
+            return false;
+        sh.GP = (int)(G / sh.F), sh.RBU = (int)(l->group_size / (16 * rbw));
+    }
     const int sk = gemv::table_kind(l->scale), zk = gemv::table_kind(l->zero);
     sh.f16_tables = sk == gemv::TK_F16 && zk == gemv::TK_F16;
     if (sh.f16_tables)
@@ -42,18 +53,19 @@ bool shape_of(const hqq_linear *l, Shape &sh)
 
 // How M rows are cut: ncol blocks of ct tiles of sixteen rows, as even as they come
 struct Cut {
-    int ct, ncol, kw;
+    int ct, ncol;
+    int share; // waves of a block that work on the same output rows (of one projection)
 };
 Cut cut_rows(int nbits, int64_t M)
 {
     const int tiles = (int)((M + 15) / 16), most = max_tiles(nbits), n = (tiles + most - 1) / most;
     Cut c;
-    c.ct = (tiles + n - 1) / n, c.ncol = (tiles + c.ct - 1) / c.ct, c.kw = c.ct <= kHalvesTiles ? 2 : 1;
+    c.ct = (tiles + n - 1) / n, c.ncol = (tiles + c.ct - 1) / c.ct, c.share = (nbits == 3 ? c.ct > kHalfFields3 : c.ct <= kHalvesTiles) ? 2 : 1;
     return c;
 }
 int units(const Shape &sh, const Cut &c, bool gate)
 {
-    const int jw = kBlockWaves / c.kw / (gate ? 2 : 1);
+    const int jw = kBlockWaves / c.share / (gate ? 2 : 1);
     return (sh.GP + jw - 1) / jw * sh.RBU;
 }
 
@@ -80,30 +92,29 @@ int64_t rows_blocks(const hqq_linear *l, int64_t M, bool gate)
     return (int64_t)units(sh, c, gate) * c.ncol;
 }
 
-int rows_k_blocks(const hqq_linear *l, int64_t M, int64_t blocks)
+int rows_outputs_together(const hqq_linear *l) { return l->nbits == 3 ? 10 : 8 / l->nbits; }
+
+int rows_k_blocks(const hqq_linear *l, int64_t blocks, bool wide)
 {
     Shape sh;
     if (!shape_of(l, sh))
         return 1;
-    const auto whole = [&](int k) { // blocks of equal length, none of them empty
-        const int spp = (sh.steps + k - 1) / k;
-        return (sh.steps + spp - 1) / spp;
-    };
-    if (M <= kFixedSplitRows)
-        return whole(std::min(8, std::max(1, sh.steps / 28)));
+    const int64_t slots = wide || l->nbits == 3 ? 256 : 512; // blocks that run at a time
     int best = 1;
     int64_t cost = -1;
-    for (int k = 1; k <= 8 && sh.steps / k >= 4; ++k) {
-        const int64_t c = (blocks * k + 255) / 256 * ((sh.steps + k - 1) / k + 4) + (k > 1 ? 4 + k : 0);
+    for (int k = 1; k <= 8 && sh.steps / k >= 4; ++k) { // in steps of a block; 4: its first loads and its end
+        const int64_t c = (blocks * k + slots - 1) / slots * ((sh.steps + k - 1) / k + 4) + (k > 1 ? 4 + k : 0);
         if (cost < 0 || c < cost)
             best = k, cost = c;
     }
-    return whole(tuning_int("HQQ_ROWS_KPB", best));
+    const int spp = (sh.steps + best - 1) / best; // parts of equal length, none of them empty
+    return (sh.steps + spp - 1) / spp;
 }
 
 size_t rows_partial_bytes(const hqq_linear *l, int64_t M, int kpb)
 {
-    return kpb > 1 ? ((size_t)kpb * (size_t)M * (size_t)l->N * sizeof(float) + 255) & ~(size_t)255 : 0;
+    const int64_t F = rows_outputs_together(l), N = (l->N + F - 1) / F * F;
+    return kpb > 1 ? ((size_t)kpb * (size_t)M * (size_t)N * sizeof(float) + 255) & ~(size_t)255 : 0;
 }
 
 int launch_rows(const RowsItem *item, const int *kpb, int n, bool gate, hipStream_t s)
@@ -121,6 +132,7 @@ int launch_rows(const RowsItem *item, const int *kpb, int n, bool gate, hipStrea
             return HQQ_E_UNSUPPORTED;
         Params p = {};
         p.N = (int)l->N, p.K = (int)l->K, p.GP = sh.GP, p.RBU = sh.RBU, p.steps = sh.steps;
+        p.words = sh.words, p.G = sh.G, p.dstep = sh.dstep, p.inv = sh.inv;
         p.s_cols = (uint32_t)l->scale.meta_cols;
         p.s_inv = p.s_cols ? (uint32_t)(0xFFFFFFFFull / p.s_cols) : 0;
         int64_t slots = 0;
@@ -152,6 +164,8 @@ int launch_rows(const RowsItem *item, const int *kpb, int n, bool gate, hipStrea
             return HQQ_E_UNSUPPORTED;
         if (l->nbits == 2)
             launch_w2(p, gate, wide, sh.f16_tables, (unsigned)(slots * 8), s);
+        else if (l->nbits == 3)
+            launch_w3(p, gate, wide, sh.f16_tables, (unsigned)(slots * 8), s);
         else
             launch_w4(p, gate, wide, sh.f16_tables, (unsigned)(slots * 8), s);
         const int rc = launch_status();

@@ -11,6 +11,8 @@ constexpr int kBlockWaves = 8;
 constexpr int kMembers = 12;   // layers (gates: pairs of layers) of a launch: their records travel in the kernel arguments
 // 16-row tiles of a block: what the accumulators leave registers for (4-bit codes: two row blocks' codes in flight)
 constexpr int max_tiles(int nbits) { return nbits == 2 ? 8 : 6; }
+constexpr int kHalfFields3 = 3; // 3-bit codes: with more tiles two waves share a window's ten fields
+constexpr int kMaxStep3 = 2; // 3-bit codes: table rows from one window to the next, at most
 // up to so many tiles the waves of a block split its columns in two halves
 constexpr int kHalvesTiles = 4;
 
@@ -36,7 +38,8 @@ struct Member {
 
 struct Params {
     int n;
-    int N, K, GP, RBU; // GP: packed rows that share nothing, RBU: row blocks of one packed row
+    int N, K, GP, RBU; // GP: packed rows that share no table rows (3-bit: windows), RBU: row blocks of one packed row
+    int words, G, dstep, inv; // 3-bit: word rows, table rows, table rows from window to window, window (idx * inv) mod GP is idx-th
     int steps;
     uint32_t s_cols, s_inv; // meta columns of the scale tables, floor(2^32 / columns)
     Member m[kMembers];
@@ -44,6 +47,7 @@ struct Params {
 
 // kernels of one code width (a translation unit each); wide: some member has more than 32 rows
 void launch_w2(const Params &p, bool gate, bool wide, bool f16_tables, unsigned blocks, hipStream_t s);
+void launch_w3(const Params &p, bool gate, bool wide, bool f16_tables, unsigned blocks, hipStream_t s);
 void launch_w4(const Params &p, bool gate, bool wide, bool f16_tables, unsigned blocks, hipStream_t s);
 
 } // namespace rows

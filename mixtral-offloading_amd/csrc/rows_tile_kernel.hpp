@@ -19,30 +19,13 @@
 //     1376 -> 1332.
 #pragma once
 
-#include "gemv_parts.hpp"
-#include "rows_tile.hpp"
+#include "rows_tile_parts.hpp"
 
 namespace hqq {
 namespace rows {
 namespace {
 
 using gemv::gload;
-// The arguments stay where the launch put them: read through a pointer to them, not copied to be indexed.
-#define HQQ_KERNARG __attribute__((address_space(4)))
-#define HQQ_LDS __attribute__((address_space(3)))
-
-// A load from a base that is the same for the whole wave and a 32-bit byte offset of the lane
-template <typename T> __device__ __forceinline__ T load_at(const void *base, uint32_t offset)
-{
-    return *(const T __attribute__((address_space(1))) *)((const char __attribute__((address_space(1))) *)base + offset);
-}
-
-__device__ __forceinline__ float uniform(float v)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
-}
-
-constexpr int kWaitLoads = 0x0F70; // vmcnt(0), the other counters left alone
 
 template <int BITS> struct Codes {
     static constexpr int F = 8 / BITS;       // output rows per packed row
@@ -53,9 +36,6 @@ template <int BITS> struct Codes {
     // a field masked in place and OR-ed into the mantissa of 2^(10 - pos) reads as 2^(10 - pos) + code
     static constexpr uint32_t expo(int f) { return (uint32_t)((10 - pos(f) + 15) << 10) * 0x00010001u; }
 };
-
-__device__ __forceinline__ f16x2 h2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
-__device__ __forceinline__ uint32_t u2(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
 
 template <int BITS, int CT, bool GATE, int KW, bool F16T>
 __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member HQQ_KERNARG &g, int unit, int kp, int col, char *lds)
@@ -102,12 +82,8 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
         zneg = uniform(-(float)gload<f16>(g.l[proj].z_ms));
         zoff = uniform(-(float)gload<f16>(g.l[proj].z_mz) * zneg);
         const uint32_t c = trow + (uint32_t)s0 * kStep;
-        cm0 = c - __umulhi(c, p.s_inv) * p.s_cols; // c mod columns: the quotient estimate is at most 2 short
-        cm0 -= cm0 >= p.s_cols ? p.s_cols : 0;
-        cm0 -= cm0 >= p.s_cols ? p.s_cols : 0;
+        cm0 = mod_cols(c, p.s_cols, p.s_inv);
     }
-    // The x tile goes to LDS without passing the registers, sixteen bytes a lane in operand order.  (By hand: the compiler
-    // would wait for the transfer before the next LDS read, whichever half of the buffer that reads.)
     const f16 *xb = g.x + (size_t)m0 * K + (size_t)s0 * kStep;
     uint32_t xo[XCH], xd[XCH]; // byte offsets: a lane's in x, the wave's in LDS
 #pragma unroll
@@ -137,18 +113,14 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
         const f16 *const xs = xb + (size_t)st * kStep;
 #pragma unroll
         for (int c = 0; c < XCH; ++c) // (past the end: the last operand once more, the same bytes to the same place)
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         : : "v"(xo[c]), "s"(xs), "s"(xd[c] + buf * (KW * XTILE)) : "memory");
+            load_to_lds(xo[c], xs, xd[c] + buf * (KW * XTILE));
         if constexpr (F16T) {
             r.a = load_at<Halves>(l_sq + 2 * (size_t)k0, 2 * trow);
             r.b = load_at<Halves>(l_zq + 2 * (size_t)k0, 2 * trow);
         } else {
             r.sq = load_at<Bytes>(l_sq + k0, trow);
             r.zq = load_at<Bytes>(l_zq + k0, trow);
-            uint32_t cm = cm0 + (uint32_t)st * kStep; // less than K + columns
-            cm -= __umulhi(cm, p.s_inv) * p.s_cols;
-            cm -= cm >= p.s_cols ? p.s_cols : 0;
-            cm -= cm >= p.s_cols ? p.s_cols : 0;
+            const uint32_t cm = mod_cols(cm0 + (uint32_t)st * kStep, p.s_cols, p.s_inv); // less than K + columns before
             r.a = load_at<Halves>(l_sms, 2 * cm);
             r.b = load_at<Halves>(l_smz, 2 * cm);
         }
@@ -161,29 +133,7 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
     char *const t_w = t_lds + wave * TTILE + (((((tk >> 6) * 2 + ((tk >> 3) & 1)) * F + ti) * 4 + ((tk >> 4) & 3)) * 32) + 2 * (tk & 7);
     auto stage = [&](const Next &r, int buf) __attribute__((always_inline)) {
         Halves S, Z;
-#pragma unroll
-        for (int e = 0; e < TE / 2; ++e) {
-            if constexpr (F16T) {
-                S[e] = r.a[e];
-                Z[e] = u2(-(h2(r.b[e]) * h2(r.a[e])));
-            } else {
-                f16x2 sv, zv;
-#pragma unroll
-                for (int o = 0; o < 2; ++o) {
-                    uint32_t sw, zw;
-                    if constexpr (TE == 8)
-                        sw = r.sq[e >> 1], zw = r.zq[e >> 1];
-                    else
-                        sw = r.sq[0], zw = r.zq[0];
-                    const int sh = 8 * ((2 * e + o) & 3);
-                    const float sc = (float)((sw >> sh) & 0xFFu), zc = (float)((zw >> sh) & 0xFFu);
-                    const float d = __builtin_fmaf((float)h2(r.b[e])[o], -1.0f, sc);
-                    sv[o] = (f16)__builtin_fmaf(d, (float)h2(r.a[e])[o], 0.0f);
-                    zv[o] = (f16)__builtin_fmaf(__builtin_fmaf(zc, zneg, zoff), (float)sv[o], 0.0f);
-                }
-                S[e] = u2(sv), Z[e] = u2(zv);
-            }
-        }
+        decode_tables<F16T, TE>(r.a, r.b, r.sq, r.zq, zneg, zoff, S, Z);
         char *const d = t_w + buf * (kBlockWaves * TTILE);
         *reinterpret_cast<Halves *>(d) = S;
         *reinterpret_cast<Halves *>(d + 16) = Z;
@@ -240,11 +190,16 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
                         P[t] = __builtin_amdgcn_perm(0u, cw[w][q >> 1][2 * (q & 1) + (t >> 1)], t & 1 ? 0x0c030c02u : 0x0c010c00u);
                 const f16 offv = (f16)(float)(1 << (10 - C::pos(f)));
                 const f16x2 off = {offv, offv};
+                f16x2 v[4]; // stage by stage: a packed instruction's result can be read by the next but one
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const f16x2 v = h2((P[t] & C::mask(f)) | expo[f]) - off; // the exact code
-                    A[gi & 1][t] = u2(__builtin_elementwise_fma(v, h2(S[h & 1][t]), h2(Z[h & 1][t])));
-                }
+                for (int t = 0; t < 4; ++t)
+                    v[t] = h2((P[t] & C::mask(f)) | expo[f]);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    v[t] = v[t] - off; // the exact code
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    A[gi & 1][t] = u2(__builtin_elementwise_fma(v[t], h2(S[h & 1][t]), h2(Z[h & 1][t])));
             };
             tables(0);
 #pragma unroll
@@ -426,17 +381,11 @@ __global__ __launch_bounds__(kBlockWaves * 64, WIDE ? 2 : 4) void rows_tile_kern
 {
     const Params HQQ_KERNARG &p = *(const Params HQQ_KERNARG *)__builtin_amdgcn_kernarg_segment_ptr();
     __shared__ __attribute__((aligned(16))) char lds[WIDE ? lds_bytes<BITS>(8, 1) : lds_bytes<BITS>(2, 2)];
-    // eight consecutive blocks run on eight dies: entry e of the list stands for a row block of each
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    int k = 0;
-    while (k + 1 < p.n && p.m[k + 1].first <= slot)
-        ++k;
-    const Member HQQ_KERNARG &g = p.m[k];
-    const int local = slot - g.first, rr = local / g.ncol, col = local - rr * g.ncol;
-    const int ru = rr * 8 + xcd;
-    if (ru >= g.units * g.kpb)
+    int unit, kp, col;
+    const Member HQQ_KERNARG *at = work_of(p, unit, kp, col);
+    if (!at)
         return;
-    const int kp = ru / g.units, unit = ru - kp * g.units;
+    const Member HQQ_KERNARG &g = *at;
     if constexpr (WIDE) {
         switch (g.ct) {
         case 1: return tile<BITS, 1, GATE, 2, F16T>(p, g, unit, kp, col, lds);

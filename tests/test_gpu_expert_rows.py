@@ -15,6 +15,7 @@ pytestmark = pytest.mark.gpu
 # 128 rows), enough groups for the common launches
 FEW = [1, 2, 15, 16, 17, 31, 32, 0, 3, 5, 8, 1, 30, 4, 18, 9, 2, 1, 16, 7, 11, 32]
 MANY = [33, 48, 49, 64, 65, 80, 96, 97, 112, 113, 128, 129, 1, 16, 0, 200]
+FEW3 = [1, 2, 15, 16, 17, 31, 32, 0] * 2 + [3, 5, 8, 1, 30, 4, 18, 9, 2, 1, 16, 7, 11, 32]  # (a block is four windows of 56)
 # (nbits, hidden, ffn, group size, 8-bit tables, rows of the groups)
 CASES = [
     (2, 1024, 3584, 16, True, FEW), (2, 1024, 3584, 16, True, MANY),
@@ -23,6 +24,10 @@ CASES = [
     (2, 896, 3840, 32, False, FEW), (2, 896, 3840, 32, False, MANY),  # fp16 tables, two row blocks of a packed row
     (4, 1024, 3584, 64, True, FEW), (4, 1024, 3584, 64, True, MANY),
     (4, 1152, 3712, 32, False, MANY),
+    # 3-bit: 28 windows of 13 word rows, the last of them with fields to spare (3584 rows are 358 words and four fields)
+    (3, 1536, 3584, 64, True, FEW3), (3, 1536, 3584, 64, True, MANY),
+    (3, 1536, 7552, 64, True, MANY),  # 59 windows (a block with some to spare), K split
+    (3, 3456, 3712, 128, False, MANY),  # fp16 tables, 27 and 29 windows one table row apart
 ]
 
 
