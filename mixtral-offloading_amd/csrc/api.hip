@@ -663,7 +663,7 @@ static const hqq_linear *const *expert_rows_lead(const hqq_linear *const *w1, co
             blocks += rows_blocks(w1[lead - w2], row_start[g + 1] - row_start[g], true);
             wide = wide || row_start[g + 1] - row_start[g] > 32;
         }
-    return blocks >= (wide || (*lead)->nbits == 3 ? 160 : 512) ? lead : nullptr;
+    return blocks >= (wide || (*lead)->nbits != 2 ? 160 : 512) ? lead : nullptr;
 }
 
 // blocks along K of the groups' down projections

@@ -99,7 +99,7 @@ int rows_k_blocks(const hqq_linear *l, int64_t blocks, bool wide)
     Shape sh;
     if (!shape_of(l, sh))
         return 1;
-    const int64_t slots = wide || l->nbits == 3 ? 256 : 512; // blocks that run at a time
+    const int64_t slots = wide || l->nbits != 2 ? 256 : 512; // blocks that run at a time
     int best = 1;
     int64_t cost = -1;
     for (int k = 1; k <= 8 && sh.steps / k >= 4; ++k) { // in steps of a block; 4: its first loads and its end

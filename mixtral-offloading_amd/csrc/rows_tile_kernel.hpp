@@ -44,10 +44,12 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
     constexpr int F = C::F, RBW = C::RBW, RT = C::RT;
     constexpr int NWK = kBlockWaves / KW;           // waves per K half
     constexpr int JW = NWK / (GATE ? 2 : 1);        // packed rows per block
-    constexpr int XTILE = 4 * CT * 64 * 16;         // bytes of one x tile: [q][row tile][lane] 16-byte operands
+    constexpr int XTILE = 2 * CT * 2048;            // bytes of one x tile: [64 columns][row tile][row] 128 bytes, see below
+    constexpr int CTILE = RBW * 2048;               // bytes of one wave's codes: [row block][row] 128 bytes
     constexpr int TTILE = 4 * F * 4 * 32;           // bytes of one wave's tables: [q][field][k group] 8 scales, 8 zeros
-    constexpr int XCH = (4 * CT + NWK - 1) / NWK;   // operands a lane stages per step
-    char *const x_lds = lds, *const t_lds = lds + 2 * KW * XTILE;
+    constexpr int XCH = (4 * CT + NWK - 1) / NWK;   // kilobytes of the x tile a wave brings in per step
+    char *const x_lds = lds, *const c_lds = lds + 2 * KW * XTILE + (threadIdx.x >> 6) * (2 * CTILE);
+    char *const t_lds = lds + 2 * KW * XTILE + kBlockWaves * 2 * CTILE + (threadIdx.x >> 6) * TTILE;
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kh = KW == 1 ? 0 : wave / NWK, wk = KW == 1 ? wave : wave % NWK;
@@ -68,10 +70,12 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
     const int mine = from >= b1 ? 0 : (b1 - from < nh ? b1 - from : nh); // steps of this wave's K half
     const int last = mine > 0 ? mine - 1 : 0;
 
-    uint32_t co[RBW];
-#pragma unroll
-    for (int w = 0; w < RBW; ++w)
-        co[w] = (uint32_t)(jp + (16 * (rbu * RBW + w) + rr) * p.GP) * (uint32_t)K + 16u * kg;
+    // Codes and x come in by eight lanes a row, 128 consecutive bytes (with a lane a row, as the matrix cores want them, the address
+    // unit took four times as long, and the waves waited to be let in), and lie in LDS as they come: sixteen-byte chunk c of row r at
+    // chunk c ^ (r / 2) % 8 of its row, so that the sixteen lanes of a read, a row each, fall into different banks.
+    const int r8 = lane >> 3, c8 = (lane & 7) ^ (r8 >> 1); // of the first eight rows of sixteen; of the other eight chunk c8 ^ 4
+    const uint32_t co = (uint32_t)(jp + (16 * rbu * RBW + r8) * p.GP) * (uint32_t)K + 16u * c8; // K is a multiple of 128
+    const uint32_t c_half = 8u * (uint32_t)p.GP * (uint32_t)K;                                  // from the first eight rows to the others
     // a lane de-quantises TE entries of one of the wave's table rows per step: columns tk .. tk + TE - 1 of row ti
     constexpr int TE = 2 * F;
     const int ti = lane / (kStep / TE), tk = TE * (lane % (kStep / TE));
@@ -84,36 +88,37 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
         const uint32_t c = trow + (uint32_t)s0 * kStep;
         cm0 = mod_cols(c, p.s_cols, p.s_inv);
     }
-    const f16 *xb = g.x + (size_t)m0 * K + (size_t)s0 * kStep;
+    // this wave's kilobytes of the x tile: 64 columns wk % 2, rows 8 * (wk / 2 % 2) .. + 7 of row tiles wk / 4, wk / 4 + NWK / 4 ...
+    const f16 *xb = g.x + (size_t)m0 * K + (size_t)s0 * kStep + 64 * (wk & 1);
     uint32_t xo[XCH], xd[XCH]; // byte offsets: a lane's in x, the wave's in LDS
 #pragma unroll
     for (int c = 0; c < XCH; ++c) {
-        int pi = wk + NWK * c;
-        pi = pi < 4 * CT ? pi : 4 * CT - 1;
-        const int q = pi & 3, b = pi >> 2;
-        const int m = m0 + 16 * b + rr < M ? 16 * b + rr : M - 1 - m0;
-        xo[c] = 2 * ((uint32_t)m * (uint32_t)K + 64 * (q >> 1) + 16 * kg + 8 * (q & 1));
-        xd[c] = (uint32_t)(uintptr_t)(HQQ_LDS char *)x_lds + kh * XTILE + (q * CT + b) * 1024;
+        int b = (wk >> 2) + NWK / 4 * c;
+        b = b < CT ? b : CT - 1; // (past the end: the last one once more, the same bytes to the same place)
+        const int hr = wk >> 1 & 1, m = m0 + 16 * b + 8 * hr + r8 < M ? 16 * b + 8 * hr + r8 : M - 1 - m0;
+        xo[c] = 2 * ((uint32_t)m * (uint32_t)K + 8 * (hr ? c8 ^ 4 : c8));
+        xd[c] = (uint32_t)(uintptr_t)(HQQ_LDS char *)x_lds + kh * XTILE + (((wk & 1) * CT + b) * 2 + hr) * 1024;
     }
+    const uint32_t cd = (uint32_t)(uintptr_t)(HQQ_LDS char *)c_lds;
 
-    // With two row blocks the codes of the next step are read into the registers of this one's as these fall free, a slab
-    // of 64 columns at a time; with one they have registers of their own and the whole step to arrive.
-    constexpr bool LATE = RBW == 2;
     typedef uint32_t Halves __attribute__((ext_vector_type(TE / 2)));
     typedef uint32_t Bytes __attribute__((ext_vector_type(TE / 4)));
     struct Next {
-        u32x4 cw[LATE ? 1 : RBW][2];
         Halves a, b; // meta of the scale / fp16 scales, fp16 zeros
         Bytes sq, zq;
     };
-    auto codes_at = [&](int w, uint32_t k) __attribute__((always_inline)) { return load_at<u32x4>(l_codes + k, co[w]); };
     auto issue = [&](Next &r, int it, int buf) __attribute__((always_inline)) {
         const int st = it < last ? it : last;
         const uint32_t k0 = (uint32_t)(s0 + st) * kStep;
         const f16 *const xs = xb + (size_t)st * kStep;
 #pragma unroll
-        for (int c = 0; c < XCH; ++c) // (past the end: the last operand once more, the same bytes to the same place)
+        for (int c = 0; c < XCH; ++c)
             load_to_lds(xo[c], xs, xd[c] + buf * (KW * XTILE));
+#pragma unroll
+        for (int w = 0; w < RBW; ++w)
+#pragma unroll
+            for (int o = 0; o < 2; ++o)
+                load_to_lds(o ? co ^ 64u : co, l_codes + k0 + (size_t)(2 * w + o) * c_half, cd + buf * CTILE + (2 * w + o) * 1024);
         if constexpr (F16T) {
             r.a = load_at<Halves>(l_sq + 2 * (size_t)k0, 2 * trow);
             r.b = load_at<Halves>(l_zq + 2 * (size_t)k0, 2 * trow);
@@ -124,19 +129,14 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
             r.a = load_at<Halves>(l_sms, 2 * cm);
             r.b = load_at<Halves>(l_smz, 2 * cm);
         }
-        if constexpr (!LATE) {
-            r.cw[0][0] = codes_at(0, k0);
-            r.cw[0][1] = codes_at(0, k0 + 64);
-        }
     };
     // where they go: slab tk / 64, k group (tk / 16) % 4, half (tk / 8) % 2
-    char *const t_w = t_lds + wave * TTILE + (((((tk >> 6) * 2 + ((tk >> 3) & 1)) * F + ti) * 4 + ((tk >> 4) & 3)) * 32) + 2 * (tk & 7);
-    auto stage = [&](const Next &r, int buf) __attribute__((always_inline)) {
+    char *const t_w = t_lds + (((((tk >> 6) * 2 + ((tk >> 3) & 1)) * F + ti) * 4 + ((tk >> 4) & 3)) * 32) + 2 * (tk & 7);
+    auto stage = [&](const Next &r) __attribute__((always_inline)) { // (a wave's own: in place of those it has read)
         Halves S, Z;
         decode_tables<F16T, TE>(r.a, r.b, r.sq, r.zq, zneg, zoff, S, Z);
-        char *const d = t_w + buf * (kBlockWaves * TTILE);
-        *reinterpret_cast<Halves *>(d) = S;
-        *reinterpret_cast<Halves *>(d + 16) = Z;
+        *reinterpret_cast<Halves *>(t_w) = S;
+        *reinterpret_cast<Halves *>(t_w + 16) = Z;
     };
 
     f32x4 acc[RT][CT];
@@ -153,41 +153,41 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
         asm volatile("" : "+v"(expo[f]));
     }
     Next nx;
-    u32x4 cw[RBW][2];
     issue(nx, 0, 0);
-#pragma unroll
-    for (int w = 0; w < RBW; ++w)
-#pragma unroll
-        for (int o = 0; o < 2; ++o)
-            cw[w][o] = LATE ? codes_at(w, (uint32_t)s0 * kStep + 64 * o) : nx.cw[0][o];
-    stage(nx, 0);
+    stage(nx);
     __builtin_amdgcn_s_waitcnt(kWaitLoads);
     __syncthreads();
+    const char *const tr = t_lds + kg * 32;
     for (int it = 0; it < nh; ++it) {
         const int buf = it & 1;
         issue(nx, it + 1, buf ^ 1);
         if (KW == 1 || it < mine) {
-            const char *xr = x_lds + (buf * KW + kh) * XTILE + lane * 16;
-            const char *tr = t_lds + buf * (kBlockWaves * TTILE) + wave * TTILE + kg * 32;
+            // chunks 2 * kg + q % 2 of the lane's batch row, kg and kg + 4 of its code rows
+            const char *const xr = x_lds + (buf * KW + kh) * XTILE + rr * 128, *const cr = c_lds + buf * CTILE + rr * 128;
+            const int xc = 16 * ((2 * kg) ^ (rr >> 1)), cc = 16 * (kg ^ (rr >> 1));
             // Groups of CT MFMAs: while those of group g run, the weights of group g + 1 are built and the tables of
             // group g + 2 are read (the compiler's own order reads them where they are used, and waits).
             constexpr int NG = 4 * RT;
             u32x4 S[2], Z[2], A[2];
             f16x8 B[CT];
             uint32_t P[4];
+            u32x4 cw[RBW]; // codes of 64 columns
+            auto codes = [&](int w, int slab) __attribute__((always_inline)) {
+                cw[w] = *reinterpret_cast<const u32x4 *>(cr + w * 2048 + (slab ? cc ^ 64 : cc));
+            };
             auto tables = [&](int h) __attribute__((always_inline)) { // h = q * F + field
                 S[h & 1] = *reinterpret_cast<const u32x4 *>(tr + h * 128);
                 Z[h & 1] = *reinterpret_cast<const u32x4 *>(tr + h * 128 + 16);
             };
             auto operand = [&](int q, int b) __attribute__((always_inline)) {
-                return *reinterpret_cast<const f16x8 *>(xr + (q * CT + b) * 1024);
+                return *reinterpret_cast<const f16x8 *>(xr + ((q >> 1) * CT + b) * 2048 + (q & 1 ? xc ^ 16 : xc));
             };
             auto build = [&](int gi) __attribute__((always_inline)) { // group gi = (q * RBW + row block) * F + field
                 const int f = gi % F, w = gi / F % RBW, q = gi / RT, h = q * F + f;
                 if (f == 0)
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
-                        P[t] = __builtin_amdgcn_perm(0u, cw[w][q >> 1][2 * (q & 1) + (t >> 1)], t & 1 ? 0x0c030c02u : 0x0c010c00u);
+                        P[t] = __builtin_amdgcn_perm(0u, cw[w][2 * (q & 1) + (t >> 1)], t & 1 ? 0x0c030c02u : 0x0c010c00u);
                 const f16 offv = (f16)(float)(1 << (10 - C::pos(f)));
                 const f16x2 off = {offv, offv};
                 f16x2 v[4]; // stage by stage: a packed instruction's result can be read by the next but one
@@ -202,6 +202,9 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
                     A[gi & 1][t] = u2(__builtin_elementwise_fma(v[t], h2(S[h & 1][t]), h2(Z[h & 1][t])));
             };
             tables(0);
+#pragma unroll
+            for (int w = 0; w < RBW; ++w)
+                codes(w, 0);
 #pragma unroll
             for (int b = 0; b < CT; ++b)
                 B[b] = operand(0, b);
@@ -219,8 +222,8 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
                     tables((gi + 1) / RT * F + (gi + 1) % F + 2);
                 else if (RBW == 1 && gi + 2 < NG && gi + 2 >= 2)
                     tables(gi + 2);
-                if (LATE && (q & 1) && f == 0) // (a slab's last codes are taken apart when its second half begins)
-                    cw[w][q >> 1] = codes_at(w, (uint32_t)(s0 + (it < last ? it + 1 : last)) * kStep + 64 * (q >> 1));
+                if (q == 1 && f == 0) // the first 64 columns' codes have been taken apart
+                    codes(w, 1);
                 const bool turn = f == F - 1 && w == RBW - 1 && q + 1 < 4; // the last MFMAs on these operands
 #pragma unroll
                 for (int b = 0; b < CT; ++b) {
@@ -242,12 +245,9 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (it + 1 < nh) {
-            stage(nx, buf ^ 1);
-            if constexpr (!LATE)
-                cw[0][0] = nx.cw[0][0], cw[0][1] = nx.cw[0][1];
-        }
-        __builtin_amdgcn_s_waitcnt(kWaitLoads); // the x tile has arrived
+        if (it + 1 < nh)
+            stage(nx);
+        __builtin_amdgcn_s_waitcnt(kWaitLoads); // x and the codes have arrived
         __syncthreads();
     }
 
@@ -370,9 +370,10 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
     }
 }
 
-template <int BITS> constexpr size_t lds_bytes(int max_ct, int kw)
+template <int BITS> constexpr size_t lds_bytes(int tiles) // tiles: row tiles times K halves
 {
-    return (size_t)2 * kw * 4 * max_ct * 1024 + (size_t)2 * kBlockWaves * 4 * Codes<BITS>::F * 128;
+    typedef Codes<BITS> C;
+    return (size_t)tiles * 8192 + (size_t)kBlockWaves * (2 * C::RBW * 2048 + 4 * C::F * 128);
 }
 
 // WIDE: members of any number of rows; else of at most 32, whose few accumulators let two blocks share a compute unit
@@ -380,7 +381,7 @@ template <int BITS, bool GATE, bool WIDE, bool F16T>
 __global__ __launch_bounds__(kBlockWaves * 64, WIDE ? 2 : 4) void rows_tile_kernel(Params)
 {
     const Params HQQ_KERNARG &p = *(const Params HQQ_KERNARG *)__builtin_amdgcn_kernarg_segment_ptr();
-    __shared__ __attribute__((aligned(16))) char lds[WIDE ? lds_bytes<BITS>(8, 1) : lds_bytes<BITS>(2, 2)];
+    __shared__ __attribute__((aligned(16))) char lds[lds_bytes<BITS>(WIDE ? 8 : 4)];
     int unit, kp, col;
     const Member HQQ_KERNARG *at = work_of(p, unit, kp, col);
     if (!at)
@@ -415,12 +416,18 @@ void launch(const Params &p, bool gate, bool wide, bool f16_tables, unsigned blo
 {
     const dim3 block(kBlockWaves * 64);
 #define HQQ_ROWS(G, W, T) rows_tile_kernel<BITS, G, W, T><<<blocks, block, 0, s>>>(p)
+    if constexpr (BITS == 2) // (4-bit: the codes' place in LDS leaves room for one block a unit in any case)
+        if (!wide) {
+            if (gate)
+                f16_tables ? HQQ_ROWS(true, false, true) : HQQ_ROWS(true, false, false);
+            else
+                f16_tables ? HQQ_ROWS(false, false, true) : HQQ_ROWS(false, false, false);
+            return;
+        }
     if (gate)
-        wide ? (f16_tables ? HQQ_ROWS(true, true, true) : HQQ_ROWS(true, true, false))
-             : (f16_tables ? HQQ_ROWS(true, false, true) : HQQ_ROWS(true, false, false));
+        f16_tables ? HQQ_ROWS(true, true, true) : HQQ_ROWS(true, true, false);
     else
-        wide ? (f16_tables ? HQQ_ROWS(false, true, true) : HQQ_ROWS(false, true, false))
-             : (f16_tables ? HQQ_ROWS(false, false, true) : HQQ_ROWS(false, false, false));
+        f16_tables ? HQQ_ROWS(false, true, true) : HQQ_ROWS(false, true, false);
 #undef HQQ_ROWS
 }
 

@@ -32,7 +32,8 @@ template <typename T> __device__ __forceinline__ T load_at(const void *base, uin
 // when the wave has waited for kWaitLoads.
 __device__ __forceinline__ void load_to_lds(uint32_t offset, const void *base, uint32_t to)
 {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(to) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 : : "v"(offset), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to)) : "memory");
 }
 constexpr int kWaitLoads = 0x0F70; // vmcnt(0), the other counters left alone
 
