@@ -90,15 +90,9 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
     }
     // this wave's kilobytes of the x tile: 64 columns wk % 2, rows 8 * (wk / 2 % 2) .. + 7 of row tiles wk / 4, wk / 4 + NWK / 4 ...
     const f16 *xb = g.x + (size_t)m0 * K + (size_t)s0 * kStep + 64 * (wk & 1);
-    uint32_t xo[XCH], xd[XCH]; // byte offsets: a lane's in x, the wave's in LDS
-#pragma unroll
-    for (int c = 0; c < XCH; ++c) {
-        int b = (wk >> 2) + NWK / 4 * c;
-        b = b < CT ? b : CT - 1; // (past the end: the last one once more, the same bytes to the same place)
-        const int hr = wk >> 1 & 1, m = m0 + 16 * b + 8 * hr + r8 < M ? 16 * b + 8 * hr + r8 : M - 1 - m0;
-        xo[c] = 2 * ((uint32_t)m * (uint32_t)K + 8 * (hr ? c8 ^ 4 : c8));
-        xd[c] = (uint32_t)(uintptr_t)(HQQ_LDS char *)x_lds + kh * XTILE + (((wk & 1) * CT + b) * 2 + hr) * 1024;
-    }
+    const int xhr = wk >> 1 & 1;
+    const uint32_t xc8 = 16u * (xhr ? c8 ^ 4 : c8), x_last = 2u * (uint32_t)(M - 1 - m0) * (uint32_t)K + xc8;
+    uint32_t x_from = 2u * (uint32_t)(16 * (wk >> 2) + 8 * xhr + r8) * (uint32_t)K + xc8; // byte offset of the lane's part of the first
     const uint32_t cd = (uint32_t)(uintptr_t)(HQQ_LDS char *)c_lds;
 
     typedef uint32_t Halves __attribute__((ext_vector_type(TE / 2)));
@@ -107,29 +101,36 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
         Halves a, b; // meta of the scale / fp16 scales, fp16 zeros
         Bytes sq, zq;
     };
-    auto issue = [&](Next &r, int it, int buf) __attribute__((always_inline)) {
+    // What a wave requests for a step, a piece at a time: all at once, it would wait to be let in by the address unit.
+    auto issue = [&](Next &r, int it, int buf, int order) __attribute__((always_inline)) {
+        const int piece = (order + XCH + 2 * RBW) % (XCH + 2 * RBW + 2); // the tables first: they have a way to go after they arrive
         const int st = it < last ? it : last;
         const uint32_t k0 = (uint32_t)(s0 + st) * kStep;
-        const f16 *const xs = xb + (size_t)st * kStep;
-#pragma unroll
-        for (int c = 0; c < XCH; ++c)
-            load_to_lds(xo[c], xs, xd[c] + buf * (KW * XTILE));
-#pragma unroll
-        for (int w = 0; w < RBW; ++w)
-#pragma unroll
-            for (int o = 0; o < 2; ++o)
-                load_to_lds(o ? co ^ 64u : co, l_codes + k0 + (size_t)(2 * w + o) * c_half, cd + buf * CTILE + (2 * w + o) * 1024);
-        if constexpr (F16T) {
-            r.a = load_at<Halves>(l_sq + 2 * (size_t)k0, 2 * trow);
-            r.b = load_at<Halves>(l_zq + 2 * (size_t)k0, 2 * trow);
-        } else {
+        if (piece < XCH) {
+            int b = (wk >> 2) + NWK / 4 * piece;
+            b = b < CT ? b : CT - 1; // (past the end: the last one once more, the same bytes to the same place)
+            asm volatile("" : "+v"(x_from)); // the sum is made here, not kept in a register over the loop
+            const uint32_t o = x_from + 32u * (uint32_t)(b - (wk >> 2)) * (uint32_t)K; // past the last row: that row once more
+            load_to_lds(o < x_last ? o : x_last, xb + (size_t)st * kStep,
+                        (uint32_t)(uintptr_t)(HQQ_LDS char *)x_lds + (buf * KW + kh) * XTILE + (((wk & 1) * CT + b) * 2 + xhr) * 1024);
+        } else if (piece < XCH + 2 * RBW) {
+            const int i = piece - XCH;
+            load_to_lds(i & 1 ? co ^ 64u : co, l_codes + k0 + (size_t)i * c_half, cd + buf * CTILE + i * 1024);
+        } else if constexpr (F16T) {
+            if (piece == XCH + 2 * RBW)
+                r.a = load_at<Halves>(l_sq + 2 * (size_t)k0, 2 * trow);
+            else
+                r.b = load_at<Halves>(l_zq + 2 * (size_t)k0, 2 * trow);
+        } else if (piece == XCH + 2 * RBW) {
             r.sq = load_at<Bytes>(l_sq + k0, trow);
             r.zq = load_at<Bytes>(l_zq + k0, trow);
+        } else {
             const uint32_t cm = mod_cols(cm0 + (uint32_t)st * kStep, p.s_cols, p.s_inv); // less than K + columns before
             r.a = load_at<Halves>(l_sms, 2 * cm);
             r.b = load_at<Halves>(l_smz, 2 * cm);
         }
     };
+    constexpr int PIECES = XCH + 2 * RBW + 2;
     // where they go: slab tk / 64, k group (tk / 16) % 4, half (tk / 8) % 2
     char *const t_w = t_lds + (((((tk >> 6) * 2 + ((tk >> 3) & 1)) * F + ti) * 4 + ((tk >> 4) & 3)) * 32) + 2 * (tk & 7);
     auto stage = [&](const Next &r) __attribute__((always_inline)) { // (a wave's own: in place of those it has read)
@@ -153,14 +154,15 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
         asm volatile("" : "+v"(expo[f]));
     }
     Next nx;
-    issue(nx, 0, 0);
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+        issue(nx, 0, 0, i);
     stage(nx);
     __builtin_amdgcn_s_waitcnt(kWaitLoads);
     __syncthreads();
     const char *const tr = t_lds + kg * 32;
     for (int it = 0; it < nh; ++it) {
         const int buf = it & 1;
-        issue(nx, it + 1, buf ^ 1);
         if (KW == 1 || it < mine) {
             // chunks 2 * kg + q % 2 of the lane's batch row, kg and kg + 4 of its code rows
             const char *const xr = x_lds + (buf * KW + kh) * XTILE + rr * 128, *const cr = c_lds + buf * CTILE + rr * 128;
@@ -222,6 +224,8 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
                     tables((gi + 1) / RT * F + (gi + 1) % F + 2);
                 else if (RBW == 1 && gi + 2 < NG && gi + 2 >= 2)
                     tables(gi + 2);
+                if (gi < PIECES)
+                    issue(nx, it + 1, buf ^ 1, gi);
                 if (q == 1 && f == 0) // the first 64 columns' codes have been taken apart
                     codes(w, 1);
                 const bool turn = f == F - 1 && w == RBW - 1 && q + 1 < 4; // the last MFMAs on these operands
@@ -254,9 +258,12 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
     // The K halves' sums meet in LDS; the first half finishes the tiles below CB, the second one the others.  (Which
     // values a wave keeps is selected value by value: with one branch per half the accumulators would be addressed.)
     constexpr int CB = KW == 1 ? CT : (CT + 1) / 2;
+    int tid = threadIdx.x; // (the lane's place is worked out again: kept over the loop it would cost the loop registers)
+    asm volatile("" : "+v"(tid));
+    const int el = tid & 63, er = tid & 15, eg = (tid >> 4) & 3;
     f32x4 sum[RT][CB];
     if constexpr (KW == 2) {
-        f32x4 *const kx = reinterpret_cast<f32x4 *>(lds) + lane; // [wk][K half][tile][row tile][lane]
+        f32x4 *const kx = reinterpret_cast<f32x4 *>(lds) + el; // [wk][K half][tile][row tile][lane]
 #pragma unroll
         for (int j = 0; j < CB; ++j)
 #pragma unroll
@@ -280,14 +287,14 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
             for (int i = 0; i < RT; ++i)
                 sum[i][j] = acc[i][j];
     }
-    // sum[i][j][v]: batch row 16 * (kh * CB + j) + rr of the block's, field i % F, row 4 * kg + v of row block i / F
+    // sum[i][j][v]: batch row 16 * (kh * CB + j) + er of the block's, field i % F, row 4 * eg + v of row block i / F
     auto row_group = [&](int w, int v) __attribute__((always_inline)) {
-        return (uint32_t)jp + (uint32_t)(16 * (rbu * RBW + w) + 4 * kg + v) * (uint32_t)p.GP;
+        return (uint32_t)jp + (uint32_t)(16 * (rbu * RBW + w) + 4 * eg + v) * (uint32_t)p.GP;
     };
     if constexpr (GATE) {
         // both projections' waves hold the same outputs: each sends the other the tiles that it finishes
         constexpr int M0 = (CB + 1) / 2; // the first projection's waves finish the tiles below M0
-        uint32_t *const gx = reinterpret_cast<uint32_t *>(lds) + lane; // [wave][tile][8 pairs][lane]
+        uint32_t *const gx = reinterpret_cast<uint32_t *>(lds) + el; // [wave][tile][8 pairs][lane]
         f32x4 own[RT][M0];
 #pragma unroll
         for (int j = 0; j < M0; ++j)
@@ -302,7 +309,7 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < M0; ++j) {
-            const int jb = proj * M0 + j, tb = kh * CB + jb, m = m0 + 16 * tb + rr;
+            const int jb = proj * M0 + j, tb = kh * CB + jb, m = m0 + 16 * tb + er;
             if (jb >= CB || tb >= CT || m >= M || !live)
                 continue;
             f16 o[RT][4];
@@ -333,7 +340,7 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
     } else {
 #pragma unroll
         for (int j = 0; j < CB; ++j) {
-            const int tb = kh * CB + j, m = m0 + 16 * tb + rr;
+            const int tb = kh * CB + j, m = m0 + 16 * tb + er;
             if (tb >= CT || m >= M || !live)
                 continue;
 #pragma unroll
