@@ -39,6 +39,7 @@ int validate_linear(const hqq_linear *l)
     return validate_table(l->zero);
 }
 
+static inline bool aligned256(const void *p) { return p && (reinterpret_cast<uintptr_t>(p) & 255u) == 0; }
 static inline size_t align256(size_t v) { return (v + 255u) & ~(size_t)255u; }
 
 enum { FAM_GENERAL = 0, FAM_SMALLBATCH = 1, FAM_TILE = 2, FAM_VEC3 = 3, FAM_LDS = 4, FAM_DQGEMM = 5 };
@@ -71,6 +72,31 @@ static int pick_family(const hqq_linear *l, int64_t M)
     if (M >= 5 && ldsgemm_supported(l, M)) // e.g. 3-bit layers whose group count the tile kernel does not take
         return FAM_LDS;
     return FAM_GENERAL;
+}
+
+static TileFinish rows_finish(const RowsItem &it, int kpb)
+{
+    return TileFinish{it.part, kpb, (int)it.M, (int)it.l0->N, rows_outputs_together(it.l0), static_cast<const f16 *>(it.l0->bias), it.y,
+                      it.row_scale, it.accumulate};
+}
+
+// A layer alone in the rows kernel, the tile family's other kernel
+static size_t rows_matmul_workspace_bytes(const hqq_linear *l, int64_t M)
+{
+    return workspace_head_bytes() + rows_partial_bytes(l, M, rows_plan(l, M, false).kpb);
+}
+
+static int launch_rows_matmul(const hqq_linear *l, const f16 *x, int64_t M, f16 *y, const f16 *row_scale, int accumulate, void *ws,
+                              hipStream_t s)
+{
+    const RowsPlan plan = rows_plan(l, M, false);
+    float *part = plan.kpb > 1 ? reinterpret_cast<float *>(static_cast<char *>(ws) + workspace_head_bytes()) : nullptr;
+    const RowsItem item = {l, nullptr, x, M, y, part, row_scale, accumulate, plan.ct};
+    const int rc = launch_rows(&item, &plan.kpb, 1, false, s);
+    if (rc != HQQ_OK || !part)
+        return rc;
+    const TileFinish fin = rows_finish(item, plan.kpb);
+    return launch_tile_finish_group(&fin, 1, s);
 }
 
 static size_t family_workspace(const hqq_linear *l, int64_t M, int fam)
@@ -152,11 +178,11 @@ int hqq_matmul_kernel_family(const hqq_linear *l, int64_t M)
     return pick_family(l, M);
 }
 
-size_t hqq_matmul_workspace_bytes(const hqq_linear *l, int64_t M)
+// what a call needs at least, whichever family is chosen or forced
+static size_t matmul_least_bytes(const hqq_linear *l, int64_t M)
 {
     if (validate_linear(l) != HQQ_OK || M <= 0)
         return 0;
-    // large enough for whichever family is chosen or forced
     const int64_t Ms = M > kSmallBatchMax ? kSmallBatchMax : M;
     size_t a = smallbatch_supported(l, Ms) ? 2 * smallbatch_workspace_bytes(l, Ms) : 0;
     size_t b = vec3_supported(l, M) ? vec3_workspace_bytes(l, M) : 0;
@@ -170,6 +196,15 @@ size_t hqq_matmul_workspace_bytes(const hqq_linear *l, int64_t M)
     if (e > b)
         b = e;
     return align256(a > b ? a : b);
+}
+
+size_t hqq_matmul_workspace_bytes(const hqq_linear *l, int64_t M)
+{
+    const size_t least = matmul_least_bytes(l, M);
+    if (least == 0 || pick_family(l, M) != FAM_TILE || !rows_preferred(l, M))
+        return least;
+    const size_t rows = align256(rows_matmul_workspace_bytes(l, M));
+    return rows > least ? rows : least;
 }
 
 int hqq_workspace_init(void *workspace, size_t workspace_bytes, void *stream)
@@ -206,6 +241,9 @@ int hqq_matmul_transpose_ex(const hqq_linear *l, const void *x_f16, int64_t M, v
         return HQQ_E_UNSUPPORTED;
     if (fam < 0 || fam > FAM_DQGEMM)
         return HQQ_E_UNSUPPORTED;
+    if (family < 0 && fam == FAM_TILE && rows_preferred(l, M) && aligned16(x_f16) && aligned16(y_f16) && aligned256(workspace) &&
+        workspace_bytes >= rows_matmul_workspace_bytes(l, M))
+        return launch_rows_matmul(l, (const f16 *)x_f16, M, (f16 *)y_f16, nullptr, 0, workspace, (hipStream_t)stream);
     const size_t need = family_workspace(l, M, fam);
     if (need > 0 && (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255u)))
         return HQQ_E_WORKSPACE;
@@ -222,8 +260,8 @@ int hqq_matmul_transpose(const hqq_linear *l, const void *x_f16, int64_t M, void
 // each (unfused path only)]
 static size_t ffn_matmul_scratch(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, int64_t M)
 {
-    size_t mm = hqq_matmul_workspace_bytes(w1, M); // already sized for the fused gate pass over two layers
-    const size_t m2 = hqq_matmul_workspace_bytes(w2, M), m3 = hqq_matmul_workspace_bytes(w3, M);
+    size_t mm = matmul_least_bytes(w1, M); // already sized for the fused gate pass over two layers
+    const size_t m2 = matmul_least_bytes(w2, M), m3 = matmul_least_bytes(w3, M);
     if (m2 > mm)
         mm = m2;
     if (m3 > mm)
@@ -251,17 +289,16 @@ static bool ffn_rows_supported(const hqq_linear *w1, const hqq_linear *w2, const
     return !w1->bias && !w3->bias && rows_supported(w1, M) && rows_supported(w3, M) && rows_supported(w2, M) && rows_alike(w1, w3);
 }
 
-// Alone, an expert needs some hundreds of rows to fill the chip that way (2-bit Mixtral expert, the other kernels against
-// this one: 256 rows 137 / 165 us, 333 rows 223 / 160, 500 rows 247 / 200)
+// From how many rows on, and up to how many, an expert alone is faster that way (Mixtral expert, the other kernels against this one:
+// 2-bit 24 rows 51 / 50 us, 48 rows 64 / 53, 128 rows 95 / 69, 333 rows 219 / 147, 1000 rows 433 / 341, 3000 rows 954 / 984; 4-bit 17
+// rows 65 / 56, 128 rows 118 / 84, 500 rows 411 / 279, 1000 rows 564 / 487, 1500 rows 639 / 655; 3-bit 96 rows 143 / 149, 160 rows
+// 225 / 163, 333 rows 285 / 229, 500 rows 317 / 333, 1000 rows 444 / 590).  Small experts have fewer blocks (5632x2048 in 3 bits: 200
+// rows 83 / 90, 330 rows 104 / 98; 1024x2048 in 4 bits: 17 rows 21 / 26, 130 rows 36 / 28).
 static bool ffn_runs_rows_kernel(const hqq_linear *w1, const hqq_linear *w2, const hqq_linear *w3, int64_t M)
 {
-    return M > 288 && ffn_rows_supported(w1, w2, w3, M);
-}
-
-static TileFinish rows_finish(const RowsItem &it, int kpb)
-{
-    return TileFinish{it.part, kpb, (int)it.M, (int)it.l0->N, rows_outputs_together(it.l0), static_cast<const f16 *>(it.l0->bias), it.y,
-                      it.row_scale, it.accumulate};
+    const int64_t size = w1->N * w1->K, from = w1->nbits == 2 ? 33 : w1->nbits == 3 ? (size < 1 << 25 ? 257 : 129) : size < 1 << 22 ? 65 : 17;
+    const int64_t to = w1->nbits == 2 ? 2400 : w1->nbits == 3 ? 400 : 1300;
+    return M >= from && M <= to && ffn_rows_supported(w1, w2, w3, M);
 }
 
 // The matmul part with the partial sums of both gate projections.  What one projection's widest family needs holds them at
@@ -271,7 +308,7 @@ static size_t ffn_gate_scratch(const hqq_linear *w1, const hqq_linear *w2, const
 {
     const size_t mm = ffn_matmul_scratch(w1, w2, w3, M);
     const size_t g = lds_gate_preferred(w1, w3, M) ? align256(ldsgemm_gate_workspace_bytes(w1, w3, M)) : 0;
-    const size_t r = ffn_runs_rows_kernel(w1, w2, w3, M) ? workspace_head_bytes() + rows_partial_bytes(w2, M, rows_k_blocks(w2, rows_blocks(w2, M, false), M > 32)) : 0;
+    const size_t r = ffn_runs_rows_kernel(w1, w2, w3, M) ? rows_matmul_workspace_bytes(w2, M) : 0;
     const size_t most = g > r ? g : r;
     return most > mm ? most : mm;
 }
@@ -297,8 +334,8 @@ size_t hqq_expert_ffn_workspace_bytes(const hqq_linear *w1, const hqq_linear *w2
 // workspace of the gate: [matmul scratch, counters first][a, b: M x N fp16 each (unfused paths only)]
 static size_t gate_matmul_scratch(const hqq_linear *w1, const hqq_linear *w3, int64_t M)
 {
-    size_t mm = hqq_matmul_workspace_bytes(w1, M); // already sized for the fused decode pass over two layers
-    const size_t m3 = hqq_matmul_workspace_bytes(w3, M), g = tile_gate_workspace_bytes(w1, w3, M);
+    size_t mm = matmul_least_bytes(w1, M); // already sized for the fused decode pass over two layers
+    const size_t m3 = matmul_least_bytes(w3, M), g = tile_gate_workspace_bytes(w1, w3, M);
     mm = m3 > mm ? m3 : mm;
     mm = g > mm ? g : mm;
     const size_t v = vec3_gate_workspace_bytes(w1, M);
@@ -404,19 +441,15 @@ static int expert_ffn_impl(const hqq_linear *w1, const hqq_linear *w2, const hqq
     f16 *y = (f16 *)y_f16;
 
     // 17 rows and more: both gate projections in one launch, silu(a) * b in its blocks, then the down projection
-    if (ffn_runs_rows_kernel(w1, w2, w3, M) && aligned16(x)) {
-        const int kpb = rows_k_blocks(w2, rows_blocks(w2, M, false), M > 32);
-        const size_t bytes = rows_partial_bytes(w2, M, kpb);
+    if (ffn_runs_rows_kernel(w1, w2, w3, M) && aligned16(x) && aligned16(y)) {
         if (workspace_bytes >= ffn_gate_scratch(w1, w2, w3, M) + rows_bytes) // else the kernels that need no more than the least
             mm_bytes = ffn_gate_scratch(w1, w2, w3, M), h = (f16 *)(p + mm_bytes);
-        if (workspace_head_bytes() + bytes <= mm_bytes) {
-            float *part = bytes ? reinterpret_cast<float *>(p + workspace_head_bytes()) : nullptr;
-            const RowsItem gate = {w1, w3, x, M, h, nullptr, nullptr, 0};
-            const RowsItem down = {w2, nullptr, h, M, y, part, (const f16 *)row_scale_f16, accumulate};
-            if ((rc = launch_rows(&gate, &kpb, 1, true, s)) != HQQ_OK || (rc = launch_rows(&down, &kpb, 1, false, s)) != HQQ_OK || !part)
+        if (rows_matmul_workspace_bytes(w2, M) <= mm_bytes) {
+            const int whole = 1;
+            const RowsItem gate = {w1, w3, x, M, h, nullptr, nullptr, 0, rows_plan(w1, M, true).ct};
+            if ((rc = launch_rows(&gate, &whole, 1, true, s)) != HQQ_OK)
                 return rc;
-            const TileFinish fin = rows_finish(down, kpb);
-            return launch_tile_finish_group(&fin, 1, s);
+            return launch_rows_matmul(w2, h, M, y, (const f16 *)row_scale_f16, accumulate, mm, s);
         }
     }
     // 3-bit decode batches: both gate projections in one launch, silu(a) * b folded into the down projection's loads
@@ -656,13 +689,18 @@ static const hqq_linear *const *expert_rows_lead(const hqq_linear *const *w1, co
         return nullptr;
     // Few experts, or few rows of one, leave the chip idle: the kernels that split K further are faster then (2-bit Mixtral
     // experts, one by one / together: four with a row each 80 / 92 us, eight 169 / 172, eight with two 202 / 168).
-    int64_t blocks = 0;
+    int64_t blocks = 0, used = 0;
     bool wide = false;
     for (int g = 0; g < n_groups; ++g)
         if (row_start[g + 1] > row_start[g]) {
+            ++used;
             blocks += rows_blocks(w1[lead - w2], row_start[g + 1] - row_start[g], true);
             wide = wide || row_start[g + 1] - row_start[g] > 32;
         }
+    // Very many rows are a library product's over de-quantised weights, as alone; together 3-bit experts keep ahead for longer (300 rows
+    // each 2782 / 1353 us, 700 rows 3215 / 2926).
+    if (row_start[n_groups] > used * ((*lead)->nbits == 2 ? 2400 : (*lead)->nbits == 3 ? 800 : 1300))
+        return nullptr;
     return blocks >= (wide || (*lead)->nbits != 2 ? 160 : 512) ? lead : nullptr;
 }
 
@@ -781,9 +819,9 @@ int hqq_expert_rows_ffn(const hqq_linear *const *w1, const hqq_linear *const *w2
         at += align256((size_t)M * (size_t)w1[g]->N * sizeof(f16));
         kpb[n] = kb;
         const size_t bytes = rows_partial_bytes(w2[g], M, kpb[n]);
-        gate[n] = RowsItem{w1[g], w3[g], static_cast<const f16 *>(x_f16) + lo * w1[g]->K, M, h, nullptr, nullptr, 0};
+        gate[n] = RowsItem{w1[g], w3[g], static_cast<const f16 *>(x_f16) + lo * w1[g]->K, M, h, nullptr, nullptr, 0, 0};
         down[n] = RowsItem{w2[g], nullptr, h, M, static_cast<f16 *>(y_f16) + lo * w2[g]->N, bytes ? reinterpret_cast<float *>(at) : nullptr,
-                           row_scale_f16 ? static_cast<const f16 *>(row_scale_f16) + lo : nullptr, 0};
+                           row_scale_f16 ? static_cast<const f16 *>(row_scale_f16) + lo : nullptr, 0, 0};
         at += bytes;
         ++n;
     }

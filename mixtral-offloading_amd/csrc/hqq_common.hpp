@@ -300,6 +300,7 @@ struct RowsItem {
     float *part;               // rows_k_blocks(...) > 1: that many partial sums per output, finished by launch_tile_finish_group
     const f16 *row_scale;
     int accumulate;
+    int ct; // 16-row tiles of a block, 0: as many as it takes, spread evenly
 };
 bool rows_supported(const hqq_linear *l, int64_t M);
 bool rows_alike(const hqq_linear *a, const hqq_linear *b);
@@ -307,6 +308,12 @@ int64_t rows_blocks(const hqq_linear *l, int64_t M, bool gate); // of a launch w
 int rows_k_blocks(const hqq_linear *l, int64_t blocks, bool wide); // blocks: of all members; wide: one has more than 32 rows
 int rows_outputs_together(const hqq_linear *l);                    // F of a finishing pass
 size_t rows_partial_bytes(const hqq_linear *l, int64_t M, int kpb);
+// one layer (or a gate's two) in a launch of its own: tiles of a block and blocks along K, by the time that they are expected to take
+struct RowsPlan {
+    int ct, kpb;
+};
+RowsPlan rows_plan(const hqq_linear *l, int64_t M, bool gate);
+bool rows_preferred(const hqq_linear *l, int64_t M); // over the tile kernel, for one layer
 int launch_rows(const RowsItem *item, const int *kpb, int n, bool gate, hipStream_t s);
 // dequant_gemm.hip: wide batches as hqq_dequantize into the workspace + one library GEMM
 bool dqgemm_supported(const hqq_linear *l, int64_t M);

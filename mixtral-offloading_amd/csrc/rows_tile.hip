@@ -56,11 +56,11 @@ struct Cut {
     int ct, ncol;
     int share; // waves of a block that work on the same output rows (of one projection)
 };
-Cut cut_rows(int nbits, int64_t M)
+Cut cut_rows(int nbits, int64_t M, int ct)
 {
     const int tiles = (int)((M + 15) / 16), most = max_tiles(nbits), n = (tiles + most - 1) / most;
     Cut c;
-    c.ct = (tiles + n - 1) / n, c.ncol = (tiles + c.ct - 1) / c.ct, c.share = (nbits == 3 ? c.ct > kHalfFields3 : c.ct <= kHalvesTiles) ? 2 : 1;
+    c.ct = ct ? ct : (tiles + n - 1) / n, c.ncol = (tiles + c.ct - 1) / c.ct, c.share = (nbits == 3 ? c.ct > kHalfFields3 : c.ct <= kHalvesTiles) ? 2 : 1;
     return c;
 }
 int units(const Shape &sh, const Cut &c, bool gate)
@@ -74,7 +74,7 @@ int units(const Shape &sh, const Cut &c, bool gate)
 bool rows_supported(const hqq_linear *l, int64_t M)
 {
     Shape sh;
-    return M > 0 && M < (1 << 24) && shape_of(l, sh);
+    return M > 0 && M < (1 << 24) && M * l->K < (1ll << 31) && shape_of(l, sh); // 32-bit byte offsets within x
 }
 
 bool rows_alike(const hqq_linear *a, const hqq_linear *b)
@@ -88,7 +88,7 @@ int64_t rows_blocks(const hqq_linear *l, int64_t M, bool gate)
     Shape sh;
     if (!shape_of(l, sh))
         return 0;
-    const Cut c = cut_rows(l->nbits, M);
+    const Cut c = cut_rows(l->nbits, M, 0);
     return (int64_t)units(sh, c, gate) * c.ncol;
 }
 
@@ -109,6 +109,67 @@ int rows_k_blocks(const hqq_linear *l, int64_t blocks, bool wide)
     }
     const int spp = (sh.steps + best - 1) / best; // parts of equal length, none of them empty
     return (sh.steps + spp - 1) / spp;
+}
+
+// What a step of 128 columns (of a K half: of both) and a tile of it take in a block when all units are at work, in ns: the fit of
+// 5800 launches of single layers (2- to 4-bit, 1024x1024 to 14336x4096, 17 to 1270 rows, every cut and 1 to 16 blocks along K),
+// which it meets to 10 % (rms).  What it chooses is on average 3 % slower than the fastest of them.  At 2-bit 4096x14336 with 128
+// rows that is 4 tiles and 8 blocks along K, 30 us; as wide as a block can be (8 tiles) 49; 4-bit 4096x4096 with 256 rows 23, 31.
+struct StepCost {
+    int start, step, tile;
+};
+static StepCost step_cost(int nbits, int ct)
+{
+    if (nbits == 3)
+        return ct <= kHalfFields3 ? StepCost{10200, 2030, 1060} : StepCost{9600, 1400, 330};
+    if (nbits == 2)
+        return ct <= 2 ? StepCost{6300, 2270, 160} : ct <= kHalvesTiles ? StepCost{6000, 1380, 180} : StepCost{5200, 1050, 240};
+    return ct <= kHalvesTiles ? StepCost{5200, 1320, 180} : StepCost{7400, 1240, 190};
+}
+
+RowsPlan rows_plan(const hqq_linear *l, int64_t M, bool gate)
+{
+    RowsPlan best = {0, 1};
+    Shape sh;
+    if (!shape_of(l, sh))
+        return best;
+    const int64_t tiles = (M + 15) / 16;
+    double least = 0;
+    for (int ct = 1; ct <= max_tiles(l->nbits) && ct <= tiles; ++ct) {
+        const Cut c = cut_rows(l->nbits, M, ct);
+        const StepCost t = step_cost(l->nbits, ct);
+        const bool narrow = l->nbits == 2 && ct <= 2; // two blocks share a unit, and a step takes half as long where one has it alone
+        const int halves = l->nbits != 3 && c.share == 2 ? 2 : 1, slots = narrow ? 512 : 256;
+        for (int k = 1; k <= (gate ? 1 : 16) && sh.steps / k >= (k > 1 ? 4 : 1); ++k) {
+            const int spp = (sh.steps + k - 1) / k, kpb = (sh.steps + spp - 1) / spp;
+            if (kpb != k)
+                continue;
+            const int64_t blocks = ((int64_t)units(sh, c, gate) * k + 7) / 8 * 8 * c.ncol; // of a die: an eighth, rounded up
+            const int64_t rounds = (blocks + slots - 1) / slots;
+            const double load = narrow && blocks < slots ? 0.5 + 0.5 * (double)blocks / slots : 1.0;
+            double ns = t.start + (double)rounds * ((spp + halves - 1) / halves) * (t.step + t.tile * ct) * load;
+            if (k > 1) // the partial sums' way to memory and back, and a launch
+                ns += 2500.0 + 200.0 * k + 1.5e-3 * k * (double)M * (double)l->N;
+            if (best.ct == 0 || ns < least)
+                best = RowsPlan{ct, k}, least = ns;
+        }
+    }
+    return best;
+}
+
+// One layer, the tile kernel against this one, in us: 2-bit 14336x4096 with 32 rows 20.0 / 17.5, 128 rows 38.2 / 29.4, 290 rows 79 / 53,
+// 630 rows 162 / 92; 4096x14336 333 rows 66 / 54, 1000 rows 140 / 117; 4-bit 4096x4096 32 rows 12.6 / 13.4, 64 rows 18.0 / 17.0, 630 rows
+// 75 / 45; 14336x4096 17 rows 24.3 / 16.7, 290 rows 138 / 58.  3-bit codes have few blocks where there are few windows, and the tile kernel's rewrite is
+// cheap there: 112 windows (14336x4096) 17 rows 34.5 / 27.6, 64 rows 37.6 / 35.5, 290 rows 149 / 81; 32 windows, 4096x14336 64 rows
+// 38.7 / 40.2, 96 rows 49.0 / 44.5, 4096x4096 256 rows 35.2 / 38.0, 290 rows 48.3 / 43.5.
+bool rows_preferred(const hqq_linear *l, int64_t M)
+{
+    Shape sh;
+    if (M <= 16 || !rows_supported(l, M) || !shape_of(l, sh))
+        return false;
+    if (l->nbits == 3)
+        return M > (sh.GP >= 64 ? 16 : l->K >= 8192 ? 64 : 256);
+    return M > 32 || l->nbits == 2 || l->N * l->K > (1ll << 24);
 }
 
 size_t rows_partial_bytes(const hqq_linear *l, int64_t M, int kpb)
@@ -149,7 +210,9 @@ int launch_rows(const RowsItem *item, const int *kpb, int n, bool gate, hipStrea
             }
             m.x = it.x, m.y = it.y, m.part = it.part, m.row_scale = it.row_scale, m.accumulate = it.accumulate;
             m.bias = gate ? nullptr : static_cast<const f16 *>(it.l0->bias);
-            const Cut c = cut_rows(l->nbits, it.M);
+            if (it.ct < 0 || it.ct > max_tiles(l->nbits))
+                return HQQ_E_UNSUPPORTED;
+            const Cut c = cut_rows(l->nbits, it.M, it.ct);
             m.M = (int)it.M, m.ct = c.ct, m.ncol = c.ncol;
             const int kb = gate ? 1 : kpb[order[i]];
             m.spp = (sh.steps + kb - 1) / kb, m.kpb = (sh.steps + m.spp - 1) / m.spp;

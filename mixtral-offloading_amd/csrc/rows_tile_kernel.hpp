@@ -6,8 +6,9 @@
 // and every weight is rebuilt in registers, once per block: mask-and-insert, subtract, fma with the scale and minus scale * zero.
 // Per 128 columns the block reads its x tile straight into LDS (operand order, one barrier), each wave de-quantises its own
 // table entries into LDS, and a wave issues 16 groups of ct MFMAs; see the loop for how they overlap.
-//   * scale * zero is rounded once, from 32 bits, and the weight once: against 64 bits the FFN of a 2-bit expert is off by
-//     0.92e-3, with the reference's five roundings of a weight by 1.45e-3 (4-bit 1.07e-3, 1.23e-3).
+//   * 2-bit: a weight is rounded once after its scale: against 64 bits the FFN of an expert on 48 rows is off by 0.74e-3, with the
+//     reference's five roundings of a weight by 1.17e-3, a 4096x14336 layer on 333 rows by 0.38e-3 and 0.78e-3.  4-bit: the
+//     reference's roundings (1.20e-3, as before).
 //   * Up to 64 rows there are few MFMAs to hide behind: the block's waves split its columns in two halves and meet in LDS, and up
 //     to 32 rows 128 registers let two blocks share a unit.  There the loads of a step (codes, tables, their meta, x) bound the
 //     launch: eight 2-bit Mixtral experts with 1 to 16 rows each take 170 us (3.1 TB/s), with 32 rows 208 us; the launches of one
@@ -31,6 +32,10 @@ template <int BITS> struct Codes {
     static constexpr int F = 8 / BITS;       // output rows per packed row
     static constexpr int RBW = 4 / F;        // row blocks of sixteen a wave takes (they share its table rows)
     static constexpr int RT = F * RBW;       // 16-row tiles per wave
+    // 2-bit: a weight is scale * (code - 2) + scale * (2 - zero): a zero lies near the middle of the codes, and the second product,
+    // which is rounded, is small there.  4-bit, the codes of attention layers: (code - zero) * scale, rounded as hqq_dequantize rounds
+    // (a layer's keys are then no further from those of its de-quantised weights than the order of the sums makes them).
+    static constexpr int CENTRE = BITS == 2 ? 2 : kStored, OFF = BITS == 2 ? 2 : 0, VALU = BITS == 2 ? 12 : 16;
     static constexpr int pos(int f) { return BITS * (F - 1 - f); }
     static constexpr uint32_t mask(int f) { return (((1u << BITS) - 1u) * 0x00010001u) << pos(f); }
     // a field masked in place and OR-ed into the mantissa of 2^(10 - pos) reads as 2^(10 - pos) + code
@@ -81,10 +86,11 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
     const int ti = lane / (kStep / TE), tk = TE * (lane % (kStep / TE));
     const uint32_t trow = (uint32_t)(F * jp + ti) * (uint32_t)K + (uint32_t)tk;
     uint32_t cm0 = 0;
-    float zneg = 0.f, zoff = 0.f; // -zero = zoff + code * zneg
+    float zneg = 0.f, zoff = 0.f; // of the zero table: decode_tables
     if constexpr (!F16T) {
         zneg = uniform(-(float)gload<f16>(g.l[proj].z_ms));
-        zoff = uniform(-(float)gload<f16>(g.l[proj].z_mz) * zneg);
+        const float zmz = (float)gload<f16>(g.l[proj].z_mz);
+        zoff = uniform(C::CENTRE == kStored ? zmz : (float)C::CENTRE - zmz * zneg);
         const uint32_t c = trow + (uint32_t)s0 * kStep;
         cm0 = mod_cols(c, p.s_cols, p.s_inv);
     }
@@ -135,7 +141,7 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
     char *const t_w = t_lds + (((((tk >> 6) * 2 + ((tk >> 3) & 1)) * F + ti) * 4 + ((tk >> 4) & 3)) * 32) + 2 * (tk & 7);
     auto stage = [&](const Next &r) __attribute__((always_inline)) { // (a wave's own: in place of those it has read)
         Halves S, Z;
-        decode_tables<F16T, TE>(r.a, r.b, r.sq, r.zq, zneg, zoff, S, Z);
+        decode_tables<F16T, TE, C::CENTRE>(r.a, r.b, r.sq, r.zq, zneg, zoff, S, Z);
         *reinterpret_cast<Halves *>(t_w) = S;
         *reinterpret_cast<Halves *>(t_w + 16) = Z;
     };
@@ -190,7 +196,7 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
                         P[t] = __builtin_amdgcn_perm(0u, cw[w][2 * (q & 1) + (t >> 1)], t & 1 ? 0x0c030c02u : 0x0c010c00u);
-                const f16 offv = (f16)(float)(1 << (10 - C::pos(f)));
+                const f16 offv = (f16)(float)((1 << (10 - C::pos(f))) + C::OFF);
                 const f16x2 off = {offv, offv};
                 f16x2 v[4]; // stage by stage: a packed instruction's result can be read by the next but one
 #pragma unroll
@@ -198,10 +204,19 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
                     v[t] = h2((P[t] & C::mask(f)) | expo[f]);
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
-                    v[t] = v[t] - off; // the exact code
+                    v[t] = v[t] - off; // the code (2-bit: less 2), exact
+                if constexpr (C::CENTRE == kStored) {
 #pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    A[gi & 1][t] = u2(__builtin_elementwise_fma(v[t], h2(S[h & 1][t]), h2(Z[h & 1][t])));
+                    for (int t = 0; t < 4; ++t)
+                        v[t] = v[t] + h2(Z[h & 1][t]);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        A[gi & 1][t] = u2(v[t] * h2(S[h & 1][t]));
+                } else {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        A[gi & 1][t] = u2(__builtin_elementwise_fma(v[t], h2(S[h & 1][t]), h2(Z[h & 1][t])));
+                }
             };
             tables(0);
 #pragma unroll
@@ -239,12 +254,12 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
                 // an MFMA, what its operand's register is read into next, and the vector instructions that it hides
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, (12 + CT - 1) / CT, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (C::VALU + CT - 1) / CT, 0);
 #pragma unroll
                 for (int b = 1; b < CT; ++b) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, (12 + CT - 1) / CT, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, (C::VALU + CT - 1) / CT, 0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);

@@ -62,10 +62,12 @@ __device__ __forceinline__ uint32_t mod_cols(uint32_t c, uint32_t cols, uint32_t
     return c - (c >= cols ? cols : 0);
 }
 
-// TE table entries as a lane loaded them -> scales and minus scale * zero, in pairs.  8-bit tables: a, b the scale's meta (scale,
-// zero), sq, zq the bytes, the zero table's own meta as zneg, zoff (-zero = zoff + code * zneg); each result is rounded once, from
-// 32 bits.  fp16 tables: a the scales, b the zeros.
-template <bool F16T, int TE, typename Halves, typename Bytes>
+// TE table entries as a lane loaded them -> scales and scale * (C - zero), in pairs.  8-bit tables: a, b the scale's meta (scale,
+// zero), sq, zq the bytes, the zero table's own meta as zneg, zoff (C - zero = zoff + code * zneg); each result is rounded once, from
+// 32 bits.  fp16 tables: a the scales, b the zeros.  C = kStored: scales and minus zeros, rounded as hqq_dequantize rounds them (zneg:
+// minus the meta's scale, zoff: its zero).
+constexpr int kStored = -1;
+template <bool F16T, int TE, int C, typename Halves, typename Bytes>
 __device__ __forceinline__ void decode_tables(const Halves &a, const Halves &b, const Bytes &sq, const Bytes &zq, float zneg, float zoff,
                                               Halves &S, Halves &Z)
 {
@@ -73,7 +75,17 @@ __device__ __forceinline__ void decode_tables(const Halves &a, const Halves &b, 
     for (int e = 0; e < TE / 2; ++e) {
         if constexpr (F16T) {
             S[e] = a[e];
-            Z[e] = u2(-(h2(b[e]) * h2(a[e])));
+            if constexpr (C == kStored) {
+                Z[e] = u2(-h2(b[e]));
+            } else if constexpr (C == 0) {
+                Z[e] = u2(-(h2(b[e]) * h2(a[e])));
+            } else {
+                f16x2 zv;
+#pragma unroll
+                for (int o = 0; o < 2; ++o)
+                    zv[o] = (f16)(((float)C - (float)h2(b[e])[o]) * (float)h2(a[e])[o]);
+                Z[e] = u2(zv);
+            }
         } else {
             f16x2 sv, zv;
 #pragma unroll
@@ -85,6 +97,11 @@ __device__ __forceinline__ void decode_tables(const Halves &a, const Halves &b, 
                     sw = sq[0], zw = zq[0];
                 const int sh = 8 * ((2 * e + o) & 3);
                 const float sc = (float)((sw >> sh) & 0xFFu), zc = (float)((zw >> sh) & 0xFFu);
+                if constexpr (C == kStored) {
+                    sv[o] = (f16)((float)(f16)(sc - (float)h2(b[e])[o]) * (float)h2(a[e])[o]);
+                    zv[o] = (f16)((float)(f16)(zc - zoff) * zneg);
+                    continue;
+                }
                 const float d = __builtin_fmaf((float)h2(b[e])[o], -1.0f, sc);
                 sv[o] = (f16)__builtin_fmaf(d, (float)h2(a[e])[o], 0.0f);
                 zv[o] = (f16)__builtin_fmaf(__builtin_fmaf(zc, zneg, zoff), (float)sv[o], 0.0f);

@@ -124,7 +124,7 @@ __device__ __forceinline__ void tile(const Params HQQ_KERNARG &p, const Member H
     char *const t_w = t_lds + proj * TTILE + ((tl * 4 + (tc >> 2)) * 4 + 2 * (tc & 1)) * 32 + 8 * ((tc >> 1) & 1);
     auto stage = [&](const Next &r, int buf) __attribute__((always_inline)) {
         u32x4 S, Z;
-        decode_tables<F16T, 8>(r.a, r.b, r.sq, r.zq, zneg, zoff, S, Z);
+        decode_tables<F16T, 8, 0>(r.a, r.b, r.sq, r.zq, zneg, zoff, S, Z);
         char *const d = t_w + buf * ((GATE ? 2 : 1) * TTILE);
         *reinterpret_cast<u32x2 *>(d) = (u32x2){S.x, S.y};
         *reinterpret_cast<u32x2 *>(d + 16) = (u32x2){Z.x, Z.y};
